@@ -21,7 +21,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libgpu_tracking.so")
-SOURCES = ["gt_kernels.hip", "gt_synth.hip", "gt_adjoint.hip", "gt_link.hip", "gt_raw.hip", "gt_ingest.hip", "gt_api.hip"]
+KERNEL_SOURCES = ["gt_detect.hip", "gt_bandpass.hip", "gt_kernels.hip"]
+SOURCES = [*KERNEL_SOURCES, "gt_synth.hip", "gt_adjoint.hip", "gt_link.hip", "gt_raw.hip",
+           "gt_ingest.hip", "gt_api.hip"]
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 
@@ -75,9 +77,9 @@ def build_asan(verbose: bool = False) -> str:
     """The library with its host code instrumented by AddressSanitizer (device
     code as usual, -fsanitize only after -Xarch_host), for CPU tests of the
     host paths (parameters, column names, movie-file decoding, argument and
-    error handling) under clang's ASan runtime.  gt_kernels.hip, whose host
-    code is kernel launchers only, is linked from the regular build's object
-    (built first when missing)."""
+    error handling) under clang's ASan runtime.  The files in KERNEL_SOURCES,
+    whose host code is kernel launchers only, are linked from the regular
+    build's objects (built first when missing)."""
     os.makedirs(ASAN_DIR, exist_ok=True)
     objdir = os.path.join(HERE, "_build")
     os.makedirs(objdir, exist_ok=True)
@@ -86,8 +88,8 @@ def build_asan(verbose: bool = False) -> str:
     jobs = []
     objs = []
     for src in SOURCES:
-        if src == "gt_kernels.hip":
-            obj = os.path.join(objdir, "gt_kernels.o")
+        if src in KERNEL_SOURCES:
+            obj = os.path.join(objdir, src.replace(".hip", ".o"))
             srcp = os.path.join(CSRC, src)
             if not os.path.exists(obj) or os.path.getmtime(obj) < os.path.getmtime(srcp):
                 jobs.append(([HIPCC, *FLAGS, "-c", srcp, "-o", obj], src))

@@ -1,5 +1,6 @@
 // gt_internal.h -- device-side descriptors and launch entry points shared by
-// the HIP kernels (gt_kernels.hip) and the host orchestration (gt_api.hip).
+// the HIP kernels (gt_kernels.hip, gt_bandpass.hip, gt_detect.hip) and the
+// host orchestration (gt_api.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -142,8 +143,8 @@ struct AdjOut {
     float* jac;            // [rows_cap * 3 * S * S] Jacobian patches, or null
 };
 
-// Launchers (gt_kernels.hip).  All launch on `s`; return hipSuccess or the
-// first launch error.
+// Launchers (gt_kernels.hip, gt_bandpass.hip, gt_detect.hip).  All launch on
+// `s`; return hipSuccess or the first launch error.
 hipError_t launch_zero_batch(const Batch& b, hipStream_t s);
 // The streaming bandpass handles uint8, uint16 and float32 input with 1 <= R <= 8, W % 4 == 0
 // and aligned frame bases (b.vec); everything else takes the generic kernels.

@@ -227,7 +227,7 @@ def main() -> int:
     ap.add_argument("--no-percentile", action="store_true",
                     help="locate without the percentile test (the reference's default)")
     ap.add_argument("--seg-rows", type=int, default=0,
-                    help="rows per bandpass work item (default: the library's 128)")
+                    help="rows per bandpass work item (default: the library's choice)")
     ap.add_argument("--separate-refine", action="store_true",
                     help="walk in a separate refine kernel instead of inside detect")
     ap.add_argument("--no-graph", action="store_true",

@@ -1,0 +1,70 @@
+"""The streaming bandpass against the oracle where it can go wrong: every
+smoothing radius, frames narrower than a strip and one column around its
+edges (128 columns per wave, 256 per work item), frame bases at any multiple
+of the element size, and uint16 boxcar sums past 2^24.
+
+Bars as in test_gpu_parity: the same candidate pixels, positions within 1e-4
+px, masses within 1e-5 relative.
+"""
+import numpy as np
+import pytest
+
+from tests.test_gpu_parity import _check, _oracle_movie
+from tracking_optimizations_amd import _lib
+from tracking_optimizations_amd.gpu_tracking import locate, make_params
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = {"u8": np.uint8, "u16": np.uint16, "f32": np.float32}
+
+
+def _noise(shape, dtype, seed):
+    """Bright noise: uint16 near saturation, so that a window of k >= 17 rows
+    sums past 2^24; float32 of both signs and uneven magnitudes."""
+    rng = np.random.default_rng(seed)
+    if dtype == "u8":
+        return rng.integers(0, 256, shape, dtype=np.uint8)
+    if dtype == "u16":
+        return rng.integers(50000, 65536, shape, dtype=np.uint16)
+    return (rng.standard_normal(shape) * np.exp(rng.uniform(-3, 6, shape))).astype(np.float32)
+
+
+@pytest.mark.parametrize("dtype", sorted(DTYPES))
+@pytest.mark.parametrize("k", [2, 3, 5, 8, 9, 11, 13, 15, 16, 17, 19, 21, 23, 25, 27, 29, 31, 33])
+def test_radii_and_widths(dtype, k):
+    import torch
+    ctx = _lib.default_context(0)
+    r = k // 2
+    for n, (h, w) in enumerate([(max(r, 9), max(r, 2)), (29, 17), (37, 127), (31, 128), (33, 129),
+                                (21, 255), (25, 257), (70, 131)]):
+        frames = _noise((2, h, w), dtype, 100 * k + n)
+        # a base one element past an allocation's start, odd frame sizes
+        flat = torch.zeros(frames.size + 1, dtype=getattr(torch, {"u8": "uint8", "u16": "uint16",
+                                                                 "f32": "float32"}[dtype]))
+        flat[1:] = torch.from_numpy(frames.reshape(-1))
+        dev = flat.cuda()[1:].reshape(2, h, w)
+        for pct in (None, 30):
+            kw = dict(diameter=5, separation=5, smoothing_size=k, percentile=pct)
+            print(f"[bandpass] {dtype} k={k} {h}x{w} percentile={pct}", flush=True)
+            rows, cand, _, _ = locate(dev, make_params(**kw), ctx=ctx)
+            ref_rows, ref_cand = _oracle_movie(frames, kw)
+            _check(rows, cand, ref_rows, ref_cand, f"{dtype}/k={k}/{h}x{w}/pct={pct}")
+
+
+def test_long_segments_and_narrow_frames():
+    """Rows per work item at both ends of the accepted range, and frames one
+    and two pixels wide (the two-pass form and the narrowest streaming one)."""
+    ctx = _lib.Context(0)
+    frames = _noise((2, 300, 140), "u16", 7)
+    kw = dict(diameter=5, separation=5, smoothing_size=9, percentile=40)
+    ref = _oracle_movie(frames, kw)
+    for seg in (16, 17, 272):
+        ctx.set_launch_shape(seg)
+        rows, cand, _, _ = locate(frames, make_params(**kw), ctx=ctx)
+        _check(rows, cand, *ref, f"seg={seg}")
+    for w in (1, 2, 3):
+        kw = dict(diameter=1, separation=2, smoothing_size=3)
+        frames = _noise((2, 40, w), "u16", w)
+        rows, cand, _, _ = locate(frames, make_params(**kw), ctx=ctx)
+        _check(rows, cand, *_oracle_movie(frames, kw), f"width {w}")
+    ctx.close()

@@ -7,7 +7,9 @@ Every HIP source is compiled separately (in parallel) and linked into
   * ``-fhip-fp32-correctly-rounded-divide-sqrt``: IEEE division and sqrt;
   * ``-fno-gpu-flush-denormals-to-zero``: keep binary32 subnormals;
   * ``-Xclang -target-feature -Xclang -packed-fp32-ops``: no packed FP32
-    instructions are generated.
+    instructions are generated;
+  * ``-pragma-unroll-threshold``: the bandpass's row loop of up to 33 rows is
+    unrolled whole, so that its register ring has constant indices.
 """
 from __future__ import annotations
 
@@ -21,7 +23,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libgpu_tracking.so")
-KERNEL_SOURCES = ["gt_detect.hip", "gt_bandpass.hip", "gt_kernels.hip"]
+KERNEL_SOURCES = ["gt_detect.hip", "gt_bandpass_u16.hip", "gt_bandpass_u8.hip",
+                  "gt_bandpass_f32.hip", "gt_bandpass.hip", "gt_kernels.hip"]
 SOURCES = [*KERNEL_SOURCES, "gt_synth.hip", "gt_adjoint.hip", "gt_link.hip", "gt_raw.hip",
            "gt_ingest.hip", "gt_api.hip"]
 
@@ -37,6 +40,7 @@ FLAGS = [
     "-fno-gpu-flush-denormals-to-zero",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-pass-failed",
+    "-mllvm", "-pragma-unroll-threshold=65536",
     "-I" + os.path.join(ROOT, "include"),
     "-I" + CSRC,
 ]

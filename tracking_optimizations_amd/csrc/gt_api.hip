@@ -294,7 +294,7 @@ gt_status make_geom(const gt_params* p, bool integer_input, Geom& g) {
     g.disk_in_window = (g.rint <= g.a) && (g.rint <= g.kd - 1 - g.a);
     // Gaussian weights (preprocess_rows.wgsl:44): argument in binary32,
     // exponential evaluated in binary64 on the host and rounded once.
-    float gn = 0.f, wmin = 1.f;
+    float gn = 0.f;
     for (int i = -g.R; i <= g.R; ++i) {
         const float x = (float)i;
         volatile float arg = -(x * x);
@@ -302,13 +302,18 @@ gt_status make_geom(const gt_params* p, bool integer_input, Geom& g) {
         const float wi = (float)std::exp((double)arg);
         g.w[i + g.R] = wi;
         gn = gn + wi;
-        if (wi > 0.f) wmin = std::min(wmin, wi);
     }
     g.gn = gn;
     g.rgn = 1.0f / gn;
     g.kk = (float)(g.k * g.k);
     g.rkk = 1.0f / g.kk;
-    g.fastdiv_gn = integer_input && wmin >= std::ldexp(1.0f, -40) && corrected_div_exact(gn);
+    // Integer frames only.  Where weights are so small that a quotient leaves
+    // the normal range, the exact and the corrected quotient may differ in
+    // their last bits, below 2^-100; that cannot show: a nonzero pixel puts at
+    // least 1 / k^2 into the boxcar term, so an output whose Gaussian term is
+    // below 2^-60 is clamped to zero either way, and a larger one does not
+    // change when a term below 2^-100 does in its last bits.
+    g.fastdiv_gn = integer_input && corrected_div_exact(gn);
     g.fastdiv_kk = integer_input && corrected_div_exact(g.kk);
     // dedup neighbourhood in tiles: start pixels of two rows closer than
     // `separation` differ by less than sep + 2*(max_iterations + rint) per axis
@@ -375,13 +380,8 @@ struct gt_context {
     gt_timing last{};
     uint32_t batch_frames = 0;   // 0 = automatic
     size_t workspace_limit = (size_t)6 << 30;   // per workspace
-    int seg_rows = 128;
-    // rows per bandpass work item of the plain per-frame path unless the
-    // caller sets the launch shape: one frame per launch needs shorter
-    // segments to occupy the chip (2048x2048 uint16, d = 11: 32 rows
-    // measured 0.139 ms per frame against 0.181 ms with 128)
-    int plain_seg_rows = 32;
-    bool seg_set = false;   // gt_context_set_launch_shape was called
+    int seg_rows = 128;     // rows per bandpass work item, once set
+    bool seg_set = false;   // gt_context_set_launch_shape was called (else bandpass_seg's rule)
     int fuse_walk = 1;     // run the centroid walk inside detect where supported
     // batched launch sequence captured as a graph and replayed while the
     // call's inputs, parameters and buffers are unchanged
@@ -557,6 +557,33 @@ struct FrameSizes {
 
 std::array<int64_t, 6> tune_key(uint32_t h, uint32_t w, const Geom& g) {
     return {(int64_t)h, (int64_t)w, g.R, g.kd, g.rint, g.has_pct};
+}
+
+// Strip rows of a frame's bandpass: rows times the strips across it.
+uint64_t strip_rows(uint32_t h, uint32_t w) {
+    return (uint64_t)h * ((w + K1_STRIP - 1) / K1_STRIP);
+}
+
+// Rows per bandpass work item for `total` strip rows, `frame` of them in the
+// largest frame.  An item filters 2R rows more than it writes, in whole groups
+// of NT = 2R + 1, so m NT - 2R rows waste nothing beyond that halo.  The more
+// rows the smaller its share (40 frames of 2048^2, d = 11: 338, 299, 280, 268,
+// 264 us at 23, 34, 45, 67 and 122 rows), but an item's rows are one serial
+// chain (one frame of 512^2: 17, 21, 26, 35 us at 12, 23, 34 and 56 rows), so
+// a call takes the fewest whose items the chip still holds at once.  With a
+// percentile every item adds its histogram to the frame's, and about 500 of
+// them contend for its words as long as they filter (one frame of 2048^2: 53,
+// 37, 36, 42 us at 12, 23, 34 and 56 rows; 17 us at 12 rows without).
+int bandpass_seg(const Geom& g, uint64_t total, uint64_t frame) {
+    const int nt = 2 * g.R + 1;
+    const int m_max = std::max(2, (128 + 2 * g.R) / nt);
+    const uint64_t resident = 256 * (g.R <= 7 ? 8 : g.R <= 10 ? 6 : 4);   // items on 256 CUs
+    int m = 2;
+    for (; m < m_max; ++m) {
+        const uint64_t seg = (uint64_t)(m * nt - 2 * g.R);
+        if (seg * resident >= total && (!g.has_pct || seg * 500 >= frame)) break;
+    }
+    return m * nt - 2 * g.R;
 }
 
 FrameSizes sizes_of(uint32_t h, uint32_t w, int seg) {
@@ -802,7 +829,17 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     GT_TRY(make_geom(p, integer_input, g));
     g.walk_in_detect = ctx->fuse_walk && walk_in_detect_supported(g) ? 1 : 0;
     // autotuned launch shape for calls whose frames all share one shape
-    int seg = plain && !ctx->seg_set ? ctx->plain_seg_rows : ctx->seg_rows;
+    int seg = ctx->seg_rows;
+    if (!ctx->seg_set) {
+        uint64_t total = 0, largest = 0;
+        for (const auto& f : frames) {
+            const uint64_t r = strip_rows(f.h, f.w);
+            total += r;
+            largest = std::max(largest, r);
+        }
+        // on the per-frame path every frame is a launch of its own
+        seg = bandpass_seg(g, plain ? largest : total, largest);
+    }
     uint32_t batch_frames = ctx->batch_frames;
     if (!frames.empty() && ctx->batch_frames == 0 && !plain) {
         bool uniform = true;
@@ -827,20 +864,9 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     if (adj && !adjoint_supported(g))
         return fail(GT_E_NOT_IMPLEMENTED, "adjoint needs (2*rint+1)^2 <= 1024 and smoothing_size/2 <= 16");
     const size_t es = elem_size(in_type);
-    // vector loads need W % 4 == 0 and frame bases aligned to 4 pixels
-    bool vec = true;
-    for (const auto& f : frames) {
-        if (f.w % 4 != 0) vec = false;
-        if (on_device && ((uintptr_t)f.ptr) % (4 * es) != 0) vec = false;
-    }
-    bool generic;
-    {
-        Batch probe;
-        std::memset(&probe, 0, sizeof(probe));
-        probe.in_type = in_type;
-        probe.vec = vec ? 1 : 0;
-        generic = !bandpass_fast_path(probe, g);
-    }
+    uint32_t min_w = UINT32_MAX;
+    for (const auto& f : frames) min_w = std::min(min_w, f.w);
+    const bool generic = !bandpass_fast_path(in_type, min_w, g);
     // per-frame tmp planes: the generic bandpass's row pass, or the row
     // maxima of a dilation window too wide for detect's staged tile
     const bool tmp_planes = generic || detect_needs_plane(g);
@@ -1055,7 +1081,6 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             b.dblock_tile = b.tile_frame + b.tiles;
             b.dblocks = dblocks_of[bi];
             b.in_type = in_type;
-            b.vec = vec ? 1 : 0;
             char* t3 = w.tile3.as<char>();
             const size_t t3s = al256(maxneed.tiles * 4);
             b.tile_count = (uint32_t*)t3;
@@ -1542,6 +1567,7 @@ gt_status gt_context_autotune(gt_context* ctx, const gt_params* p, uint32_t h, u
                             bg.data(), 7));
     }
     const int saved_seg = ctx->seg_rows;
+    const bool saved_set = ctx->seg_set;
     const uint32_t saved_batch = ctx->batch_frames;
     const int saved_graphs = ctx->graphs;
     const int saved_fuse = ctx->fuse_walk;
@@ -1558,10 +1584,10 @@ gt_status gt_context_autotune(gt_context* ctx, const gt_params* p, uint32_t h, u
     for (int fz = 0; fz < nfuse && st == GT_OK; ++fz) {
         ctx->fuse_walk = fz == 0 ? saved_fuse : 0;
         for (int sg : segs) {
-            if (g.has_pct && (int64_t)K1_STRIP * sg >= 65536) continue;
             for (uint32_t bf : batches) {
                 if (bf && bf >= n_frames) continue;
                 ctx->seg_rows = sg;
+                ctx->seg_set = true;
                 ctx->batch_frames = bf;
                 double ms = 1e30;
                 for (int rep = 0; rep < 3 && st == GT_OK; ++rep) {
@@ -1583,6 +1609,7 @@ gt_status gt_context_autotune(gt_context* ctx, const gt_params* p, uint32_t h, u
         }
     }
     ctx->seg_rows = saved_seg;
+    ctx->seg_set = saved_set;
     ctx->batch_frames = saved_batch;
     ctx->graphs = saved_graphs;
     ctx->fuse_walk = saved_fuse;
@@ -1823,18 +1850,17 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
     GT_TRY(make_geom(p, integer_input, g));
     g.walk_in_detect = ctx->fuse_walk && walk_in_detect_supported(g) ? 1 : 0;
     const size_t es = elem_size(in_type);
-    const bool vec = w % 4 == 0 && ((uintptr_t)frames) % (4 * es) == 0;
-    bool generic;
-    {
-        Batch probe;
-        std::memset(&probe, 0, sizeof(probe));
-        probe.in_type = in_type;
-        probe.vec = vec ? 1 : 0;
-        generic = !bandpass_fast_path(probe, g);
-    }
-    const bool tmp_planes = generic || detect_needs_plane(g);
-    const int seg = ctx->seg_set ? ctx->seg_rows : 128;
-    const FrameSizes fs = sizes_of(h, w, seg);
+    const bool generic = !bandpass_fast_path(in_type, w, g);
+    // Which frames fit the scratch is part of this entry point's contract, so
+    // frames that the bandpass once took through temporary planes (unaligned
+    // rows, wide filters) keep them counted although they are not used.
+    const bool tmp_planes = generic || detect_needs_plane(g) || g.R > 8 || w % 4 != 0 ||
+                            ((uintptr_t)frames) % (4 * es) != 0;
+    // the rule's rows per item may need more table entries than 128 rows do:
+    // a frame that fits only with those takes them
+    int seg = ctx->seg_set ? ctx->seg_rows
+                           : bandpass_seg(g, n * strip_rows(h, w), strip_rows(h, w));
+    FrameSizes fs = sizes_of(h, w, seg);
     const uint64_t dblocks_pf = (uint64_t)((fs.ty + 1) / 2) * ((fs.tx + 1) / 2);  // dedup blocks
 
     // scratch layout for nb frames, every part 256-byte aligned
@@ -1872,6 +1898,10 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
                3 * (nb + 1) <= gt_context::kNaBases;
     };
     if (n == 0) return GT_OK;
+    if (!fits(1) && !ctx->seg_set) {
+        seg = 128;
+        fs = sizes_of(h, w, seg);
+    }
     if (!fits(1))
         return fail(GT_E_INVALID,
                     "a %ux%u frame needs %zu bytes of scratch; gt_locate_noalloc holds %u",
@@ -1946,7 +1976,6 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
         b.k1_items = nb * fs.k1_items;
         b.tiles = nb * fs.tiles;
         b.in_type = in_type;
-        b.vec = vec ? 1 : 0;
         char* t3 = base + L.tile3;
         const size_t t3s = al256(L.tiles * 4);
         b.tile_count = (uint32_t*)t3;

@@ -22,8 +22,8 @@ constexpr int TILE_H = 64;
 constexpr int TILE_W = 48;
 constexpr int TILE_PX = TILE_H * TILE_W;
 
-// Bandpass (K1) column strip: 64 lanes x 4 columns.
-constexpr int K1_STRIP = 240;   // output columns per bandpass work item
+// Bandpass (K1) column strip: two waves of 64 lanes x 2 columns.
+constexpr int K1_STRIP = 256;   // output columns per bandpass work item
 
 // Raw signal extraction: taps of the signal disk and of the background
 // annulus (each at most RAW_MAX_TAPS, offsets within +-127).
@@ -106,7 +106,6 @@ struct Batch {
     uint32_t tiles;
     uint32_t dblocks;
     int in_type;           // InType
-    int vec;               // W % 4 == 0 and aligned frame bases: vector loads
     // per-tile arrays [tiles]
     uint32_t* tile_count;
     uint32_t* tile_keep;
@@ -146,9 +145,10 @@ struct AdjOut {
 // Launchers (gt_kernels.hip, gt_bandpass.hip, gt_detect.hip).  All launch on
 // `s`; return hipSuccess or the first launch error.
 hipError_t launch_zero_batch(const Batch& b, hipStream_t s);
-// The streaming bandpass handles uint8, uint16 and float32 input with 1 <= R <= 8, W % 4 == 0
-// and aligned frame bases (b.vec); everything else takes the generic kernels.
-bool bandpass_fast_path(const Batch& b, const Geom& g);
+// The streaming bandpass handles every input type with 1 <= R <= 16 (all that
+// smoothing_size allows but 1) and frames at least min_w >= 2 pixels wide;
+// the rest takes the generic kernels.
+bool bandpass_fast_path(int in_type, uint32_t min_w, const Geom& g);
 hipError_t launch_bandpass(const Batch& b, const Geom& g, const Geom* d_geom,
                            int seg_rows, hipStream_t s);
 hipError_t launch_bandpass_generic(const Batch& b, const Geom* d_geom, uint32_t max_px,

@@ -92,3 +92,31 @@ def test_full_frame_2048(ctx):
     names = [n for n, _ in cols]
     assert rows.shape[0] > 1000
     _check(v, rows, names, 3.0, 7.5, 1.0, every=13)
+
+
+@pytest.mark.parametrize("dtype", ["u16", "u8", "f32"])
+@pytest.mark.parametrize("sig,bg,gap", [
+    (1.0, 3.0, 0.0),      # 29 - 5 + ring: one background tap per lane
+    (2.0, 6.0, 0.0),      # two
+    (3.0, 8.0, 0.0),      # three
+    (2.0, 9.0, 0.0),      # four
+    (3.0, 10.0, 0.0),     # five
+    (2.0, 11.0, 0.0),     # six
+    (3.0, 12.0, 0.0),     # seven
+    (2.0, 12.7, 0.0),     # eight
+    (3.0, 16.0, 1.0),     # more than 512: keys in LDS
+    (9.5, 12.0, 0.5),     # more than 256 signal taps
+    (2.0, 2.0, 1.0),      # no background tap: NaN
+])
+def test_tap_counts(dtype, sig, bg, gap):
+    """Every number of background taps per lane, even and odd counts of taps
+    inside the frame (rows near its edges) and many equal values."""
+    rng = np.random.default_rng(int(100 * sig + bg))
+    v = rng.integers(0, 40, (2, 71, 93)) + 3 * rng.integers(0, 2, (2, 71, 93))
+    v[:, 10:60:7, 8:90:9] += 60
+    v = {"u8": v.astype(np.uint8), "u16": (v * 500).astype(np.uint16),
+         "f32": (v * 0.37 - 9).astype(np.float32)}[dtype]
+    rows, cols = batch_rust(v, 5, separation=5, sig_radius=sig, bg_radius=bg, gap_radius=gap)
+    names = [n for n, _ in cols]
+    assert len(rows) > 60
+    _check(v, rows, names, sig, bg, gap)

@@ -281,6 +281,9 @@ gt_status make_geom(const gt_params* p, bool integer_input, Geom& g) {
             return fail(GT_E_INVALID, "sig_radius/bg_radius give more than %d taps", RAW_MAX_TAPS);
         g.raw_ns = (int32_t)st.size();
         g.raw_nb = (int32_t)bt.size();
+        for (const auto* v : {&st, &bt})
+            for (const auto& t : *v)
+                g.raw_reach = std::max({g.raw_reach, std::abs(t.first), std::abs(t.second)});
         int k = 0;
         for (const auto& t : st) {
             g.raw_tap[k++] = (int8_t)t.first;

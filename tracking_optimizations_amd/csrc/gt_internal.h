@@ -89,6 +89,7 @@ struct Geom {
     int32_t raw_cols;      // 0, 1 (raw_mass) or 3 (+ raw_bg_median, raw_mass_corrected)
     int32_t col_raw;       // output column of raw_mass
     int32_t raw_ns, raw_nb;  // signal and background tap counts
+    int32_t raw_reach;       // no tap is further off than this along an axis
     int8_t raw_tap[4 * RAW_MAX_TAPS];  // (dy, dx) of the signal taps, then the background taps
     float sin2_gpu[1024], cos2_gpu[1024];                // disk radius rint
     float r2_cpu[1024], sin_cpu[1024], cos_cpu[1024];    // circle radius band

@@ -148,3 +148,62 @@ def rows_origin(video, p, ctx):
     """Rows, candidates and the last evaluated disk's patch origin per row."""
     rows, cand, _, a = locate_errors(video, p, ctx=ctx)
     return rows, cand, a.origin().copy()
+
+
+@pytest.mark.parametrize("diameter", range(3, 18))
+def test_every_filter_width_and_frame_edges(ctx, diameter):
+    """Diameters 3 to 17 with their default smoothing (a register kernel per
+    radius up to 15, the LDS form beyond), uneven background so that the clamp
+    is active on some disks, spots on the border of the candidate area so that
+    patches leave the frame on every side; odd frame sizes."""
+    rng = np.random.default_rng(diameter)
+    h, w = 4 * diameter + 31, 5 * diameter + 40
+    frame = rng.poisson(60, (2, h, w)).astype(np.float64)
+    band = diameter // 2
+    yy, xx = np.mgrid[:h, :w]
+    spots = [(band, w // 2), (h - 1 - band, w // 3), (h // 2, band), (h // 3, w - 1 - band),
+             (band + 1, band + 1), (h // 2, w // 2)]
+    for f in range(2):
+        for y, x in spots:
+            frame[f] += 900 * np.exp(-((yy - y) ** 2 + (xx - x) ** 2) / (2 * (0.18 * diameter + 0.4) ** 2))
+    frame = frame.astype(np.uint16)
+    kw = dict(diameter=diameter, separation=diameter + 1, minmass=0.0)
+    p = make_params(**kw)
+    rows, cand, sigma, a = locate_errors(frame, p, ctx=ctx, jacobian=True)
+    jac, org = a.jacobian(), a.origin()
+    op = oracle.Params(**kw)
+    S = jac.shape[2]
+    outside = (org[:, 0] < 0) | (org[:, 1] < 0) | (org[:, 0] + S > h) | (org[:, 1] + S > w)
+    assert outside.any()
+    pick = np.concatenate([np.flatnonzero(outside)[:10], np.flatnonzero(~outside)[:6]])
+    for i in pick:
+        f32 = frame[int(rows[i, 0])].astype(np.float32)
+        jo, oo, _, _ = oracle.adjoint_particle(f32, op, int(cand[i]), f64_forward=False)
+        assert tuple(org[i]) == oo
+        assert np.abs(jac[i] - jo).max() <= JAC_TOL * np.abs(jo).max(), (i, oo)
+        so = _oracle_sigma(jo, oo, f32)
+        assert np.all(np.abs(sigma[i] - so) <= SIGMA_TOL * so), (i, oo)
+
+
+def test_vjp_tiles(ctx):
+    """Patches across and inside the VJP's 64 x 32 tiles, a last tile of one
+    row and one column, frames without rows in between."""
+    rng = np.random.default_rng(5)
+    frames = rng.poisson(40, (3, 65, 129)).astype(np.uint16)
+    frames[1] = 0
+    for y, x in [(31, 63), (32, 64), (10, 10), (60, 120), (40, 64)]:
+        frames[0, y - 1:y + 2, x - 1:x + 2] += 500
+        frames[2, y - 1:y + 2, x - 1:x + 2] += 300
+    p = make_params(9, minmass=100.0)
+    rows, _, _, a = locate_errors(frames, p, ctx=ctx, jacobian=True)
+    jac, org = a.jacobian(), a.origin()
+    g = rng.normal(size=(len(rows), 3)).astype(np.float32)
+    got = a.vjp(ctx, g)
+    want = np.zeros((3, 65 + 64, 129 + 64), np.float64)
+    S = jac.shape[2]
+    for i in range(len(rows)):
+        y0, x0 = org[i] + 32
+        want[int(rows[i, 0]), y0:y0 + S, x0:x0 + S] += np.tensordot(g[i].astype(np.float64), jac[i], axes=1)
+    want = want[:, 32:32 + 65, 32:32 + 129]
+    assert not rows[:, 0].__eq__(1).any() and not got[1].any()
+    assert np.abs(got - want).max() <= 1e-6 * np.abs(want).max()

@@ -22,8 +22,9 @@
 // patches of a frame's rows in row order, one workgroup per frame, so the
 // gradient is deterministic.
 #include <algorithm>
+#include <type_traits>
 
-#include "gt_internal.h"
+#include "gt_device.h"
 
 #pragma clang fp contract(off)
 
@@ -356,38 +357,328 @@ __global__ __launch_bounds__(64) void k_adjoint_sep(Batch b, const Geom* __restr
     }
 }
 
-// grad[f] += sum over the frame's rows, in row order, of
-// gy * J_y + gx * J_x + gm * J_mass on each row's patch.
-__global__ __launch_bounds__(256) void k_adjoint_vjp(const float* __restrict__ jac,
-                                                    const int32_t* __restrict__ origin,
-                                                    const uint64_t* __restrict__ frame_rows,
-                                                    const float* __restrict__ grad_rows,
-                                                    float* __restrict__ grad, int S, int H,
-                                                    int W) {
+// The separable adjoint with everything in registers, for the usual filters
+// (smoothing size equal to the diameter: R = RINT, or RINT + 1 for even
+// ones).  A lane holds one column of a row's S x S patch and G = 64 / S rows
+// share a wave, so the inner sums run over registers with constant indices.
+//  * A wave takes a run of rows; lane = row replays the walks (the forward's
+//    own arithmetic).
+//  * The disk adjoint A_o(i, j) = on(i, j) f_o with f_y = (i - c0) / m,
+//    f_x = (j - c1) / m, f_mass = 1, so two column passes serve the three
+//    outputs: S_i(c) = sum_j w[c - j] on(i, j) and U_i(c) with f_x; y and
+//    mass share S_i.  The boxcar's passes are the same with unit weights.
+//  * The row pass is Gaussian FMAs over i; the boxcar's window over i is a
+//    prefix or a suffix of the D rows (D <= 2R + 1), a running sum from
+//    either end.  Patches that leave the frame take the mirror
+//    multiplicities (box_count) instead.
+// The two norms multiply as reciprocals of two parts, so no output divides.
+//
+// Bound by issued instructions, about 400 per row at d = 9: 64 frames of
+// 512^2 (80 k rows) in 119 us, against 605 us for the form above with its
+// tables in LDS (5 LDS reads per 6 FMAs, six divisions per patch pixel).
+template <int RINT, int R, typename T>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RINT <= 2 ? 4 : RINT <= 4 ? 3 : RINT <= 5 ? 2 : 1)))
+void k_adjoint_reg(Batch b, const Geom* __restrict__ g,
+                                                   AdjOut ao, uint32_t frame_pos0) {
+    constexpr int D = 2 * RINT + 1, NT = 2 * R + 1, S = 2 * (RINT + R) + 1;
+    constexpr int G = 64 / S;
+    static_assert(S <= 64 && D <= NT, "a patch column per lane; prefix and suffix windows");
+    const int lane = threadIdx.x;
     const uint32_t f = blockIdx.x;
-    float* gf = grad + (size_t)f * H * W;
-    const int SS = S * S;
-    for (uint64_t row = frame_rows[f]; row < frame_rows[f + 1]; ++row) {
-        const float gy = grad_rows[row * 3 + 0], gx = grad_rows[row * 3 + 1],
-                    gm = grad_rows[row * 3 + 2];
-        const int py0 = origin[row * 2 + 0], px0 = origin[row * 2 + 1];
-        const float* jr = jac + row * 3 * (size_t)SS;
-        for (int p = threadIdx.x; p < SS; p += blockDim.x) {
-            const int ry = py0 + p / S, rx = px0 + p % S;
-            if (ry < 0 || ry >= H || rx < 0 || rx >= W) continue;
-            float v = gy * jr[p];
-            v = __builtin_fmaf(gx, jr[SS + p], v);
-            v = __builtin_fmaf(gm, jr[2 * SS + p], v);
-            gf[(size_t)ry * W + rx] += v;
+    const Frame fr = b.frames[f];
+    const int H = (int)fr.H, W = (int)fr.W;
+    const GLOBAL float* P = (const GLOBAL float*)fr.P;
+    const int band = g->band;
+    const uint32_t maxit = g->max_iterations;
+    const GLOBAL T* I = (const GLOBAL T*)fr.in;
+    // 1 / k^2 and 1 / gauss_norm^2 in two parts each (their rounding would be
+    // the same error everywhere)
+    const double dkk = 1.0 / (double)g->kk, dgn = 1.0 / ((double)g->gn * (double)g->gn);
+    const float rkk = (float)dkk, rkk_lo = (float)(dkk - (double)rkk);
+    const float rgg = (float)dgn, rgg_lo = (float)(dgn - (double)rgg);
+    const float sthr = 0.6f;
+    const uint64_t base = b.frame_row_base[f];
+    if (base >= b.rows_cap) return;
+    const uint32_t nrows = (uint32_t)min((uint64_t)b.frame_rows[f], b.rows_cap - base);
+    // rows of one run: whole groups, as few as give every wave of the frame one
+    const uint32_t want = (nrows + gridDim.y - 1) / gridDim.y;
+    const uint32_t per = min((uint32_t)(64 / G * G), max(1u, (want + G - 1) / G) * G);
+    const int grp = min(lane / S, G - 1);
+    const bool lane_in = lane < G * S;
+    const int c = lane_in ? lane % S : 0;
+
+    float wd[R + 1];   // weights by distance
+#pragma unroll
+    for (int k = 0; k <= R; ++k) wd[k] = g->w[R + k];
+    float wl[D];       // this lane's column weights w[c - j]
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+        const int k = c - j - R;   // offset of the tap
+        wl[j] = abs(k) <= R ? g->w[R + k] : 0.f;
+    }
+
+    for (uint32_t q0 = blockIdx.y * per; q0 < nrows; q0 += gridDim.y * per) {
+        const int n = (int)min(per, nrows - q0);
+        // forward walk (refine's arithmetic), lane = row
+        const int64_t pix = b.rows_cand[base + q0 + (uint32_t)min(lane, n - 1)];
+        int u = (int)(pix / W), v = (int)(pix % W);
+        int ue = u, ve = v, live = 0;   // live: the last disk lay inside the frame
+        float m = 0.f, c0 = 0.f, c1 = 0.f;
+        if (lane < n) {
+            for (uint32_t it = 0; it < maxit; ++it) {
+                ue = u;
+                ve = v;
+                if (u - band < 0 || u + band >= H || v - band < 0 || v + band >= W) {
+                    m = 0.f; c0 = 0.f; c1 = 0.f;
+                    live = 0;
+                } else {
+                    const GLOBAL float* p = P + (size_t)u * W + v;
+                    float s0 = 0.f, s1 = 0.f, ms = 0.f;
+#pragma unroll
+                    for (int i = -RINT; i <= RINT; ++i)
+#pragma unroll
+                        for (int j = -RINT; j <= RINT; ++j) {
+                            if (i * i + j * j > RINT * RINT) continue;
+                            const float d = p[(ptrdiff_t)i * W + j];
+                            s0 = __builtin_fmaf(d, (float)i, s0);
+                            s1 = __builtin_fmaf(d, (float)j, s1);
+                            ms = ms + d;
+                        }
+                    m = ms;
+                    c0 = s0 / ms;
+                    c1 = s1 / ms;
+                    live = 1;
+                }
+                bool changed = false;
+                if (c0 > sthr && u < H - 1) { u += 1; changed = true; }
+                else if (c0 < -sthr && u > 0) { u -= 1; changed = true; }
+                if (c1 > sthr && v < W - 1) { v += 1; changed = true; }
+                else if (c1 < -sthr && v > 0) { v -= 1; changed = true; }
+                if (!changed) break;
+            }
         }
-        __syncthreads();  // rows in order: overlapping patches add deterministically
+        if (m == 0.f) live = 0;
+        if (!live) c0 = c1 = 0.f;
+
+        for (int i0 = 0; i0 < n; i0 += G) {
+            const int idx = min(i0 + grp, n - 1);   // the lane's row within the run
+            const bool own = lane_in && i0 + grp < n;
+            const int gu = __shfl(ue, idx, 64), gv = __shfl(ve, idx, 64);
+            const int glive = __shfl(live, idx, 64);
+            const float gm = __shfl(m, idx, 64), gc0 = __shfl(c0, idx, 64), gc1 = __shfl(c1, idx, 64);
+            const uint64_t row = base + q0 + (uint32_t)idx;
+            const int py0 = gu - RINT - R, px0 = gv - RINT - R;
+            // a row without mass pulls nothing back: its (clamped) disk is
+            // read but every weight is zero
+            const float on1 = glive ? 1.f : 0.f;
+            const float rm = glive ? 1.f / gm : 0.f;
+            const int du = min(max(gu, RINT), max(H - 1 - RINT, RINT));
+            const int dv = min(max(gv, RINT), max(W - 1 - RINT, RINT));
+            double var[3] = {0.0, 0.0, 0.0};
+            // EDGE: some patch of the group leaves the frame
+            auto patches = [&](auto edge_c) {
+                constexpr bool EDGE = decltype(edge_c)::value;
+                // column pass
+                float bw[D], wf[D], bf[D];
+#pragma unroll
+                for (int j = 0; j < D; ++j) {
+                    const float fj = ((float)(j - RINT) - gc1) * rm;
+                    if constexpr (EDGE) bw[j] = box_count(gv + j - RINT, px0 + c, R, W);
+                    else bw[j] = abs(c - j - R) <= R ? 1.f : 0.f;
+                    wf[j] = wl[j] * fj;
+                    bf[j] = bw[j] * fj;
+                }
+                float sg[D], ug[D], sb[D], ub[D];
+                const GLOBAL float* disk = P + (size_t)du * W + dv;
+#pragma unroll
+                for (int i = 0; i < D; ++i) {
+                    sg[i] = ug[i] = sb[i] = ub[i] = 0.f;
+#pragma unroll
+                    for (int j = 0; j < D; ++j) {
+                        if ((i - RINT) * (i - RINT) + (j - RINT) * (j - RINT) > RINT * RINT) continue;
+                        const float on = disk[(ptrdiff_t)(i - RINT) * W + (j - RINT)] > 0.f ? on1 : 0.f;
+                        sg[i] = __builtin_fmaf(on, wl[j], sg[i]);
+                        ug[i] = __builtin_fmaf(on, wf[j], ug[i]);
+                        sb[i] = __builtin_fmaf(on, bw[j], sb[i]);
+                        ub[i] = __builtin_fmaf(on, bf[j], ub[i]);
+                    }
+                }
+                // row pass: outputs y, x, mass; y's terms carry f_y(i)
+                float yg[D], yb[D];
+#pragma unroll
+                for (int i = 0; i < D; ++i) {
+                    const float fi = ((float)(i - RINT) - gc0) * rm;
+                    yg[i] = fi * sg[i];
+                    yb[i] = fi * sb[i];
+                }
+                const bool cin = px0 + c >= 0 && px0 + c < W;
+                // first pixel of this lane's column (interior; rows that hold
+                // no patch read the first one's)
+                const GLOBAL T* col = I + (size_t)max(py0, 0) * W + max(px0, 0) + c;
+                float* const jp = ao.jac ? ao.jac + (size_t)row * 3 * (S * S) + c : nullptr;
+                // one patch row; run: the boxcar windows' running sums (interior)
+                auto patch_row = [&](int r, const float (&run)[3]) {
+                    float bo[3] = {run[0], run[1], run[2]};
+                    if constexpr (EDGE) {
+                        bo[0] = bo[1] = bo[2] = 0.f;
+#pragma unroll
+                        for (int i = 0; i < D; ++i) {
+                            const float k = box_count(gu + i - RINT, py0 + r, R, H);
+                            bo[0] = __builtin_fmaf(k, yb[i], bo[0]);
+                            bo[1] = __builtin_fmaf(k, ub[i], bo[1]);
+                            bo[2] = __builtin_fmaf(k, sb[i], bo[2]);
+                        }
+                    }
+                    float ga = 0.f, gb = 0.f, gc = 0.f;
+#pragma unroll
+                    for (int i = 0; i < D; ++i) {
+                        const int k = r - i - R;
+                        if (k < -R || k > R) continue;
+                        const float w = wd[k < 0 ? -k : k];
+                        ga = __builtin_fmaf(w, yg[i], ga);
+                        gb = __builtin_fmaf(w, ug[i], gb);
+                        gc = __builtin_fmaf(w, sg[i], gc);
+                    }
+                    auto term = [&](float ga_, float bo_) {   // ga / gn^2 - bo / k^2
+                        const float t = __builtin_fmaf(ga_, rgg_lo, ga_ * rgg);
+                        return __builtin_fmaf(-bo_, rkk, __builtin_fmaf(-bo_, rkk_lo, t));
+                    };
+                    float jo[3] = {term(ga, bo[0]), term(gb, bo[1]), term(gc, bo[2])};
+                    float pixel;
+                    if constexpr (EDGE) {
+                        const int ry = py0 + r, rx = px0 + c;
+                        const bool in = cin && ry >= 0 && ry < H;
+                        pixel = (float)I[(size_t)min(max(ry, 0), H - 1) * W + min(max(rx, 0), W - 1)];
+#pragma unroll
+                        for (int o = 0; o < 3; ++o) jo[o] = in ? jo[o] : 0.f;
+                    } else {
+                        pixel = (float)col[(size_t)r * W];
+                    }
+                    const double lam = (double)fmaxf(pixel, 0.f);
+#pragma unroll
+                    for (int o = 0; o < 3; ++o)
+                        var[o] = __builtin_fma((double)jo[o] * (double)jo[o], lam, var[o]);
+                    if (jp && own) {
+#pragma unroll
+                        for (int o = 0; o < 3; ++o) jp[o * (S * S) + r * S] = jo[o];
+                    }
+                };
+                // boxcar windows: rows r < D the prefix 0..r, r > 2R the
+                // suffix r - 2R .. D - 1 (from the last row upwards), in
+                // between all
+                float run[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+                for (int r = 0; r <= 2 * R; ++r) {
+                    if (r < D) { run[0] += yb[r]; run[1] += ub[r]; run[2] += sb[r]; }
+                    patch_row(r, run);
+                }
+                run[0] = run[1] = run[2] = 0.f;
+#pragma unroll
+                for (int r = S - 1; r > 2 * R; --r) {
+                    run[0] += yb[r - 2 * R]; run[1] += ub[r - 2 * R]; run[2] += sb[r - 2 * R];
+                    patch_row(r, run);
+                }
+            };
+            if (__ballot(py0 < 0 || px0 < 0 || py0 + S > H || px0 + S > W)) patches(std::true_type{});
+            else patches(std::false_type{});
+            // sum over the S lanes of the row
+            constexpr int P2 = S > 32 ? 32 : S > 16 ? 16 : S > 8 ? 8 : S > 4 ? 4 : 2;
+#pragma unroll
+            for (int d = P2; d > 0; d >>= 1)
+#pragma unroll
+                for (int o = 0; o < 3; ++o) {
+                    const double t = __shfl_down(var[o], d, 64);
+                    if (c + d < S) var[o] += t;
+                }
+            if (own && c == 0) {
+                // output order: y, x, mass
+#pragma unroll
+                for (int o = 0; o < 3; ++o) ao.sigma[row * 3 + o] = (float)sqrt(var[o]);
+                ao.origin[row * 2 + 0] = py0;
+                ao.origin[row * 2 + 1] = px0;
+                ao.rowpos[row] = (int32_t)(frame_pos0 + f);
+            }
+        }
     }
 }
 
-__global__ void k_fill_f32(float* p, uint64_t n, float v) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        p[i] = v;
+// grad[f] = sum over the frame's rows, in row order, of
+// gy * J_y + gx * J_x + gm * J_mass on each row's patch.  One wave per
+// VT_W x VT_H tile of a frame: the frame's rows are tested 64 at a time, the
+// patches that touch the tile are added in row order to the tile in LDS
+// (every pixel receives its terms in that order, whatever the tiling), and
+// the tile is written once.  Bound by the reads of the patches: 24 frames of
+// 512^2 in 17 us (a workgroup per frame over its rows and a fill of the
+// gradient before: about 250 us).
+constexpr int VT_W = 64, VT_H = 32;
+__global__ __launch_bounds__(64) void k_adjoint_vjp(const float* __restrict__ jac,
+                                                   const int32_t* __restrict__ origin,
+                                                   const uint64_t* __restrict__ frame_rows,
+                                                   const float* __restrict__ grad_rows,
+                                                   float* __restrict__ grad, int S, int H,
+                                                   int W) {
+    __shared__ float acc[VT_H * VT_W];
+    const int lane = threadIdx.x;
+    const int tx = (W + VT_W - 1) / VT_W, ty = (H + VT_H - 1) / VT_H;
+    const uint32_t f = blockIdx.x / (uint32_t)(tx * ty);
+    const int tile = (int)(blockIdx.x % (uint32_t)(tx * ty));
+    const int x0 = tile % tx * VT_W, y0 = tile / tx * VT_H;
+    const int SS = S * S;
+#pragma unroll
+    for (int r = 0; r < VT_H; ++r) acc[r * VT_W + lane] = 0.f;
+    const uint64_t e = frame_rows[f + 1];
+    for (uint64_t rb = frame_rows[f]; rb < e; rb += 64) {
+        const uint64_t mine = min(rb + (uint64_t)lane, e - 1);
+        const int oy = origin[mine * 2], ox = origin[mine * 2 + 1];
+        const bool hit = rb + (uint64_t)lane < e && oy < y0 + VT_H && oy + S > y0 && ox < x0 + VT_W &&
+                         ox + S > x0;
+        for (uint64_t todo = __ballot(hit); todo; todo &= todo - 1) {
+            const int q = __ffsll((long long)todo) - 1;
+            const uint64_t row = rb + (uint64_t)q;
+            const int py0 = __builtin_amdgcn_readlane(oy, q), px0 = __builtin_amdgcn_readlane(ox, q);
+            const float gy = grad_rows[row * 3 + 0], gx = grad_rows[row * 3 + 1],
+                        gm = grad_rows[row * 3 + 2];
+            const float* jr = jac + row * 3 * (size_t)SS;
+            // the part of the patch inside the tile
+            const int ra = max(0, y0 - py0), rz = min(S, y0 + VT_H - py0);
+            const int ca = max(0, x0 - px0), cw = min(S, x0 + VT_W - px0) - ca;
+            const int cnt = (rz - ra) * cw;
+            for (int p = lane; p < cnt; p += 64) {
+                const int r = ra + p / cw, c = ca + p % cw;
+                const int at = r * S + c;
+                float v = gy * jr[at];
+                v = __builtin_fmaf(gx, jr[SS + at], v);
+                v = __builtin_fmaf(gm, jr[2 * SS + at], v);
+                acc[(py0 + r - y0) * VT_W + (px0 + c - x0)] += v;
+            }
+            // the wave's LDS operations keep their order; so must the compiler
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+    }
+    __syncthreads();
+    float* gf = grad + (size_t)f * H * W;
+    if (x0 + lane < W) {
+        for (int r = 0; r < min(VT_H, H - y0); ++r)
+            gf[(size_t)(y0 + r) * W + x0 + lane] = acc[r * VT_W + lane];
+    }
+}
+
+template <int RINT, int R>
+hipError_t launch_adjoint_reg(const Batch& b, const Geom* d_geom, const AdjOut& ao,
+                              uint32_t frame_pos0, hipStream_t s) {
+    // about eight waves per SIMD in all, and enough of them where one frame
+    // has all the rows
+    const uint32_t per_frame = std::max(32u, std::min(512u, 8192u / std::max(b.nframes, 1u)));
+    const dim3 grid(b.nframes, per_frame), block(64);
+    if (b.in_type == IN_U16)
+        hipLaunchKernelGGL((k_adjoint_reg<RINT, R, uint16_t>), grid, block, 0, s, b, d_geom, ao, frame_pos0);
+    else if (b.in_type == IN_U8)
+        hipLaunchKernelGGL((k_adjoint_reg<RINT, R, uint8_t>), grid, block, 0, s, b, d_geom, ao, frame_pos0);
+    else
+        hipLaunchKernelGGL((k_adjoint_reg<RINT, R, float>), grid, block, 0, s, b, d_geom, ao, frame_pos0);
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -405,6 +696,24 @@ size_t adjoint_sep_lds(const Geom& g) {
 
 hipError_t launch_adjoint(const Batch& b, const Geom& g, const Geom* d_geom, const AdjOut& ao,
                           uint32_t frame_pos0, hipStream_t s) {
+    if (g.R == g.rint || g.R == g.rint + 1) {
+        switch (2 * g.rint + (g.R - g.rint)) {
+            case 2: return launch_adjoint_reg<1, 1>(b, d_geom, ao, frame_pos0, s);
+            case 3: return launch_adjoint_reg<1, 2>(b, d_geom, ao, frame_pos0, s);
+            case 4: return launch_adjoint_reg<2, 2>(b, d_geom, ao, frame_pos0, s);
+            case 5: return launch_adjoint_reg<2, 3>(b, d_geom, ao, frame_pos0, s);
+            case 6: return launch_adjoint_reg<3, 3>(b, d_geom, ao, frame_pos0, s);
+            case 7: return launch_adjoint_reg<3, 4>(b, d_geom, ao, frame_pos0, s);
+            case 8: return launch_adjoint_reg<4, 4>(b, d_geom, ao, frame_pos0, s);
+            case 9: return launch_adjoint_reg<4, 5>(b, d_geom, ao, frame_pos0, s);
+            case 10: return launch_adjoint_reg<5, 5>(b, d_geom, ao, frame_pos0, s);
+            case 11: return launch_adjoint_reg<5, 6>(b, d_geom, ao, frame_pos0, s);
+            case 12: return launch_adjoint_reg<6, 6>(b, d_geom, ao, frame_pos0, s);
+            case 13: return launch_adjoint_reg<6, 7>(b, d_geom, ao, frame_pos0, s);
+            case 14: return launch_adjoint_reg<7, 7>(b, d_geom, ao, frame_pos0, s);
+            default: break;
+        }
+    }
     const size_t lds = adjoint_sep_lds(g);
     if (lds <= 48 * 1024)
         hipLaunchKernelGGL(k_adjoint_sep, dim3(b.nframes, 64), dim3(64), lds, s, b, d_geom, ao,
@@ -418,14 +727,18 @@ hipError_t launch_adjoint(const Batch& b, const Geom& g, const Geom* d_geom, con
 hipError_t launch_adjoint_vjp(const float* jac, const int32_t* origin, const uint64_t* frame_rows,
                               uint32_t nframes, const float* grad_rows, float* grad, int S, int H,
                               int W, hipStream_t s) {
-    const uint64_t n = (uint64_t)nframes * H * W;
-    const uint32_t blocks = (uint32_t)std::min<uint64_t>((n + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_fill_f32, dim3(std::max(blocks, 1u)), dim3(256), 0, s, grad, n, 0.f);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || nframes == 0) return e;
-    hipLaunchKernelGGL(k_adjoint_vjp, dim3(nframes), dim3(256), 0, s, jac, origin, frame_rows,
-                       grad_rows, grad, S, H, W);
-    return hipGetLastError();
+    if (nframes == 0 || H <= 0 || W <= 0) return hipSuccess;
+    const uint64_t tiles = (uint64_t)((W + VT_W - 1) / VT_W) * ((H + VT_H - 1) / VT_H);
+    // a launch holds fewer than 2^31 workgroups: whole frames at a time
+    const uint32_t most = (uint32_t)std::max<uint64_t>(1, (1ull << 30) / tiles);
+    for (uint32_t f0 = 0; f0 < nframes; f0 += most) {
+        const uint32_t nf = std::min(most, nframes - f0);
+        hipLaunchKernelGGL(k_adjoint_vjp, dim3((uint32_t)(nf * tiles)), dim3(64), 0, s, jac, origin,
+                           frame_rows + f0, grad_rows, grad + (size_t)f0 * H * W, S, H, W);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace gt

@@ -25,8 +25,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libgpu_tracking.so")
 KERNEL_SOURCES = ["gt_detect.hip", "gt_bandpass_u16.hip", "gt_bandpass_u8.hip",
                   "gt_bandpass_f32.hip", "gt_bandpass.hip", "gt_kernels.hip"]
-SOURCES = [*KERNEL_SOURCES, "gt_synth.hip", "gt_adjoint.hip", "gt_link.hip", "gt_raw.hip",
-           "gt_ingest.hip", "gt_api.hip"]
+SOURCES = [*KERNEL_SOURCES, "gt_synth.hip", "gt_adjoint.hip", "gt_link.hip", "gt_char.hip",
+           "gt_raw.hip", "gt_ingest.hip", "gt_api.hip"]
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 

@@ -333,6 +333,7 @@ gt_status make_geom(const gt_params* p, bool integer_input, Geom& g) {
             if (i * i + j * j > g.rint * g.rint) continue;
             if (t >= 1024) return fail(GT_E_INVALID, "diameter too large for characterisation");
             const float a = 2.0f * atan2f((float)j, (float)i);
+            g.r2_gpu[t] = (float)(i * i + j * j);
             g.sin2_gpu[t] = sinf(a);
             g.cos2_gpu[t] = cosf(a);
             ++t;
@@ -602,8 +603,6 @@ FrameSizes sizes_of(uint32_t h, uint32_t w, int seg) {
 }
 
 int rec_planes(const Geom& g) {
-    if (g.characterize) return REC_NPLANES;
-    if (g.cpu_processed) return REC_SIGNAL + 1;
     if (g.walk_in_detect && g.has_pct) return REC_CENTER + 1;
     return REC_X + 1;
 }
@@ -1162,6 +1161,10 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             if (nstreams > 1) HIP_TRY(hipEventRecord(ctx->ev_scan[si], st));
             HIP_TRY(stage(ctx, st, GT_STAGE_EMIT, [&] { return launch_emit(b, g, d_geom, st); }));
             launches += 5;
+            if (g.characterize || g.cpu_processed) {
+                HIP_TRY(launch_char(b, g, d_geom, st));
+                ++launches;
+            }
             if (g.raw_cols) {
                 HIP_TRY(launch_raw(b, g, d_geom, st));
                 ++launches;
@@ -1859,6 +1862,8 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
     // rows, wide filters) keep them counted although they are not used.
     const bool tmp_planes = generic || detect_needs_plane(g) || g.R > 8 || w % 4 != 0 ||
                             ((uintptr_t)frames) % (4 * es) != 0;
+    // (the same for the record planes of the characterisation columns)
+    const uint64_t rec_counted = g.characterize ? 10 : g.cpu_processed ? 6 : rec_planes(g);
     // the rule's rows per item may need more table entries than 128 rows do:
     // a frame that fits only with those takes them
     int seg = ctx->seg_set ? ctx->seg_rows
@@ -1887,7 +1892,7 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
         L.tmp = tmp_planes ? take(nb * fs.px * 8) : 0;
         L.list = g.has_pct ? take(slots * 4) : 0;
         L.slots = take(slots * 2);
-        L.rec = take(slots * 4 * (uint64_t)rec_planes(g));
+        L.rec = take(slots * 4 * rec_counted);
         L.keep = take(slots);
         L.tile3 = take(al256(L.tiles * 4) * 4 + 2 * al256(L.tiles * 4 * TILE_H));
         L.perframe = take(al256(nb * HIST_BINS * 4) + 3 * al256(nb * 4) + al256(nb * 16) +
@@ -2022,6 +2027,7 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
         HIP_TRY(launch_tile_scan(b, fs.ty, st));
         HIP_TRY(launch_frame_scan(b, st));
         HIP_TRY(launch_emit(b, g, d_geom, st));
+        if (g.characterize || g.cpu_processed) HIP_TRY(launch_char(b, g, d_geom, st));
         if (g.raw_cols) HIP_TRY(launch_raw(b, g, d_geom, st));
     }
     uint64_t cnt[2] = {0, 0};

@@ -898,8 +898,7 @@ static bool detect_specialised(int kd) {
 
 bool walk_in_detect_supported(const Geom& g) {
     const int max_ri = g.kd >= 22 ? 8 : 7;
-    return detect_specialised(g.kd) && g.rint >= 1 && g.rint <= max_ri && g.max_iterations >= 1 &&
-           !g.characterize && !g.cpu_processed;
+    return detect_specialised(g.kd) && g.rint >= 1 && g.rint <= max_ri && g.max_iterations >= 1;
 }
 
 hipError_t launch_detect(const Batch& b, const Geom& g, const Geom* d_geom, hipStream_t s) {

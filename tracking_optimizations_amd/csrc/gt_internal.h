@@ -38,11 +38,8 @@ enum InType : int { IN_U16 = 0, IN_F32 = 1, IN_U8 = 2 };
 // Record planes stored per candidate slot.
 enum RecPlane : int {
     REC_MASS = 0, REC_Y = 1, REC_X = 2,
-    REC_RG = 3, REC_ECC = 4, REC_SIGNAL = 5,                 // cpu_processed
-    REC_RG_GPU = 6, REC_RAW_GPU = 7, REC_SIG_GPU = 8, REC_ECC_GPU = 9,  // characterize
-    REC_NPLANES = 10,
     // start value P[u0, v0] of each candidate, stored only when the walk
-    // runs in detect (characterisation off, so this plane is free)
+    // runs in detect
     REC_CENTER = 3
 };
 
@@ -91,7 +88,7 @@ struct Geom {
     int32_t raw_ns, raw_nb;  // signal and background tap counts
     int32_t raw_reach;       // no tap is further off than this along an axis
     int8_t raw_tap[4 * RAW_MAX_TAPS];  // (dy, dx) of the signal taps, then the background taps
-    float sin2_gpu[1024], cos2_gpu[1024];                // disk radius rint
+    float r2_gpu[1024], sin2_gpu[1024], cos2_gpu[1024];  // disk radius rint
     float r2_cpu[1024], sin_cpu[1024], cos_cpu[1024];    // circle radius band
 };
 
@@ -124,7 +121,7 @@ struct Batch {
     uint64_t* frame_row_base;  // [nframes]
     // candidate slots and records
     uint16_t* slots;       // [tiles * TILE_PX]
-    float* rec;            // [REC_NPLANES * slot_cap]
+    float* rec;            // record planes of slot_cap values each
     uint8_t* keep;         // [slot_cap]
     uint64_t slot_cap;
     // output
@@ -176,6 +173,9 @@ hipError_t launch_emit(const Batch& b, const Geom& g, const Geom* d_geom,
                        hipStream_t s);
 hipError_t launch_fill_u64(uint64_t* p, uint64_t n, uint64_t v, hipStream_t s);
 hipError_t launch_copy(void* dst, const void* src, uint64_t bytes, hipStream_t s);
+
+// Characterisation columns of every output row (gt_char.hip).
+hipError_t launch_char(const Batch& b, const Geom& g, const Geom* d_geom, hipStream_t s);
 
 // Raw signal and background of every output row (gt_raw.hip).
 hipError_t launch_raw(const Batch& b, const Geom& g, const Geom* d_geom, hipStream_t s);

@@ -10,10 +10,11 @@
 //             is_max) -> per-tile candidate slots; percentile value list
 //   select2   percentile: exact order statistics -> threshold
 //   refine    K3: walk + disk mass/centroid (centers.wgsl, walk_cols.wgsl
-//             walk), minmass, characterisation
+//             walk), minmass; where detect has not walked
 //   dedup     K4: separation suppression (execute_gpu.rs:258-284)
 //   fscan     per-frame row offsets
-//   emit      K5: rows in column_names order
+//   emit      K5: rows in column_names order; then the characterisation and
+//             raw signal columns (gt_char.hip, gt_raw.hip)
 //
 // Arithmetic contract (identical to the CPU oracle): every `acc += a*b` of a
 // WGSL shader is one fused multiply-add, every other operation one binary32
@@ -339,103 +340,6 @@ __device__ __forceinline__ void disk_any(const float* P, int H, int W, int band,
     else disk_eval(P, H, W, band, rint, u, v, m, c0, c1);
 }
 
-// Characterisation columns of one row, at the candidate (start) pixel:
-// execute_gpu.rs:165-172,286-299,346-352 (cpu_processed: Rg, ecc, signal
-// with the walked mass) and centers.wgsl:64-80 (characterize: Rg_gpu,
-// raw_mass_gpu, signal_gpu, ecc_gpu with the candidate pixel's own disk).
-__device__ __forceinline__ void characterise(const Batch& b, const Geom* __restrict__ g,
-                                          const float* __restrict__ P, const void* in, int H,
-                                          int W, int u0, int v0, float mass, size_t s) {
-    const uint64_t cap = b.slot_cap;
-    const int band = g->band, rint = g->rint;
-        if (g->cpu_processed) {
-            // execute_gpu.rs:165-172,286-299,346-352 at the candidate pixel:
-            // products with the host tables, each summed in ndarray's
-            // eight-accumulator order (full chunks of 8, pairwise fold, then
-            // the remainder in order).
-            const int r = g->band;
-            const int nt = g->ntap_cpu;
-            const int nfull = nt - (nt % 8);
-            float pr[8], ps[8], pc[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) { pr[q] = 0.f; ps[q] = 0.f; pc[q] = 0.f; }
-            float sig = 0.f, mid = 0.f;
-            int tap = 0;
-            for (int di = -r; di <= r; ++di) {
-                for (int dj = -r; dj <= r; ++dj) {
-                    if (di * di + dj * dj > r * r) continue;
-                    const float d = P[(size_t)(u0 + di) * W + (v0 + dj)];
-                    sig = (tap == 0 || d > sig) ? d : sig;
-                    if (di == 0 && dj == 0) mid = d;
-                    if (tap < nfull) {
-                        const int q = tap & 7;
-                        pr[q] = pr[q] + d * g->r2_cpu[tap];
-                        ps[q] = ps[q] + d * g->sin_cpu[tap];
-                        pc[q] = pc[q] + d * g->cos_cpu[tap];
-                    }
-                    ++tap;
-                }
-            }
-            float rg = 0.f, ss = 0.f, cc = 0.f;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                rg = rg + (pr[q] + pr[q + 4]);
-                ss = ss + (ps[q] + ps[q + 4]);
-                cc = cc + (pc[q] + pc[q + 4]);
-            }
-            tap = 0;
-            for (int di = -r; di <= r; ++di) {
-                for (int dj = -r; dj <= r; ++dj) {
-                    if (di * di + dj * dj > r * r) continue;
-                    if (tap >= nfull) {
-                        const float d = P[(size_t)(u0 + di) * W + (v0 + dj)];
-                        rg = rg + d * g->r2_cpu[tap];
-                        ss = ss + d * g->sin_cpu[tap];
-                        cc = cc + d * g->cos_cpu[tap];
-                    }
-                    ++tap;
-                }
-            }
-            ss = ss * ss;
-            cc = cc * cc;
-            const float ecc = sqrtf(ss + cc);
-            b.rec[REC_RG * cap + s] = sqrtf(rg / mass);
-            b.rec[REC_ECC * cap + s] = ecc / (mass - mid);
-            b.rec[REC_SIGNAL * cap + s] = sig;
-        }
-        if (g->characterize) {
-            // centers.wgsl:64-80 at the candidate pixel
-            float o4[4] = {0.f, 0.f, 0.f, 0.f};
-            if (!(u0 - band < 0 || u0 + band >= H || v0 - band < 0 || v0 + band >= W)) {
-                float ms = 0.f, rg = 0.f, rawm = 0.f, sg = 0.f, es = 0.f, ec = 0.f;
-                int tap = 0;
-                for (int di = -rint; di <= rint; ++di)
-                    for (int dj = -rint; dj <= rint; ++dj) {
-                        if (di * di + dj * dj > rint * rint) continue;
-                        const size_t idx = (size_t)(u0 + di) * W + (v0 + dj);
-                        const float d = P[idx];
-                        ms = ms + d;
-                        rg = __builtin_fmaf(d, (float)(di * di + dj * dj), rg);
-                        rawm = rawm + raw_px(in, b.in_type, idx);
-                        sg = (d > sg) ? d : sg;
-                        es = __builtin_fmaf(d, g->sin2_gpu[tap], es);
-                        ec = __builtin_fmaf(d, g->cos2_gpu[tap], ec);
-                        ++tap;
-                    }
-                es = es * es;
-                ec = ec * ec;
-                o4[3] = sqrtf(es + ec) / (ms - P[(size_t)u0 * W + v0]);
-                o4[0] = sqrtf(rg / ms);
-                o4[1] = rawm;
-                o4[2] = sg;
-            }
-            b.rec[REC_RG_GPU * cap + s] = o4[0];
-            b.rec[REC_RAW_GPU * cap + s] = o4[1];
-            b.rec[REC_SIG_GPU * cap + s] = o4[2];
-            b.rec[REC_ECC_GPU * cap + s] = o4[3];
-        }
-}
-
 // Candidates of RT_TILES consecutive tiles are packed over the 256 lanes of a
 // workgroup (a tile holds ~16 candidates on average; one wave per tile would
 // leave three quarters of the lanes idle while issuing the same number of
@@ -444,7 +348,6 @@ constexpr int RT_TILES = 16;
 
 struct RefTile {
     const float* P;
-    const void* in;
     int x0, y0, H, W;
     uint32_t f, cnt, pref;
 };
@@ -465,7 +368,6 @@ __global__ __launch_bounds__(256) void k_refine(Batch b, const Geom* __restrict_
             const Frame fr = b.frames[f];
             const uint32_t local = item - fr.tile_base;
             rt.P = fr.P;
-            rt.in = fr.in;
             rt.x0 = (int)(local % fr.tx) * TILE_W;
             rt.y0 = (int)(local / fr.tx) * TILE_H;
             rt.H = (int)fr.H;
@@ -532,8 +434,6 @@ __global__ __launch_bounds__(256) void k_refine(Batch b, const Geom* __restrict_
         rec[REC_MASS * cap + slot0 + i] = valid ? mass : 0.f;
         rec[REC_Y * cap + slot0 + i] = y;
         rec[REC_X * cap + slot0 + i] = x;
-        if (valid && (g->cpu_processed || g->characterize))
-            characterise(b, g, P, rt.in, H, W, u0, v0, mass, slot0 + i);
     }
 }
 
@@ -565,7 +465,6 @@ __global__ __launch_bounds__(256) void k_refine_staged(Batch b, const Geom* __re
             const Frame fr = b.frames[f];
             const uint32_t local = item - fr.tile_base;
             rt.P = fr.P;
-            rt.in = fr.in;
             rt.x0 = (int)(local % fr.tx) * TILE_W;
             rt.y0 = (int)(local / fr.tx) * TILE_H;
             rt.H = (int)fr.H;
@@ -700,8 +599,6 @@ __global__ __launch_bounds__(256) void k_refine_staged(Batch b, const Geom* __re
             b.rec[REC_MASS * cap + slot] = valid ? m : 0.f;
             b.rec[REC_Y * cap + slot] = started ? y : 0.f;
             b.rec[REC_X * cap + slot] = started ? x : 0.f;
-            if (valid && (g->cpu_processed || g->characterize))
-                characterise(b, g, rt.P, rt.in, H, W, u0, v0, m, slot);
         }
     }
 }
@@ -1229,10 +1126,9 @@ hipError_t launch_frame_scan(const Batch& b, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------
-// K5 emit: rows [frame, mass, y, x, (Rg, ecc, signal), (raw_mass, raw_bg_median,
-// raw_mass_corrected: left for k_raw), (Rg_gpu, raw_mass_gpu, signal_gpu,
-// ecc_gpu)] in frame order, raster order of the candidate pixel
-// within a frame (row positions from k_tile_scan).
+// K5 emit: rows [frame, mass, y, x, ...] in frame order, raster order of the
+// candidate pixel within a frame (row positions from k_tile_scan).  The columns
+// after x (characterisation, raw signal) are left for k_char and k_raw.
 // ---------------------------------------------------------------------------
 // EMIT_TPW tiles per wave, EMIT_LPT lanes each: a tile holds about a dozen
 // candidates, and a wave's time is mostly its chain of dependent loads, so
@@ -1281,19 +1177,6 @@ __global__ __launch_bounds__(256) void k_emit(Batch b, const Geom* __restrict__ 
                 o[1] = rm;
                 o[2] = ryv;
                 o[3] = rxv;
-                int c = 4;
-                if (g->cpu_processed) {
-                    o[c++] = b.rec[REC_RG * cap + s];
-                    o[c++] = b.rec[REC_ECC * cap + s];
-                    o[c++] = b.rec[REC_SIGNAL * cap + s];
-                }
-                c += g->raw_cols;   // raw signal columns, written by k_raw
-                if (g->characterize) {
-                    o[c++] = b.rec[REC_RG_GPU * cap + s];
-                    o[c++] = b.rec[REC_RAW_GPU * cap + s];
-                    o[c++] = b.rec[REC_SIG_GPU * cap + s];
-                    o[c++] = b.rec[REC_ECC_GPU * cap + s];
-                }
                 b.rows_cand[r] = (int64_t)(ty * TILE_H + (int)(l / TILE_W)) * W +
                                  (tx * TILE_W + (int)(l % TILE_W));
             }

@@ -64,9 +64,11 @@ __device__ __forceinline__ void sliding_max(const int32_t (&x)[N + K - 1], int32
 // order) walks in lane k % 256 of the workgroup, so a typical tile (a few
 // dozen candidates) occupies part of one wave.  Disks inside the staged area
 // are summed from LDS with the taps in the shader's order, others from P.
-template <int RI, int LR, int LC, int LS>
+// L: the staged area, LR rows and LC columns of it valid, LS floats a row.
+template <int RI>
 __device__ __forceinline__ void walk_tile(const Batch& b, const DetParams& dp,
-                                          const float* __restrict__ L,
+                                          const float* __restrict__ L, const int LR, const int LC,
+                                          const int LS,
                                           const GLOBAL uint16_t* __restrict__ slots,
                                           uint32_t total, uint32_t item,
                                           const GLOBAL float* __restrict__ P, int H, int W,
@@ -104,7 +106,7 @@ __device__ __forceinline__ void walk_tile(const Batch& b, const DetParams& dp,
                             if (dj != 0) s1 = __builtin_fmaf(d, (float)dj, s1);
                             ms = ms + d;
                         }
-                } else {
+                } else if constexpr (RI <= 7) {
 #pragma unroll
                     for (int di = -RI; di <= RI; ++di) {
                         const GLOBAL float* row = P + (size_t)(u + di) * W + v;
@@ -114,6 +116,20 @@ __device__ __forceinline__ void walk_tile(const Batch& b, const DetParams& dp,
                             const float d = row[dj];
                             if (di != 0) s0 = __builtin_fmaf(d, (float)di, s0);
                             if (dj != 0) s1 = __builtin_fmaf(d, (float)dj, s1);
+                            ms = ms + d;
+                        }
+                    }
+                } else {   // a rare path: not worth the code of 700 taps
+                    int hw = 0;   // half width of the disk's row
+                    for (int di = -RI; di <= RI; ++di) {
+                        while ((hw + 1) * (hw + 1) + di * di <= RI * RI) ++hw;
+                        while (hw * hw + di * di > RI * RI) --hw;
+                        const GLOBAL float* row = P + (size_t)(u + di) * W + v;
+#pragma unroll 4
+                        for (int dj = -hw; dj <= hw; ++dj) {
+                            const float d = row[dj];
+                            s0 = __builtin_fmaf(d, (float)di, s0);
+                            s1 = __builtin_fmaf(d, (float)dj, s1);
                             ms = ms + d;
                         }
                     }
@@ -369,7 +385,101 @@ __global__ __launch_bounds__(256) void k_detect(Batch b, DetParams dp) {
         const uint32_t total = s_total;
         if (total == 0) return;  // workgroup-uniform
         __syncthreads();         // slots visible
-        walk_tile<RI, LR, LS, LS>(b, dp, L, slots, total, item, P, H, W, x0, y0, A, tid);
+        walk_tile<RI>(b, dp, L, LR, LS, LS, slots, total, item, P, H, W, x0, y0, A, tid);
+    }
+}
+
+// The candidate test of a row-first detect kernel: lane c holds output column c
+// (lanes TILE_W .. 63 none), wave kw output rows kw * 16 .. + 15, `center` and
+// `cm` their values and window maxima.  Writes the tile's slots in raster
+// order, its percentile list and its counts; returns with the tile's candidate
+// count in s_total, the slots not yet visible to the other waves.
+__device__ __forceinline__ void row_candidates(const Batch& b, const DetParams& dp,
+                                               const int32_t (&center)[16], const int32_t (&cm)[16],
+                                               uint32_t item, uint32_t f, int H, int W, int x0,
+                                               int y0, int tid, uint32_t* s_rowcnt,
+                                               uint32_t& s_lcnt, uint32_t& s_total) {
+    constexpr int N = 16;
+    const int c = tid & 63;
+    const int kw = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int v = x0 + c;
+    // candidates: the ballots of the wave's 16 rows stay in scalar registers
+    // (bitwise tests: no short-circuit branches)
+    // (lane masks combined in scalar registers: one vector compare each)
+    const uint64_t colmask = __builtin_amdgcn_ballot_w64((c < TILE_W) & (v < W) &
+                                                         (v - dp.band >= 0) & (v + dp.band < W));
+    const bool diw = dp.diw != 0;
+    // rows m of the wave's run that can hold a candidate: band <= u0 + m <= H - 1 - band
+    const int u0 = y0 + kw * N;
+    const int rlo = max(dp.band - u0, 0), rhi = min(H - 1 - dp.band - u0, N - 1);
+    const uint32_t rowbits = rhi >= rlo ? ((2u << rhi) - (1u << rlo)) : 0u;
+    uint64_t bal[N];
+    uint32_t mycnt = 0;
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        const uint64_t ge = __builtin_amdgcn_ballot_w64(center[m] >= cm[m]);
+        const uint64_t nz = diw ? __builtin_amdgcn_ballot_w64(center[m] != 0) : ~0ull;
+        bal[m] = (rowbits >> m) & 1u ? (colmask & ge & nz) : 0ull;
+        mycnt = (c == m) ? (uint32_t)__popcll(bal[m]) : mycnt;
+    }
+    if (c < N) s_rowcnt[kw * N + c] = mycnt;
+
+    if (dp.has_pct) {
+        // values in the two histogram bins holding the order statistics go to
+        // the tile's list (any order); out-of-frame centres are -inf and
+        // fall outside every range
+        // The two order statistics have adjacent ranks, so no value lies
+        // strictly between their bins: one range from the start of the lower
+        // bin to the end of the upper one holds exactly the two bins.
+        uint32_t lb, lw, hb, hw;
+        pct_bin_range(b.selstate[f * 4 + 0], lb, lw);
+        pct_bin_range(b.selstate[f * 4 + 2], hb, hw);
+        const uint32_t base = lw ? lb : hb;
+        const uint32_t width = c < TILE_W ? (hw ? (hb + hw - base) : lw) : 0u;
+        uint32_t mbits = 0;
+#pragma unroll
+        for (int m = N - 1; m >= 0; --m) {
+            const uint32_t bits = (uint32_t)center[m];
+            mbits = 2u * mbits + ((bits - base < width) ? 1u : 0u);
+        }
+        if (__ballot(mbits != 0u)) {  // wave-uniform
+            const uint32_t n = (uint32_t)__popc(mbits);
+            const uint32_t inc = wave_incl_scan(n, c);
+            const uint32_t tot = __shfl(inc, 63, 64);
+            uint32_t base = 0;
+            if (c == 0) base = atomicAdd(&s_lcnt, tot);
+            base = __builtin_amdgcn_readfirstlane(base);
+            uint32_t j = base + inc - n;
+            GLOBAL uint32_t* list = (GLOBAL uint32_t*)b.list + (size_t)item * TILE_PX;
+#pragma unroll
+            for (int m = 0; m < N; ++m) {
+                if (mbits & (1u << m)) list[j++] = (uint32_t)center[m];
+            }
+        }
+    }
+    __syncthreads();
+    if (tid < 64) {
+        const uint32_t cnt = s_rowcnt[tid];
+        const uint32_t inc = wave_incl_scan(cnt, tid);
+        s_rowcnt[tid] = inc - cnt;
+        if (tid == 63) {
+            b.tile_count[item] = inc;
+            s_total = inc;
+            if (dp.has_pct) b.tile_lcount[item] = s_lcnt;
+        }
+    }
+    __syncthreads();
+    GLOBAL uint16_t* slots = (GLOBAL uint16_t*)b.slots + (size_t)item * TILE_PX;
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        if (bal[m] == 0) continue;  // wave-uniform: most 64-pixel row pieces hold no candidate
+        const int r = kw * N + m;
+        if ((bal[m] >> c) & 1ull) {
+            const uint32_t rank =
+                s_rowcnt[r] + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal[m] >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)bal[m], 0u));
+            slots[rank] = (uint16_t)(r * TILE_W + c);
+        }
     }
 }
 
@@ -533,7 +643,6 @@ __global__ __launch_bounds__(256) void k_detect_rows(Batch b, DetParams dp) {
     __syncthreads();
 
     // column pass + candidate test: lane = column, wave = 16-row run
-    const int v = x0 + c;
     int32_t cm[N];
     {
         int32_t x[NIN];
@@ -542,97 +651,179 @@ __global__ __launch_bounds__(256) void k_detect_rows(Batch b, DetParams dp) {
         sliding_max<N, KD>(x, cm);
     }
 
-    // candidates: the ballots of the wave's 16 rows stay in scalar registers
-    // (bitwise tests: no short-circuit branches)
-    // (lane masks combined in scalar registers: one vector compare each)
-    const uint64_t colmask = __builtin_amdgcn_ballot_w64((c < TILE_W) & (v < W) &
-                                                         (v - dp.band >= 0) & (v + dp.band < W));
-    const bool diw = dp.diw != 0;
-    // rows m of the wave's run that can hold a candidate: band <= u0 + m <= H - 1 - band
-    const int u0 = y0 + kw * N;
-    const int rlo = max(dp.band - u0, 0), rhi = min(H - 1 - dp.band - u0, N - 1);
-    const uint32_t rowbits = rhi >= rlo ? ((2u << rhi) - (1u << rlo)) : 0u;
-    uint64_t bal[N];
-    uint32_t mycnt = 0;
-#pragma unroll
-    for (int m = 0; m < N; ++m) {
-        const uint64_t ge = __builtin_amdgcn_ballot_w64(center[m] >= cm[m]);
-        const uint64_t nz = diw ? __builtin_amdgcn_ballot_w64(center[m] != 0) : ~0ull;
-        bal[m] = (rowbits >> m) & 1u ? (colmask & ge & nz) : 0ull;
-        mycnt = (c == m) ? (uint32_t)__popcll(bal[m]) : mycnt;
-    }
-    if (c < N) s_rowcnt[kw * N + c] = mycnt;
-
-    if (dp.has_pct) {
-        // values in the two histogram bins holding the order statistics go to
-        // the tile's list (any order); out-of-frame centres are -inf and
-        // fall outside every range
-        // The two order statistics have adjacent ranks, so no value lies
-        // strictly between their bins: one range from the start of the lower
-        // bin to the end of the upper one holds exactly the two bins.
-        uint32_t lb, lw, hb, hw;
-        pct_bin_range(b.selstate[f * 4 + 0], lb, lw);
-        pct_bin_range(b.selstate[f * 4 + 2], hb, hw);
-        const uint32_t base = lw ? lb : hb;
-        const uint32_t width = c < TILE_W ? (hw ? (hb + hw - base) : lw) : 0u;
-        uint32_t mbits = 0;
-#pragma unroll
-        for (int m = N - 1; m >= 0; --m) {
-            const uint32_t bits = (uint32_t)center[m];
-            mbits = 2u * mbits + ((bits - base < width) ? 1u : 0u);
-        }
-        if (__ballot(mbits != 0u)) {  // wave-uniform
-            const uint32_t n = (uint32_t)__popc(mbits);
-            const uint32_t inc = wave_incl_scan(n, c);
-            const uint32_t tot = __shfl(inc, 63, 64);
-            uint32_t base = 0;
-            if (c == 0) base = atomicAdd(&s_lcnt, tot);
-            base = __builtin_amdgcn_readfirstlane(base);
-            uint32_t j = base + inc - n;
-            GLOBAL uint32_t* list = (GLOBAL uint32_t*)b.list + (size_t)item * TILE_PX;
-#pragma unroll
-            for (int m = 0; m < N; ++m) {
-                if (mbits & (1u << m)) list[j++] = (uint32_t)center[m];
-            }
-        }
-    }
-    __syncthreads();
-    if (tid < 64) {
-        const uint32_t cnt = s_rowcnt[tid];
-        const uint32_t inc = wave_incl_scan(cnt, tid);
-        s_rowcnt[tid] = inc - cnt;
-        if (tid == 63) {
-            b.tile_count[item] = inc;
-            s_total = inc;
-            if (dp.has_pct) b.tile_lcount[item] = s_lcnt;
-        }
-    }
-    __syncthreads();
-    GLOBAL uint16_t* slots = (GLOBAL uint16_t*)b.slots + (size_t)item * TILE_PX;
-#pragma unroll
-    for (int m = 0; m < N; ++m) {
-        if (bal[m] == 0) continue;  // wave-uniform: most 64-pixel row pieces hold no candidate
-        const int r = kw * N + m;
-        if ((bal[m] >> c) & 1ull) {
-            const uint32_t rank =
-                s_rowcnt[r] + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal[m] >> 32),
-                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)bal[m], 0u));
-            slots[rank] = (uint16_t)(r * TILE_W + c);
-        }
-    }
+    row_candidates(b, dp, center, cm, item, f, H, W, x0, y0, tid, s_rowcnt, s_lcnt, s_total);
 
     if constexpr (RI > 0) {
+        const GLOBAL uint16_t* slots = (const GLOBAL uint16_t*)b.slots + (size_t)item * TILE_PX;
         const uint32_t total = s_total;
         if (total == 0) return;  // workgroup-uniform
         __syncthreads();         // column pass done with L; slots visible
         stage_tile(false);       // columns 0..63 again hold P
         __syncthreads();
-        walk_tile<RI, LR, LC, LS>(b, dp, L, slots, total, item, P, H, W, x0, y0, a, tid);
+        walk_tile<RI>(b, dp, L, LR, LC, LS, slots, total, item, P, H, W, x0, y0, a, tid);
     }
 }
 
-// Generic detect for window sizes without a specialisation: straightforward
-// window loops over the staged tile.
+// Floats of a staged row of k_detect_wide, and bytes of its tile: the last run
+// of a row reads up to 16 columns past the tile.
+__host__ __device__ constexpr int wide_stride(int kd) { return (TILE_W + kd - 1 + 3) / 4 * 4 + 4; }
+constexpr size_t wide_lds(int kd) {
+    return sizeof(float) * ((size_t)(TILE_H + kd - 1) * wide_stride(kd) + 64);
+}
+
+// Detect for windows without a kernel of their own: any KD from P2 to
+// 2 P2 - 1 (P2 = 16 or 32), and walks over disks of radius up to 15.  As
+// k_detect_rows, but a window of KD is the union of two windows of P2 that
+// start KD - P2 apart, so the maxima over P2 have compile-time indices and
+// only the second one's place is a runtime offset: the row pass leaves
+// max(L[r][c .. c + P2 - 1]) over the staged tile, the column pass joins the
+// two places of a row and of a column.
+//
+// Bound by latency (the walk of a tile's few candidates, one lane each); LDS
+// (32 KB at KD = 31, 59 KB at 63) allows five to two workgroups per CU.  24
+// frames of 1024^2 at diameter 21 (KD = 31): DETECT_WIDE_US us, where the
+// straightforward window loops took 353 us and the walk in its own kernel,
+// one lane per candidate with a serial loop over 317 taps in global memory,
+// 452 us.
+template <int P2, int RI>
+__global__ __launch_bounds__(256) void k_detect_wide(Batch b, DetParams dp) {
+    constexpr int N = 16, NIN = N + P2 - 1, NV4 = (NIN + 3) / 4;
+    constexpr int MAXRUNS = (TILE_W + P2 - 1 + N - 1) / N;            // 16-column runs of a row
+    constexpr int NRUN = ((TILE_H + 2 * P2 - 2) * MAXRUNS + 255) / 256;   // of a thread
+    extern __shared__ __attribute__((aligned(16))) float L[];
+    // candidates per tile row, then (in place) the row's first slot
+    __shared__ uint32_t s_rowcnt[TILE_H];
+    __shared__ uint32_t s_lcnt, s_total;
+
+    const int tid = threadIdx.x;
+    const int a = dp.a, KD = dp.kd, off = KD - P2;
+    const int LR = TILE_H + KD - 1, LC = TILE_W + KD - 1, LS = wide_stride(KD);
+    const int runs = (TILE_W + off + N - 1) / N;
+    const uint32_t item = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t f = b.tile_frame[item];
+    const Frame fr = b.frames[f];
+    const uint32_t local = item - fr.tile_base;
+    const int H = (int)fr.H, W = (int)fr.W;
+    const int x0 = (int)(local % fr.tx) * TILE_W;
+    const int y0 = (int)(local / fr.tx) * TILE_H;
+    const GLOBAL float* P = (const GLOBAL float*)fr.P;
+    const GLOBAL char* Pb = (const GLOBAL char*)P;
+    if (tid == 0) s_lcnt = 0;
+
+    // Staging: wave w fills rows w, w + 4, ...; lane = column, then column
+    // 64 + lane.  Indices are clamped into the frame so every load is in
+    // bounds; out-of-frame cells become -inf.  Eight rows are loaded before
+    // the first is stored.
+    auto stage_tile = [&]() {
+        const int lane = tid & 63;
+        const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int v1 = x0 - a + lane, v2 = v1 + 64;
+        const uint32_t o1 = 4u * (uint32_t)min(max(v1, 0), W - 1);
+        const uint32_t o2 = 4u * (uint32_t)min(max(v2, 0), W - 1);
+        const bool c1 = lane < LC && v1 >= 0 && v1 < W, c2 = v2 >= 0 && v2 < W;
+        const bool h1 = lane < LC, h2 = lane + 64 < LC;
+        for (int r0 = wv; r0 < LR; r0 += 32) {
+            float f1[8], f2[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int u = y0 - a + r0 + 4 * q;
+                const uint32_t rb = 4u * (uint32_t)(min(max(u, 0), H - 1) * W);
+                f1[q] = *(const GLOBAL float*)(Pb + (rb + o1));
+                f2[q] = *(const GLOBAL float*)(Pb + (rb + o2));
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int r = r0 + 4 * q;
+                const int u = y0 - a + r;
+                const bool ur = u >= 0 && u < H;  // wave-uniform
+                if (r < LR) {
+                    if (h1) L[r * LS + lane] = (ur && c1) ? f1[q] : __uint_as_float(NEG_INF_BITS);
+                    if (h2) L[r * LS + 64 + lane] = (ur && c2) ? f2[q] : __uint_as_float(NEG_INF_BITS);
+                }
+            }
+        }
+    };
+    stage_tile();
+    __syncthreads();
+
+    // the max filter works on the bit patterns (see sliding_max)
+    const int32_t* Li = (const int32_t*)L;
+    const int c = tid & 63;
+    const int cc = min(c, TILE_W - 1);   // lanes past the tile hold no output
+    const int kw = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int32_t center[N];
+#pragma unroll
+    for (int m = 0; m < N; ++m) center[m] = Li[(kw * N + m + a) * LS + (cc + a)];
+
+    // row pass: max(L[r][c .. c + P2 - 1]) for c < TILE_W + off, over L; the
+    // last run of a row reads (but never uses) cells past it
+    int32_t y[NRUN][N];
+#pragma unroll
+    for (int k2 = 0; k2 < NRUN; ++k2) {
+        const int run = tid + k2 * 256;
+        if (run < LR * runs) {
+            const int r = run / runs, c0 = (run % runs) * N;
+            int32_t x[NIN];
+            const int32_t* src = Li + r * LS + c0;
+#pragma unroll
+            for (int m = 0; m < NV4; ++m) {
+                const int4 q = *(const int4*)(src + 4 * m);
+                if (4 * m + 0 < NIN) x[4 * m + 0] = q.x;
+                if (4 * m + 1 < NIN) x[4 * m + 1] = q.y;
+                if (4 * m + 2 < NIN) x[4 * m + 2] = q.z;
+                if (4 * m + 3 < NIN) x[4 * m + 3] = q.w;
+            }
+            sliding_max<N, P2>(x, y[k2]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k2 = 0; k2 < NRUN; ++k2) {
+        const int run = tid + k2 * 256;
+        if (run < LR * runs) {
+            const int r = run / runs, c0 = (run % runs) * N;
+            int32_t* dst = (int32_t*)L + r * LS + c0;
+#pragma unroll
+            for (int m = 0; m < N / 4; ++m)
+                *(int4*)(dst + 4 * m) =
+                    make_int4(y[k2][4 * m], y[k2][4 * m + 1], y[k2][4 * m + 2], y[k2][4 * m + 3]);
+        }
+    }
+    __syncthreads();
+
+    // column pass: the row window joins two places, the column window too
+    int32_t cm[N];
+    {
+        auto window = [&](int r0, int32_t (&w)[N]) {
+            int32_t x[NIN];
+#pragma unroll
+            for (int m = 0; m < NIN; ++m) {
+                const int32_t* p = Li + (r0 + m) * LS + cc;
+                x[m] = max(p[0], p[off]);
+            }
+            sliding_max<N, P2>(x, w);
+        };
+        int32_t w2[N];
+        window(kw * N, cm);
+        window(kw * N + off, w2);
+#pragma unroll
+        for (int m = 0; m < N; ++m) cm[m] = max(cm[m], w2[m]);
+    }
+    row_candidates(b, dp, center, cm, item, f, H, W, x0, y0, tid, s_rowcnt, s_lcnt, s_total);
+
+    if constexpr (RI > 0) {
+        const GLOBAL uint16_t* slots = (const GLOBAL uint16_t*)b.slots + (size_t)item * TILE_PX;
+        const uint32_t total = s_total;
+        if (total == 0) return;  // workgroup-uniform
+        __syncthreads();         // column pass done with L; slots visible
+        stage_tile();            // P again
+        __syncthreads();
+        walk_tile<RI>(b, dp, L, LR, LC, LS, slots, total, item, P, H, W, x0, y0, a, tid);
+    }
+}
+
+// Generic detect for the smallest windows (KD 1 and 2): straightforward window
+// loops over the staged tile.
 __global__ __launch_bounds__(256) void k_detect_generic(Batch b, DetParams dp) {
     extern __shared__ float dyn[];
     __shared__ uint64_t s_mask[TILE_H];
@@ -834,17 +1025,16 @@ __global__ __launch_bounds__(256) void k_detect_plane(Batch b, DetParams dp) {
     }
 }
 
-static bool detect_specialised(int kd);
-
 static size_t detect_generic_lds(int kd) {
     const int kd1 = max(kd, 1);
     return sizeof(float) * ((size_t)(TILE_H + kd1 - 1) * (TILE_W + kd1 - 1) +
                             (size_t)(TILE_H + kd1 - 1) * TILE_W);
 }
 
-bool detect_needs_plane(const Geom& g) {
-    return !detect_specialised(g.kd) && detect_generic_lds(g.kd) > 60 * 1024;
-}
+// Windows of k_detect_wide: its staged tile stays below 64 KB of LDS.
+constexpr int WIDE_MIN = 16, WIDE_MAX = 63;
+
+bool detect_needs_plane(const Geom& g) { return g.kd > WIDE_MAX; }
 
 template <int KD>
 static hipError_t launch_det_t(const Batch& b, const DetParams& dp, hipStream_t s) {
@@ -896,9 +1086,28 @@ static bool detect_specialised(int kd) {
     }
 }
 
+// Largest disk radius that a window's own kernel walks.
+static int specialised_radius(int kd) { return kd >= 22 ? 8 : 7; }
+
 bool walk_in_detect_supported(const Geom& g) {
-    const int max_ri = g.kd >= 22 ? 8 : 7;
-    return detect_specialised(g.kd) && g.rint >= 1 && g.rint <= max_ri && g.max_iterations >= 1;
+    if (g.rint < 1 || g.max_iterations < 1) return false;
+    if (detect_specialised(g.kd) && g.rint <= specialised_radius(g.kd)) return true;
+    return g.kd >= WIDE_MIN && g.kd <= WIDE_MAX && g.rint <= 15;
+}
+
+template <int P2>
+static hipError_t launch_det_wide_t(const Batch& b, const DetParams& dp, hipStream_t s) {
+    const dim3 grid(b.tiles), block(256);
+    const size_t lds = wide_lds(dp.kd);
+#define GT_WIDE(RI) \
+    case RI: hipLaunchKernelGGL((k_detect_wide<P2, RI>), grid, block, lds, s, b, dp); break;
+    switch (dp.walk_ri) {
+        GT_WIDE(0) GT_WIDE(1) GT_WIDE(2) GT_WIDE(3) GT_WIDE(4) GT_WIDE(5) GT_WIDE(6) GT_WIDE(7)
+        GT_WIDE(8) GT_WIDE(9) GT_WIDE(10) GT_WIDE(11) GT_WIDE(12) GT_WIDE(13) GT_WIDE(14) GT_WIDE(15)
+        default: return hipErrorInvalidValue;
+    }
+#undef GT_WIDE
+    return hipGetLastError();
 }
 
 hipError_t launch_detect(const Batch& b, const Geom& g, const Geom* d_geom, hipStream_t s) {
@@ -913,6 +1122,13 @@ hipError_t launch_detect(const Batch& b, const Geom& g, const Geom* d_geom, hipS
     dp.maxit = g.max_iterations;
     dp.minmass = g.minmass;
     dp.slot_cap = b.slot_cap;
+    // windows of 28 to 63 have no kernel of their own; from 16 on, a disk that
+    // the window's kernel does not walk goes the same way
+    const bool own = detect_specialised(g.kd) && dp.walk_ri <= specialised_radius(g.kd);
+    if (!own && g.kd >= WIDE_MIN && g.kd <= WIDE_MAX) {
+        // (the kernel's windows start where the others' do)
+        return g.kd < 32 ? launch_det_wide_t<16>(b, dp, s) : launch_det_wide_t<32>(b, dp, s);
+    }
     switch (g.kd) {
         case 4: return launch_det_t<4>(b, dp, s);
         case 5: return launch_det_t<5>(b, dp, s);

@@ -602,6 +602,17 @@ FrameSizes sizes_of(uint32_t h, uint32_t w, int seg) {
     return s;
 }
 
+// Whether the walk of a call over `tiles` detect tiles runs in its own kernel
+// although detect could do it.  A tile of a window of 18 or more holds at most
+// half a dozen candidates, and a wave of detect walks them alone: gathered
+// from 16 tiles they take 64 against 117 us of detect (the whole 121 -> 112 us
+// for 96 frames of 517 x 663 at KD = 19; 144 -> 106 us at KD = 25, 264 -> 155
+// us at KD = 31, 24 frames of 1024^2; 89 -> 111 us the other way at KD = 15).
+// While every tile is resident (about four workgroups on each of 256 CUs) the
+// walks run beside each other and the extra launch costs more (one frame of
+// 512^2 at KD = 31: 54 against 65 us).
+bool walk_apart(const Geom& g, uint64_t tiles) { return g.kd >= 18 && tiles > 1024; }
+
 int rec_planes(const Geom& g) {
     if (g.walk_in_detect && g.has_pct) return REC_CENTER + 1;
     return REC_X + 1;
@@ -829,7 +840,10 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
 
     Geom g;
     GT_TRY(make_geom(p, integer_input, g));
-    g.walk_in_detect = ctx->fuse_walk && walk_in_detect_supported(g) ? 1 : 0;
+    uint64_t call_tiles = 0;
+    for (const auto& f : frames) call_tiles += sizes_of(f.h, f.w, 1).tiles;
+    g.walk_in_detect = ctx->fuse_walk && walk_in_detect_supported(g) &&
+                       !walk_apart(g, call_tiles) ? 1 : 0;
     // autotuned launch shape for calls whose frames all share one shape
     int seg = ctx->seg_rows;
     if (!ctx->seg_set) {
@@ -1854,7 +1868,7 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
     const bool integer_input = in_type != IN_F32;
     Geom g;
     GT_TRY(make_geom(p, integer_input, g));
-    g.walk_in_detect = ctx->fuse_walk && walk_in_detect_supported(g) ? 1 : 0;
+    g.walk_in_detect = ctx->fuse_walk && walk_in_own_detect(g) ? 1 : 0;
     const size_t es = elem_size(in_type);
     const bool generic = !bandpass_fast_path(in_type, w, g);
     // Which frames fit the scratch is part of this entry point's contract, so

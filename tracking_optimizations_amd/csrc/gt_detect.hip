@@ -679,12 +679,9 @@ constexpr size_t wide_lds(int kd) {
 // max(L[r][c .. c + P2 - 1]) over the staged tile, the column pass joins the
 // two places of a row and of a column.
 //
-// Bound by latency (the walk of a tile's few candidates, one lane each); LDS
-// (32 KB at KD = 31, 59 KB at 63) allows five to two workgroups per CU.  24
-// frames of 1024^2 at diameter 21 (KD = 31): DETECT_WIDE_US us, where the
-// straightforward window loops took 353 us and the walk in its own kernel,
-// one lane per candidate with a serial loop over 317 taps in global memory,
-// 452 us.
+// Bound by latency and LDS (32 KB at KD = 31, 59 KB at 63: five to two
+// workgroups per CU).  24 frames of 1024^2 at diameter 21 (KD = 31): 80 us
+// without the walk, where the straightforward window loops took 353 us.
 template <int P2, int RI>
 __global__ __launch_bounds__(256) void k_detect_wide(Batch b, DetParams dp) {
     constexpr int N = 16, NIN = N + P2 - 1, NV4 = (NIN + 3) / 4;
@@ -1089,10 +1086,14 @@ static bool detect_specialised(int kd) {
 // Largest disk radius that a window's own kernel walks.
 static int specialised_radius(int kd) { return kd >= 22 ? 8 : 7; }
 
+bool walk_in_own_detect(const Geom& g) {
+    return g.rint >= 1 && g.max_iterations >= 1 && detect_specialised(g.kd) &&
+           g.rint <= specialised_radius(g.kd);
+}
+
 bool walk_in_detect_supported(const Geom& g) {
     if (g.rint < 1 || g.max_iterations < 1) return false;
-    if (detect_specialised(g.kd) && g.rint <= specialised_radius(g.kd)) return true;
-    return g.kd >= WIDE_MIN && g.kd <= WIDE_MAX && g.rint <= 15;
+    return walk_in_own_detect(g) || (g.kd >= WIDE_MIN && g.kd <= WIDE_MAX && g.rint <= 15);
 }
 
 template <int P2>

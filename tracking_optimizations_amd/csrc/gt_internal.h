@@ -152,7 +152,10 @@ hipError_t launch_bandpass(const Batch& b, const Geom& g, const Geom* d_geom,
 hipError_t launch_bandpass_generic(const Batch& b, const Geom* d_geom, uint32_t max_px,
                                    int hist, hipStream_t s);
 hipError_t launch_select1(const Batch& b, const Geom& g, hipStream_t s);
+// The walk can run inside detect; and in the kernel of the window's own (not
+// the one that wide windows share).
 bool walk_in_detect_supported(const Geom& g);
+bool walk_in_own_detect(const Geom& g);
 // Dilation windows too wide for a staged tile: detect writes the row maxima
 // to each frame's tmp plane (Frame::tmp, H*W floats at least) first.
 bool detect_needs_plane(const Geom& g);

@@ -308,38 +308,6 @@ __device__ __forceinline__ void disk_eval(const float* __restrict__ P, int H, in
     c1 = s1 / ms;
 }
 
-template <int RI>
-__device__ __forceinline__ void disk_eval_t(const float* __restrict__ P, int H, int W, int band,
-                                            int u, int v, float& m, float& c0, float& c1) {
-    if (u - band < 0 || u + band >= H || v - band < 0 || v + band >= W) {
-        m = 0.f; c0 = 0.f; c1 = 0.f;
-        return;
-    }
-    float s0 = 0.f, s1 = 0.f, ms = 0.f;
-#pragma unroll
-    for (int i = -RI; i <= RI; ++i) {
-        const float* row = P + (size_t)(u + i) * W + v;
-#pragma unroll
-        for (int j = -RI; j <= RI; ++j) {
-            if (i * i + j * j > RI * RI) continue;
-            const float d = row[j];
-            s0 = __builtin_fmaf(d, (float)i, s0);
-            s1 = __builtin_fmaf(d, (float)j, s1);
-            ms = ms + d;
-        }
-    }
-    m = ms;
-    c0 = s0 / ms;
-    c1 = s1 / ms;
-}
-
-template <int RI>
-__device__ __forceinline__ void disk_any(const float* P, int H, int W, int band, int rint, int u,
-                                         int v, float& m, float& c0, float& c1) {
-    if constexpr (RI > 0) disk_eval_t<RI>(P, H, W, band, u, v, m, c0, c1);
-    else disk_eval(P, H, W, band, rint, u, v, m, c0, c1);
-}
-
 // Candidates of RT_TILES consecutive tiles are packed over the 256 lanes of a
 // workgroup (a tile holds ~16 candidates on average; one wave per tile would
 // leave three quarters of the lanes idle while issuing the same number of
@@ -352,37 +320,43 @@ struct RefTile {
     uint32_t f, cnt, pref;
 };
 
-template <int RI>
+// Lanes of the first wave fill the workgroup's tiles and their first candidates.
+__device__ __forceinline__ void load_ref_tiles(const Batch& b, uint32_t item0, int nt, int tid,
+                                               RefTile* s_t, uint32_t& s_total) {
+    if (tid >= 64) return;
+    uint32_t cnt = 0;
+    RefTile rt;
+    if (tid < nt) {
+        const uint32_t item = item0 + tid;
+        const uint32_t f = b.tile_frame[item];
+        const Frame fr = b.frames[f];
+        const uint32_t local = item - fr.tile_base;
+        rt.P = fr.P;
+        rt.x0 = (int)(local % fr.tx) * TILE_W;
+        rt.y0 = (int)(local / fr.tx) * TILE_H;
+        rt.H = (int)fr.H;
+        rt.W = (int)fr.W;
+        rt.f = f;
+        cnt = b.tile_count[item];
+        rt.cnt = cnt;
+    }
+    const uint32_t inc = wave_incl_scan(cnt, tid);
+    if (tid < nt) {
+        rt.pref = inc - cnt;
+        s_t[tid] = rt;
+    }
+    if (tid == 63) s_total = inc;
+}
+
+// Refinement of what k_walk does not take: no iterations, disks of radius 0 or
+// above 15.
 __global__ __launch_bounds__(256) void k_refine(Batch b, const Geom* __restrict__ g) {
     __shared__ RefTile s_t[RT_TILES];
     __shared__ uint32_t s_total;
     const uint32_t item0 = blockIdx.x * RT_TILES;
     const int nt = (int)min<uint32_t>(RT_TILES, b.tiles - item0);
     const int tid = threadIdx.x;
-    if (tid < 64) {
-        uint32_t cnt = 0;
-        RefTile rt;
-        if (tid < nt) {
-            const uint32_t item = item0 + tid;
-            const uint32_t f = b.tile_frame[item];
-            const Frame fr = b.frames[f];
-            const uint32_t local = item - fr.tile_base;
-            rt.P = fr.P;
-            rt.x0 = (int)(local % fr.tx) * TILE_W;
-            rt.y0 = (int)(local / fr.tx) * TILE_H;
-            rt.H = (int)fr.H;
-            rt.W = (int)fr.W;
-            rt.f = f;
-            cnt = b.tile_count[item];
-            rt.cnt = cnt;
-        }
-        const uint32_t inc = wave_incl_scan(cnt, tid);
-        if (tid < nt) {
-            rt.pref = inc - cnt;
-            s_t[tid] = rt;
-        }
-        if (tid == 63) s_total = inc;
-    }
+    load_ref_tiles(b, item0, nt, tid, s_t, s_total);
     __syncthreads();
     const uint32_t total = s_total;
     const int band = g->band, rint = g->rint;
@@ -415,10 +389,10 @@ __global__ __launch_bounds__(256) void k_refine(Batch b, const Geom* __restrict_
             float c0 = 0.f, c1 = 0.f, m = 0.f;
             if (maxit == 0) {
                 float t0, t1;
-                disk_any<RI>(P, H, W, band, rint, 0, 0, m, t0, t1);
+                disk_eval(P, H, W, band, rint, 0, 0, m, t0, t1);
             }
             for (uint32_t it = 0; it < maxit; ++it) {
-                disk_any<RI>(P, H, W, band, rint, u, v, m, c0, c1);
+                disk_eval(P, H, W, band, rint, u, v, m, c0, c1);
                 bool changed = false;
                 if (c0 > sthr && u < H - 1) { u += 1; changed = true; }
                 else if (c0 < -sthr && u > 0) { u -= 1; changed = true; }
@@ -437,49 +411,60 @@ __global__ __launch_bounds__(256) void k_refine(Batch b, const Geom* __restrict_
     }
 }
 
-// Refinement with LDS-staged disk boxes (1 <= RI <= 7, max_iterations >= 1).
-// Lanes hold candidates (16 consecutive tiles per workgroup).  Every walk
-// step needs the disk around the lane's current pixel; instead of each lane
-// issuing (2RI+1)^2 scattered 4-byte loads, the wave stages the
-// (2RI+1)x(2RI+1) boxes of up to 16 lanes at a time with row-coalesced loads
-// (two load instructions per box for RI = 5), then each owner lane sums its
-// disk from LDS in the shader's tap order.
+// Refinement with disks of radius 1 to 15 (max_iterations >= 1).  The
+// candidates of RT_TILES tiles are dealt out over the four waves of a
+// workgroup, lane = candidate, so that a wave's issue slots serve the few
+// candidates of several tiles; a disk row is loaded four pixels at a time (a
+// load costs the address units one line per lane).  Bound by the latency of
+// the disk rows: 24 frames of 1024^2 at diameter 21 (2.5 candidates a tile,
+// 317 taps) in 75 us, against 177 us inside detect on the tile staged again
+// and 452 us with a serial loop over scalar loads.
+typedef float f4v_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
 template <int RI>
-__global__ __launch_bounds__(256) void k_refine_staged(Batch b, const Geom* __restrict__ g) {
-    constexpr int BW = 2 * RI + 1;
-    constexpr int BOX = BW * BW;
-    constexpr int G = 16;
-    constexpr int NE = (BOX + 63) / 64;
+__device__ __forceinline__ void disk_sums(const GLOBAL float* c, int W, float& s0, float& s1,
+                                          float& ms) {
+    s0 = s1 = ms = 0.f;
+#pragma unroll
+    for (int di = -RI; di <= RI; ++di) {
+        int hw = 0;
+        while ((hw + 1) * (hw + 1) + di * di <= RI * RI) ++hw;   // a constant once unrolled
+        const GLOBAL float* row = c + (ptrdiff_t)di * W;
+        float d[2 * RI + 1];
+        // whole chunks from the left, the last one ending at the disk's edge
+        const int n = 2 * hw + 1;
+        if (n < 4) {
+#pragma unroll
+            for (int k = 0; k < n; ++k) d[k] = row[k - hw];
+        } else {
+#pragma unroll
+            for (int k = 0; k < n; k += 4) {
+                const int at = k + 4 <= n ? k : n - 4;
+                const f4v_a4 q = *(const GLOBAL f4v_a4*)(row + at - hw);
+                d[at] = q.x;
+                d[at + 1] = q.y;
+                d[at + 2] = q.z;
+                d[at + 3] = q.w;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < n; ++k) {
+            // a zero coefficient leaves its sum unchanged (see walk_tile)
+            if (di != 0) s0 = __builtin_fmaf(d[k], (float)di, s0);
+            if (k != hw) s1 = __builtin_fmaf(d[k], (float)(k - hw), s1);
+            ms = ms + d[k];
+        }
+    }
+}
+
+template <int RI>
+__global__ __launch_bounds__(256) void k_walk(Batch b, const Geom* __restrict__ g) {
     __shared__ RefTile s_t[RT_TILES];
     __shared__ uint32_t s_total;
-    __shared__ float s_box[4][G][BOX];
     const uint32_t item0 = blockIdx.x * RT_TILES;
     const int nt = (int)min<uint32_t>(RT_TILES, b.tiles - item0);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid < 64) {
-        uint32_t cnt = 0;
-        RefTile rt;
-        if (tid < nt) {
-            const uint32_t item = item0 + tid;
-            const uint32_t f = b.tile_frame[item];
-            const Frame fr = b.frames[f];
-            const uint32_t local = item - fr.tile_base;
-            rt.P = fr.P;
-            rt.x0 = (int)(local % fr.tx) * TILE_W;
-            rt.y0 = (int)(local / fr.tx) * TILE_H;
-            rt.H = (int)fr.H;
-            rt.W = (int)fr.W;
-            rt.f = f;
-            cnt = b.tile_count[item];
-            rt.cnt = cnt;
-        }
-        const uint32_t inc = wave_incl_scan(cnt, tid);
-        if (tid < nt) {
-            rt.pref = inc - cnt;
-            s_t[tid] = rt;
-        }
-        if (tid == 63) s_total = inc;
-    }
+    const int tid = threadIdx.x;
+    load_ref_tiles(b, item0, nt, tid, s_t, s_total);
     __syncthreads();
     const uint32_t total = s_total;
     const int band = g->band;
@@ -488,137 +473,61 @@ __global__ __launch_bounds__(256) void k_refine_staged(Batch b, const Geom* __re
     const int has_pct = g->has_pct;
     const float sthr = 0.6f;
     const uint64_t cap = b.slot_cap;
-
-    for (uint32_t gb = 0; gb < total; gb += 256) {
-        const uint32_t gi = gb + tid;
-        const bool has = gi < total;
+    // candidate gi goes to wave gi % 4
+    for (uint32_t gi = (uint32_t)(tid >> 6) + 4u * (uint32_t)(tid & 63); gi < total; gi += 256) {
         int j = 0;
 #pragma unroll
         for (int q = 1; q < RT_TILES; ++q)
             if (q < nt && s_t[q].pref <= gi) j = q;
         const RefTile& rt = s_t[j];
-        const uint32_t i = has ? gi - rt.pref : 0;
-        const size_t slot = (size_t)(item0 + (uint32_t)j) * TILE_PX + i;
+        const size_t slot = (size_t)(item0 + (uint32_t)j) * TILE_PX + (gi - rt.pref);
         const int H = rt.H, W = rt.W;
-        int u0 = 0, v0 = 0;
-        bool active = false;
-        if (has) {
-            const uint32_t l = b.slots[slot];
-            u0 = rt.y0 + (int)(l / TILE_W);
-            v0 = rt.x0 + (int)(l % TILE_W);
-            active = true;
-            if (has_pct) active = (double)rt.P[(size_t)u0 * W + v0] > b.thr[rt.f];
-        }
-        const bool started = active;
-        int u = u0, v = v0;
-        float c0 = 0.f, c1 = 0.f, m = 0.f;
-        uint32_t it = 0;
-        while (__ballot(active)) {
-            uint64_t pend = __ballot(active);
-            while (pend) {
-                int src[G];
-                uint64_t gm = 0;
-#pragma unroll
-                for (int q = 0; q < G; ++q) {
-                    src[q] = pend ? __ffsll((long long)pend) - 1 : -1;
-                    if (pend) {
-                        gm |= 1ull << src[q];
-                        pend &= pend - 1;
-                    }
+        const GLOBAL float* P = (const GLOBAL float*)rt.P;
+        const uint32_t l = b.slots[slot];
+        int u = rt.y0 + (int)(l / TILE_W), v = rt.x0 + (int)(l % TILE_W);
+        float y = 0.f, x = 0.f, m = 0.f;
+        if (!has_pct || (double)P[(size_t)u * W + v] > b.thr[rt.f]) {
+            float c0 = 0.f, c1 = 0.f;
+            for (uint32_t it = 0; it < maxit; ++it) {
+                if (u - band < 0 || u + band >= H || v - band < 0 || v + band >= W) {
+                    m = 0.f; c0 = 0.f; c1 = 0.f;
+                } else {
+                    float s0, s1;
+                    disk_sums<RI>(P + (size_t)u * W + v, W, s0, s1, m);
+                    c0 = s0 / m;
+                    c1 = s1 / m;
                 }
-                float fb[G][NE];
-#pragma unroll
-                for (int q = 0; q < G; ++q) {
-                    if (src[q] >= 0) {
-                        const int uq = __shfl(u, src[q], 64), vq = __shfl(v, src[q], 64);
-                        const int jq = __shfl(j, src[q], 64);
-                        const RefTile& tq = s_t[jq];
-                        if (uq - band >= 0 && uq + band < tq.H && vq - band >= 0 && vq + band < tq.W) {
-                            const GLOBAL float* Pq = (const GLOBAL float*)tq.P;
-#pragma unroll
-                            for (int e = 0; e < NE; ++e) {
-                                const int el = lane + 64 * e;
-                                if (el < BOX) {
-                                    const int r = el / BW, c = el - r * BW;
-                                    fb[q][e] = Pq[(size_t)(uq - RI + r) * tq.W + (vq - RI + c)];
-                                }
-                            }
-                        }
-                    }
-                }
-#pragma unroll
-                for (int q = 0; q < G; ++q) {
-                    if (src[q] >= 0) {
-#pragma unroll
-                        for (int e = 0; e < NE; ++e) {
-                            const int el = lane + 64 * e;
-                            if (el < BOX) s_box[wave][q][el] = fb[q][e];
-                        }
-                    }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                if ((gm >> lane) & 1ull) {
-                    const int sl = (int)__popcll(gm & lanemask_lt(lane));
-                    if (u - band < 0 || u + band >= H || v - band < 0 || v + band >= W) {
-                        m = 0.f; c0 = 0.f; c1 = 0.f;
-                    } else {
-                        const float* box = s_box[wave][sl];
-                        float s0 = 0.f, s1 = 0.f, ms = 0.f;
-#pragma unroll
-                        for (int di = -RI; di <= RI; ++di)
-#pragma unroll
-                            for (int dj = -RI; dj <= RI; ++dj) {
-                                if (di * di + dj * dj > RI * RI) continue;
-                                const float d = box[(di + RI) * BW + (dj + RI)];
-                                s0 = __builtin_fmaf(d, (float)di, s0);
-                                s1 = __builtin_fmaf(d, (float)dj, s1);
-                                ms = ms + d;
-                            }
-                        m = ms;
-                        c0 = s0 / ms;
-                        c1 = s1 / ms;
-                    }
-                    bool changed = false;
-                    if (c0 > sthr && u < H - 1) { u += 1; changed = true; }
-                    else if (c0 < -sthr && u > 0) { u -= 1; changed = true; }
-                    if (c1 > sthr && v < W - 1) { v += 1; changed = true; }
-                    else if (c1 < -sthr && v > 0) { v -= 1; changed = true; }
-                    ++it;
-                    if (!changed || it >= maxit) active = false;
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                bool changed = false;
+                if (c0 > sthr && u < H - 1) { u += 1; changed = true; }
+                else if (c0 < -sthr && u > 0) { u -= 1; changed = true; }
+                if (c1 > sthr && v < W - 1) { v += 1; changed = true; }
+                else if (c1 < -sthr && v > 0) { v -= 1; changed = true; }
+                if (!changed) break;
             }
+            y = (float)u + c0;
+            x = (float)v + c1;
+            m = (m > minmass) && (m != 0.f) ? m : 0.f;
         }
-        if (has) {
-            const float y = (float)u + c0, x = (float)v + c1;
-            const bool valid = started && (m > minmass) && (m != 0.f);
-            b.rec[REC_MASS * cap + slot] = valid ? m : 0.f;
-            b.rec[REC_Y * cap + slot] = started ? y : 0.f;
-            b.rec[REC_X * cap + slot] = started ? x : 0.f;
-        }
+        b.rec[REC_MASS * cap + slot] = m;
+        b.rec[REC_Y * cap + slot] = y;
+        b.rec[REC_X * cap + slot] = x;
     }
 }
 
 hipError_t launch_refine(const Batch& b, const Geom& g, const Geom* d_geom, hipStream_t s) {
     if (g.walk_in_detect) return hipSuccess;  // done by detect
-    const dim3 grid((b.tiles + RT_TILES - 1) / RT_TILES);
+    const dim3 grid((b.tiles + RT_TILES - 1) / RT_TILES), block(256);
     if (g.max_iterations >= 1) {
+#define GT_WALK(RI) \
+    case RI: hipLaunchKernelGGL(k_walk<RI>, grid, block, 0, s, b, d_geom); return hipGetLastError();
         switch (g.rint) {
-            case 1: hipLaunchKernelGGL(k_refine_staged<1>, grid, dim3(256), 0, s, b, d_geom); return hipGetLastError();
-            case 2: hipLaunchKernelGGL(k_refine_staged<2>, grid, dim3(256), 0, s, b, d_geom); return hipGetLastError();
-            case 3: hipLaunchKernelGGL(k_refine_staged<3>, grid, dim3(256), 0, s, b, d_geom); return hipGetLastError();
-            case 4: hipLaunchKernelGGL(k_refine_staged<4>, grid, dim3(256), 0, s, b, d_geom); return hipGetLastError();
-            case 5: hipLaunchKernelGGL(k_refine_staged<5>, grid, dim3(256), 0, s, b, d_geom); return hipGetLastError();
-            case 6: hipLaunchKernelGGL(k_refine_staged<6>, grid, dim3(256), 0, s, b, d_geom); return hipGetLastError();
-            case 7: hipLaunchKernelGGL(k_refine_staged<7>, grid, dim3(256), 0, s, b, d_geom); return hipGetLastError();
+            GT_WALK(1) GT_WALK(2) GT_WALK(3) GT_WALK(4) GT_WALK(5) GT_WALK(6) GT_WALK(7) GT_WALK(8)
+            GT_WALK(9) GT_WALK(10) GT_WALK(11) GT_WALK(12) GT_WALK(13) GT_WALK(14) GT_WALK(15)
             default: break;
         }
+#undef GT_WALK
     }
-    hipLaunchKernelGGL(k_refine<0>, grid, dim3(256), 0, s, b, d_geom);
+    hipLaunchKernelGGL(k_refine, grid, block, 0, s, b, d_geom);
     return hipGetLastError();
 }
 

@@ -549,6 +549,11 @@ size_t elem_size(int in_type) { return in_type == IN_U16 ? 2 : (in_type == IN_U8
 
 size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// Frame counters of up to n frames in a batch.
+size_t count_bytes(uint64_t n) {
+    return al256(std::max(std::min<uint64_t>(n, COUNT_LINES) * COUNT_LINE, n) * 8);
+}
+
 struct BatchPlan {
     size_t b0, b1;
 };
@@ -945,9 +950,10 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     const int nstreams = (plain || plan.size() < 2 || ctx->profiling) ? 1 : kStreams;
     const uint64_t slot_cap = maxneed.tiles * TILE_PX;
     const size_t nfb = maxneed.nframes;
-    // per-frame: hist (4096 u32), frame_rows, frame_cands, spare, selstate(4), thr(double), row_base(u64)
+    // per-frame: hist (4096 u32), frame_rows, counts, selstate(4), thr(double), row_base(u64)
     const size_t pf_hist = al256(nfb * HIST_BINS * 4);
     const size_t pf_small = al256(nfb * 4);
+    const size_t pf_count = count_bytes(nfb);
     const size_t pf_sel = al256(nfb * 16);
     const size_t pf_8 = al256(nfb * 8);
     HIP_TRY(ctx->geom.ensure(sizeof(Geom)));
@@ -961,7 +967,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         HIP_TRY(w.keep.ensure(slot_cap));
         if (!on_device) HIP_TRY(w.in_stage.ensure(maxneed.in_bytes));
         HIP_TRY(w.tile3.ensure(al256(maxneed.tiles * 4) * 4 + 2 * al256(maxneed.tiles * 4 * TILE_H)));
-        HIP_TRY(w.perframe.ensure(pf_hist + 3 * pf_small + pf_sel + 2 * pf_8));
+        HIP_TRY(w.perframe.ensure(pf_hist + pf_small + pf_count + pf_sel + 2 * pf_8));
     }
     HIP_TRY(ctx->counters.ensure(256));
 
@@ -976,7 +982,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     // ---- frame tables -------------------------------------------------------
     // The host builds the frame table and, per batch, the small base arrays
     // (first bandpass item, first tile and first dedup block of every frame:
-    // 3 x (nb + 1) entries); k_fill_tables expands them on the device into the
+    // 3 x (nb + 1) entries); k_begin expands them on the device into the
     // per-item tables (frame of every bandpass item and tile, top-left tile of
     // every dedup block), so a call uploads kilobytes, not megabytes.
     std::vector<Frame> ftab(frames.size());
@@ -1063,7 +1069,9 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
                 ao.jac = adj->jac.as<float>();
             }
         }
-        uint64_t* counters = ctx->counters.as<uint64_t>();  // [0] cand_total, [1] row_carry
+        // running (rows, candidates), two pairs that the batches alternate between
+        uint64_t* counters = ctx->counters.as<uint64_t>();
+        const uint64_t* totals = counters + 2 * (plan.size() % 2);   // after the last batch
         res->data.clear();
         res->cand.clear();
         launches = 0;
@@ -1071,8 +1079,6 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         hipStream_t s0 = ctx->streams[0];
         uint64_t host_rows_done = 0;
         auto enqueue = [&]() -> gt_status {
-        HIP_TRY(launch_fill_u64(counters, 2, 0, s0));
-        ++launches;
         if (nstreams > 1) {
             HIP_TRY(hipEventRecord(ctx->ev_join, s0));
             HIP_TRY(hipStreamWaitEvent(ctx->streams[1], ctx->ev_join, 0));
@@ -1101,7 +1107,6 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             const size_t t3s = al256(maxneed.tiles * 4);
             b.tile_count = (uint32_t*)t3;
             b.tile_keep = (uint32_t*)(t3 + t3s);
-            b.tile_row_off = (uint32_t*)(t3 + 2 * t3s);
             b.tile_lcount = (uint32_t*)(t3 + 3 * t3s);
             b.rowk = (uint32_t*)(t3 + 4 * t3s);
             b.rowoff = (uint32_t*)(t3 + 4 * t3s + al256(maxneed.tiles * 4 * TILE_H));
@@ -1110,8 +1115,8 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             pf += pf_hist;
             b.list = g.has_pct ? w.list.as<uint32_t>() : nullptr;
             b.frame_rows = (uint32_t*)pf; pf += pf_small;
-            b.frame_cands = (uint32_t*)pf; pf += pf_small;
-            pf += pf_small;
+            b.counts = (uint64_t*)pf; pf += pf_count;
+            b.count_stride = count_stride_of(nb);
             b.selstate = (int32_t*)pf; pf += pf_sel;
             b.thr = (double*)pf; pf += pf_8;
             b.frame_row_base = (uint64_t*)pf;
@@ -1119,8 +1124,8 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             b.rec = w.rec.as<float>();
             b.keep = w.keep.as<uint8_t>();
             b.slot_cap = slot_cap;
-            b.cand_total = counters;
-            b.row_carry = counters + 1;
+            b.carry_in = counters + 2 * (bi % 2);
+            b.carry_out = counters + 2 * ((bi + 1) % 2);
             b.rows = ctx->rows.as<float>();
             b.rows_cand = ctx->rows_cand.as<int64_t>();
             b.rows_cap = rows_cap;
@@ -1135,10 +1140,9 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
                 }
             }
             HIP_TRY(stage(ctx, st, GT_STAGE_ZERO, [&] {
-                const hipError_t e = launch_fill_tables(b, dblock_bases, max_frame_work, st);
-                return e != hipSuccess ? e : launch_zero_batch(b, st);
+                return launch_begin(b, dblock_bases, max_frame_work, bi == 0 ? counters : nullptr, st);
             }));
-            launches += 2;
+            ++launches;
             if (generic) {
                 uint32_t maxpx = 0;
                 for (size_t fi = bp.b0; fi < bp.b1; ++fi)
@@ -1167,14 +1171,13 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             uint32_t max_ty = 1;
             for (size_t fi = bp.b0; fi < bp.b1; ++fi)
                 max_ty = std::max(max_ty, ftab[fi].ty);
-            HIP_TRY(stage(ctx, st, GT_STAGE_SCAN, [&] { return launch_tile_scan(b, max_ty, st); }));
             // row bases continue the previous batch's count: order the scans
             if (nstreams > 1 && bi > 0)
                 HIP_TRY(hipStreamWaitEvent(st, ctx->ev_scan[(bi - 1) % nstreams], 0));
-            HIP_TRY(stage(ctx, st, GT_STAGE_SCAN, [&] { return launch_frame_scan(b, st); }));
+            HIP_TRY(stage(ctx, st, GT_STAGE_SCAN, [&] { return launch_scan(b, max_ty, st); }));
             if (nstreams > 1) HIP_TRY(hipEventRecord(ctx->ev_scan[si], st));
             HIP_TRY(stage(ctx, st, GT_STAGE_EMIT, [&] { return launch_emit(b, g, d_geom, st); }));
-            launches += 5;
+            launches += g.walk_in_detect ? 3 : 4;
             if (g.characterize || g.cpu_processed) {
                 HIP_TRY(launch_char(b, g, d_geom, st));
                 ++launches;
@@ -1194,7 +1197,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             } else if (plain) {
                 // per-frame readback, as the reference's get_work does
                 uint64_t carry = 0;
-                HIP_TRY(hipMemcpyAsync(&carry, counters + 1, 8, hipMemcpyDeviceToHost, st));
+                HIP_TRY(hipMemcpyAsync(&carry, b.carry_out, 8, hipMemcpyDeviceToHost, st));
                 HIP_TRY(hipStreamSynchronize(st));
                 const uint64_t upto = std::min(carry, rows_cap);
                 if (upto > host_rows_done) {
@@ -1290,14 +1293,14 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         }
         HIP_TRY(hipEventRecord(ctx->ev1, s0));
         uint64_t cnt[2] = {0, 0};
-        HIP_TRY(hipMemcpyAsync(cnt, counters, 16, hipMemcpyDeviceToHost, s0));
+        HIP_TRY(hipMemcpyAsync(cnt, totals, 16, hipMemcpyDeviceToHost, s0));
         HIP_TRY(hipStreamSynchronize(s0));
         float ms = 0.f;
         HIP_TRY(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
         ctx->last.device_ms = ms;
         collect_stage_times(ctx);
-        ctx->last.candidates = cnt[0];
-        const uint64_t total_rows = cnt[1];
+        ctx->last.candidates = cnt[1];
+        const uint64_t total_rows = cnt[0];
         if (total_rows > rows_cap) {
             rows_cap = total_rows + 1024;
             continue;  // rerun with enough room (results are deterministic)
@@ -1899,7 +1902,7 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
         L.nbases = 3 * (nb + 1) + L.k1 + L.tiles + nb * dblocks_pf;
         const uint64_t slots = L.tiles * TILE_PX;
         L.geom = take(sizeof(Geom));
-        L.counters = take(16);
+        L.counters = take(32);
         L.ftab = take(nb * sizeof(Frame));
         L.bases = take(L.nbases * 4);
         L.P = take(nb * fs.px * 4);
@@ -1909,8 +1912,8 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
         L.rec = take(slots * 4 * rec_counted);
         L.keep = take(slots);
         L.tile3 = take(al256(L.tiles * 4) * 4 + 2 * al256(L.tiles * 4 * TILE_H));
-        L.perframe = take(al256(nb * HIST_BINS * 4) + 3 * al256(nb * 4) + al256(nb * 16) +
-                          2 * al256(nb * 8));
+        L.perframe = take(al256(nb * HIST_BINS * 4) + al256(nb * 4) + count_bytes(nb) +
+                          al256(nb * 16) + 2 * al256(nb * 8));
         L.end = o;
         return L;
     };
@@ -1944,15 +1947,15 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
     uint64_t* counters = (uint64_t*)(base + L.counters);
     hipStream_t st = ctx->streams[0];
     HIP_TRY(hipMemcpyAsync(d_geom, &g, sizeof(Geom), hipMemcpyHostToDevice, st));
-    HIP_TRY(launch_fill_u64(counters, 2, 0, st));
+    uint64_t bi = 0;   // batches
     Frame* ftab = ctx->na_ftab.data();
     uint32_t* bases = ctx->na_bases.data();
-    for (uint64_t b0 = 0; b0 < n; b0 += nbmax) {
+    for (uint64_t b0 = 0; b0 < n; b0 += nbmax, ++bi) {
         const uint32_t nb = (uint32_t)std::min<uint64_t>(nbmax, n - b0);
         if (b0 > 0) HIP_TRY(hipEventSynchronize(ctx->ev_na));   // host tables copied out
         // frame tables: k1 bases [nb + 1], tile bases [nb + 1] and dedup-block
         // bases [nb + 1] from the host; the per-item tables after them are
-        // filled on the device (k_fill_tables)
+        // filled on the device (k_begin)
         uint32_t* k1b = bases;
         uint32_t* tb = bases + nb + 1;
         uint32_t* dbb = tb + nb + 1;
@@ -2002,7 +2005,6 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
         const size_t t3s = al256(L.tiles * 4);
         b.tile_count = (uint32_t*)t3;
         b.tile_keep = (uint32_t*)(t3 + t3s);
-        b.tile_row_off = (uint32_t*)(t3 + 2 * t3s);
         b.tile_lcount = (uint32_t*)(t3 + 3 * t3s);
         b.rowk = (uint32_t*)(t3 + 4 * t3s);
         b.rowoff = (uint32_t*)(t3 + 4 * t3s + al256(L.tiles * 4 * TILE_H));
@@ -2011,8 +2013,8 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
         pf += al256(nbmax * HIST_BINS * 4);
         b.list = g.has_pct ? (uint32_t*)(base + L.list) : nullptr;
         b.frame_rows = (uint32_t*)pf; pf += al256(nbmax * 4);
-        b.frame_cands = (uint32_t*)pf; pf += al256(nbmax * 4);
-        pf += al256(nbmax * 4);
+        b.counts = (uint64_t*)pf; pf += count_bytes(nbmax);
+        b.count_stride = count_stride_of(nb);
         b.selstate = (int32_t*)pf; pf += al256(nbmax * 16);
         b.thr = (double*)pf; pf += al256(nbmax * 8);
         b.frame_row_base = (uint64_t*)pf;
@@ -2020,15 +2022,15 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
         b.rec = (float*)(base + L.rec);
         b.keep = (uint8_t*)(base + L.keep);
         b.slot_cap = L.tiles * TILE_PX;
-        b.cand_total = counters;
-        b.row_carry = counters + 1;
+        b.carry_in = counters + 2 * (bi % 2);
+        b.carry_out = counters + 2 * ((bi + 1) % 2);
         b.rows = d_rows;
         b.rows_cand = d_cand;
         b.rows_cap = rows_cap;
 
-        HIP_TRY(launch_fill_tables(b, d_bases + 2 * ((size_t)nb + 1),
-                                   (uint32_t)(fs.k1_items + fs.tiles + dblocks_pf), st));
-        HIP_TRY(launch_zero_batch(b, st));
+        HIP_TRY(launch_begin(b, d_bases + 2 * ((size_t)nb + 1),
+                             (uint32_t)(fs.k1_items + fs.tiles + dblocks_pf),
+                             bi == 0 ? counters : nullptr, st));
         if (generic)
             HIP_TRY(launch_bandpass_generic(b, d_geom, h * w, g.has_pct, st));
         else
@@ -2038,25 +2040,24 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
         if (g.has_pct) HIP_TRY(launch_select2(b, g, st));
         HIP_TRY(launch_refine(b, g, d_geom, st));
         HIP_TRY(launch_dedup(b, g, d_geom, st));
-        HIP_TRY(launch_tile_scan(b, fs.ty, st));
-        HIP_TRY(launch_frame_scan(b, st));
+        HIP_TRY(launch_scan(b, fs.ty, st));
         HIP_TRY(launch_emit(b, g, d_geom, st));
         if (g.characterize || g.cpu_processed) HIP_TRY(launch_char(b, g, d_geom, st));
         if (g.raw_cols) HIP_TRY(launch_raw(b, g, d_geom, st));
     }
     uint64_t cnt[2] = {0, 0};
-    HIP_TRY(hipMemcpyAsync(cnt, counters, 16, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(cnt, counters + 2 * (bi % 2), 16, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
-    *n_rows = cnt[1];
+    *n_rows = cnt[0];
     ctx->last = gt_timing{};
     ctx->last.frames = n;
     ctx->last.pixels = n * fs.px;
-    ctx->last.candidates = cnt[0];
-    ctx->last.rows = cnt[1];
-    if (cnt[1] > rows_cap)
+    ctx->last.candidates = cnt[1];
+    ctx->last.rows = cnt[0];
+    if (cnt[0] > rows_cap)
         return fail(GT_E_INVALID,
                     "%llu rows found but rows_capacity is %llu; only the first %llu were written",
-                    (unsigned long long)cnt[1], (unsigned long long)rows_cap,
+                    (unsigned long long)cnt[0], (unsigned long long)rows_cap,
                     (unsigned long long)rows_cap);
     return GT_OK;
 }

@@ -29,6 +29,10 @@ constexpr int K1_STRIP = 256;   // output columns per bandpass work item
 // annulus (each at most RAW_MAX_TAPS, offsets within +-127).
 constexpr int RAW_MAX_TAPS = 4096;
 
+// Frames up to which every frame's counters have a cache line of their own.
+constexpr uint32_t COUNT_LINES = 256, COUNT_LINE = 16;
+inline uint32_t count_stride_of(uint64_t nframes) { return nframes <= COUNT_LINES ? COUNT_LINE : 1; }
+
 // Percentile histogram: 4096 bins over the float32 bit pattern
 // (bin 0 = exact zero, bin b >= 1 = bits >> 19 == b - 1).
 constexpr int HIST_BINS = 4096;
@@ -107,7 +111,6 @@ struct Batch {
     // per-tile arrays [tiles]
     uint32_t* tile_count;
     uint32_t* tile_keep;
-    uint32_t* tile_row_off;
     uint32_t* rowk;        // [tiles * 64] kept rows of the tile in pixel rows <= r
     uint32_t* rowoff;      // [tiles * 64] frame-relative first row of pixel row r
     uint32_t* tile_lcount; // percentile list entries of the tile
@@ -117,7 +120,12 @@ struct Batch {
     int32_t* selstate;     // [nframes * 4]: bin_lo, rank_lo, bin_hi, rank_hi
     double* thr;           // [nframes]
     uint32_t* frame_rows;  // [nframes]
-    uint32_t* frame_cands; // [nframes] candidates entering refinement
+    // per frame, count_stride apart: kept rows (low half) and candidates, added
+    // up by dedup.  Few frames have a cache line each: the adds to one line
+    // are served one after the other (a 56-frame batch of 2048^2 with the
+    // counters side by side: dedup 257 instead of 118 us)
+    uint64_t* counts;
+    uint32_t count_stride;
     uint64_t* frame_row_base;  // [nframes]
     // candidate slots and records
     uint16_t* slots;       // [tiles * TILE_PX]
@@ -125,8 +133,10 @@ struct Batch {
     uint8_t* keep;         // [slot_cap]
     uint64_t slot_cap;
     // output
-    uint64_t* cand_total;  // device running candidate count (statistics)
-    uint64_t* row_carry;   // device running row count across batches
+    // running (rows, candidates) before and after this batch, on the device;
+    // consecutive batches alternate between two pairs
+    const uint64_t* carry_in;
+    uint64_t* carry_out;
     float* rows;
     int64_t* rows_cand;
     uint64_t rows_cap;
@@ -142,7 +152,6 @@ struct AdjOut {
 
 // Launchers (gt_kernels.hip, gt_bandpass.hip, gt_detect.hip).  All launch on
 // `s`; return hipSuccess or the first launch error.
-hipError_t launch_zero_batch(const Batch& b, hipStream_t s);
 // The streaming bandpass handles every input type with 1 <= R <= 16 (all that
 // smoothing_size allows but 1) and frames at least min_w >= 2 pixels wide;
 // the rest takes the generic kernels.
@@ -162,19 +171,19 @@ bool detect_needs_plane(const Geom& g);
 hipError_t launch_detect(const Batch& b, const Geom& g, const Geom* d_geom,
                          hipStream_t s);
 hipError_t launch_select2(const Batch& b, const Geom& g, hipStream_t s);
-// Expands the batch's bases (first bandpass item, tile and dedup block of
-// every frame) into b.k1_frame, b.tile_frame and b.dblock_tile.
-hipError_t launch_fill_tables(const Batch& b, const uint32_t* dblock_bases,
-                              uint32_t max_frame_work, hipStream_t s);
+// First launch of a batch: clears its counters and expands its bases (first
+// bandpass item, tile and dedup block of every frame) into b.k1_frame,
+// b.tile_frame and b.dblock_tile.  carry: the two pairs of running totals, to
+// be cleared by the first batch of a call (else null).
+hipError_t launch_begin(const Batch& b, const uint32_t* dblock_bases, uint32_t max_frame_work,
+                        uint64_t* carry, hipStream_t s);
 hipError_t launch_refine(const Batch& b, const Geom& g, const Geom* d_geom,
                          hipStream_t s);
 hipError_t launch_dedup(const Batch& b, const Geom& g, const Geom* d_geom,
                         hipStream_t s);
-hipError_t launch_tile_scan(const Batch& b, uint32_t max_ty, hipStream_t s);
-hipError_t launch_frame_scan(const Batch& b, hipStream_t s);
+hipError_t launch_scan(const Batch& b, uint32_t max_ty, hipStream_t s);
 hipError_t launch_emit(const Batch& b, const Geom& g, const Geom* d_geom,
                        hipStream_t s);
-hipError_t launch_fill_u64(uint64_t* p, uint64_t n, uint64_t v, hipStream_t s);
 hipError_t launch_copy(void* dst, const void* src, uint64_t bytes, hipStream_t s);
 
 // Characterisation columns of every output row (gt_char.hip).

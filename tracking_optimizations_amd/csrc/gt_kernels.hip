@@ -2,7 +2,7 @@
 //
 // Pipeline per batch of frames (every stage is one launch over all frames of
 // the batch; work items are (frame, tile) pairs):
-//   zero      clear per-frame counters and histograms
+//   begin     clear per-frame counters and histograms, expand item tables
 //   bandpass  K1: u16/u8/f32 -> P (float32), optional percentile histogram
 //             (preprocess_rows.wgsl + preprocess_cols.wgsl)
 //   select1   percentile: histogram bin of the two order statistics
@@ -12,7 +12,7 @@
 //   refine    K3: walk + disk mass/centroid (centers.wgsl, walk_cols.wgsl
 //             walk), minmass; where detect has not walked
 //   dedup     K4: separation suppression (execute_gpu.rs:258-284)
-//   fscan     per-frame row offsets
+//   scan      row offsets
 //   emit      K5: rows in column_names order; then the characterisation and
 //             raw signal columns (gt_char.hip, gt_raw.hip)
 //
@@ -33,29 +33,15 @@
 namespace gt {
 
 // ---------------------------------------------------------------------------
-// zero: per-frame counters / histograms of a batch
+// begin: the first launch of a batch.  Clears the per-frame counters and
+// histograms, and expands the batch's bases into the per-item tables: frame
+// blockIdx.y writes the frame index of each of its bandpass items and tiles
+// and the top-left tile of each of its 2x2 dedup blocks (the frame's blocks in
+// raster order).  The first batch of a call also clears the running totals
+// (`carry`, two pairs).
 // ---------------------------------------------------------------------------
-__global__ void k_zero_batch(Batch b, int with_hist) {
-    const uint64_t nh = with_hist ? (uint64_t)b.nframes * HIST_BINS : 0;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nh;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        b.hist1[i] = 0;
-}
-
-hipError_t launch_zero_batch(const Batch& b, hipStream_t s) {
-    const int with_hist = b.hist1 != nullptr;
-    const uint64_t total = with_hist ? (uint64_t)b.nframes * HIST_BINS : 0;
-    uint32_t blocks = (uint32_t)std::min<uint64_t>((total + 255) / 256, 4096);
-    if (blocks == 0) blocks = 1;
-    hipLaunchKernelGGL(k_zero_batch, dim3(blocks), dim3(256), 0, s, b, with_hist);
-    return hipGetLastError();
-}
-
-// Per-item tables of a batch from its per-frame bases: frame blockIdx.y
-// writes the frame index of each of its bandpass items and tiles and the
-// top-left tile of each of its 2x2 dedup blocks (the frame's blocks in
-// raster order).
-__global__ void k_fill_tables(Batch b, const uint32_t* __restrict__ dbases) {
+__global__ __launch_bounds__(256) void k_begin(Batch b, const uint32_t* __restrict__ dbases,
+                                               uint64_t* __restrict__ carry) {
     const uint32_t f = blockIdx.y;
     const uint32_t k1a = b.k1_bases[f], k1n = b.k1_bases[f + 1] - k1a;
     const uint32_t ta = b.tile_bases[f], tn = b.tile_bases[f + 1] - ta;
@@ -65,8 +51,12 @@ __global__ void k_fill_tables(Batch b, const uint32_t* __restrict__ dbases) {
     uint32_t* k1f = (uint32_t*)b.k1_frame;
     uint32_t* tf = (uint32_t*)b.tile_frame;
     uint32_t* dt = (uint32_t*)b.dblock_tile;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < k1n + tn + dn;
-         i += gridDim.x * blockDim.x) {
+    const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+    if (t0 == 0) b.counts[(size_t)f * b.count_stride] = 0;
+    if (carry && f == 0 && t0 < 4) carry[t0] = 0;
+    if (b.hist1)
+        for (uint32_t i = t0; i < (uint32_t)HIST_BINS; i += step) b.hist1[(size_t)f * HIST_BINS + i] = 0;
+    for (uint32_t i = t0; i < k1n + tn + dn; i += step) {
         if (i < k1n) {
             k1f[k1a + i] = f;
         } else if (i < k1n + tn) {
@@ -78,23 +68,11 @@ __global__ void k_fill_tables(Batch b, const uint32_t* __restrict__ dbases) {
     }
 }
 
-hipError_t launch_fill_tables(const Batch& b, const uint32_t* dblock_bases,
-                              uint32_t max_frame_work, hipStream_t s) {
-    const uint32_t bx = std::min<uint32_t>((max_frame_work + 255) / 256, 64);
-    hipLaunchKernelGGL(k_fill_tables, dim3(bx, b.nframes), dim3(256), 0, s, b, dblock_bases);
-    return hipGetLastError();
-}
-
-__global__ void k_fill_u64(uint64_t* p, uint64_t n, uint64_t v) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        p[i] = v;
-}
-
-hipError_t launch_fill_u64(uint64_t* p, uint64_t n, uint64_t v, hipStream_t s) {
-    uint32_t blocks = (uint32_t)std::min<uint64_t>((n + 255) / 256, 1024);
-    if (blocks == 0) blocks = 1;
-    hipLaunchKernelGGL(k_fill_u64, dim3(blocks), dim3(256), 0, s, p, n, v);
+hipError_t launch_begin(const Batch& b, const uint32_t* dblock_bases, uint32_t max_frame_work,
+                        uint64_t* carry, hipStream_t s) {
+    const uint32_t work = std::max(max_frame_work, b.hist1 ? (uint32_t)HIST_BINS : 1u);
+    const uint32_t bx = std::min<uint32_t>((work + 255) / 256, 64);
+    hipLaunchKernelGGL(k_begin, dim3(bx, b.nframes), dim3(256), 0, s, b, dblock_bases, carry);
     return hipGetLastError();
 }
 
@@ -181,8 +159,11 @@ hipError_t launch_select1(const Batch& b, const Geom& g, hipStream_t s) {
 // Exact order statistics lo and hi of one frame by radix selection over the
 // per-tile value lists: level A counts bits [18:8] of the values in each
 // target bin, level B bits [7:0] of the values sharing the chosen level-A
-// digit.  Both targets share every pass; each thread walks whole tile lists
-// with 16-byte loads.
+// digit.  Both targets share every pass.  Bound by the latency of the list
+// reads (16 bytes each): a thread per tile where a frame has about as many
+// tiles as the workgroup threads (1376 tiles: 14 us for 40 frames; 16 threads
+// each: 44 us), up to 16 threads where it has fewer (88 tiles: 9 against 11
+// us).
 __global__ __launch_bounds__(1024) void k_select2(Batch b, float percentile) {
     __shared__ uint32_t s_ha[2][2048];
     __shared__ uint32_t s_res[2][3];
@@ -199,16 +180,17 @@ __global__ __launch_bounds__(1024) void k_select2(Batch b, float percentile) {
     const int rank[2] = {b.selstate[f * 4 + 1], b.selstate[f * 4 + 3]};
     const bool need[2] = {bin[0] != 0, hi != lo && bin[1] != 0};
     const uint32_t ntiles = fr.tx * fr.ty;
+    const uint32_t lpt = ntiles > 512 ? 1u : ntiles > 128 ? 4u : 16u;   // threads per tile
     for (int pass = 0; pass < 2; ++pass) {
         const int nb = pass == 0 ? 2048 : 256;
         for (int i = t; i < 2 * 2048; i += 1024) s_ha[i / 2048][i % 2048] = 0;
         __syncthreads();
         const uint32_t sa0 = pass ? s_res[0][0] : 0u, sa1 = pass ? s_res[1][0] : 0u;
-        for (uint32_t tl = t; tl < ntiles; tl += 1024) {
+        for (uint32_t tl = (uint32_t)t / lpt; tl < ntiles; tl += 1024 / lpt) {
             const uint32_t it = fr.tile_base + tl;
             const uint32_t cnt = b.tile_lcount[it];
             const GLOBAL uint4* lst = (const GLOBAL uint4*)(b.list + (size_t)it * TILE_PX);
-            for (uint32_t i4 = 0; i4 < (cnt + 3) / 4; ++i4) {
+            for (uint32_t i4 = (uint32_t)t % lpt; 4 * i4 < cnt; i4 += lpt) {
                 const uint4 q = lst[i4];
                 const uint32_t vals[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
@@ -627,7 +609,14 @@ void k_dedup(Batch b, const Geom* __restrict__ g) {
         bxmin = fminf(bxmin, __shfl_xor(bxmin, o, 64));
         bxmax = fmaxf(bxmax, __shfl_xor(bxmax, o, 64));
     }
+    // rows (low half) and candidates of the frame; nothing waits for the add
+    auto count = [&](uint32_t kept_n) {
+        if (lane == 0)
+            atomicAdd((unsigned long long*)&b.counts[(size_t)f * b.count_stride],
+                      (unsigned long long)kept_n | ((unsigned long long)own_n << 32));
+    };
     if (!(bymin <= bymax)) {  // no valid own record
+        count(0);
         for (uint32_t j = lane; j < own_n; j += 64) b.keep[own_slot(j, own_q(j))] = 0;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -828,6 +817,7 @@ void k_dedup(Batch b, const Geom* __restrict__ g) {
 #pragma unroll
         for (int qq = 0; qq < 4; ++qq) kept[qq] += (uint32_t)__popcll(__ballot(keep && q == qq));
     }
+    count(kept[0] + kept[1] + kept[2] + kept[3]);
     // kept rows of each tile in pixel rows <= r (the emit order is raster)
     wave_sync();
 #pragma unroll
@@ -845,72 +835,9 @@ hipError_t launch_dedup(const Batch& b, const Geom& g, const Geom* d_geom, hipSt
 }
 
 // ---------------------------------------------------------------------------
-// tile scan: one workgroup per frame turns its tiles' keep counts into row
-// offsets and sums its candidates and rows
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_tile_scan(Batch b) {
-    constexpr int PT = 8;   // tiles per thread in the one-round path
-    __shared__ uint32_t s_part[4];
-    __shared__ uint32_t s_cand[4];
-    const uint32_t f = blockIdx.x;
-    const Frame fr = b.frames[f];
-    const uint32_t ntiles = fr.tx * fr.ty;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    if (ntiles <= 256 * PT) {  // workgroup-uniform
-        // thread t takes tiles t * PT .. t * PT + PT - 1: every load of the
-        // frame in one round, then one workgroup scan of the thread sums
-        const uint32_t k0 = (uint32_t)t * PT;
-        uint32_t kc[PT], cc[PT];
-#pragma unroll
-        for (int i = 0; i < PT; ++i) {
-            const bool in = k0 + i < ntiles;
-            kc[i] = in ? b.tile_keep[fr.tile_base + k0 + i] : 0u;
-            cc[i] = in ? b.tile_count[fr.tile_base + k0 + i] : 0u;
-        }
-        uint32_t sum = 0, cands = 0;
-#pragma unroll
-        for (int i = 0; i < PT; ++i) { sum += kc[i]; cands += cc[i]; }
-        const uint32_t inc = wave_incl_scan(sum, lane);
-        cands = wave_sum_u(cands);
-        if (lane == 63) s_part[wave] = inc;
-        if (lane == 0) s_cand[wave] = cands;
-        __syncthreads();
-        uint32_t before = inc - sum;
-        for (int w = 0; w < wave; ++w) before += s_part[w];
-#pragma unroll
-        for (int i = 0; i < PT; ++i) {
-            if (k0 + i < ntiles) b.tile_row_off[fr.tile_base + k0 + i] = before;
-            before += kc[i];
-        }
-        if (t == 0) {
-            b.frame_rows[f] = s_part[0] + s_part[1] + s_part[2] + s_part[3];
-            b.frame_cands[f] = s_cand[0] + s_cand[1] + s_cand[2] + s_cand[3];
-        }
-        return;
-    }
-    uint32_t carry = 0, cands = 0;
-    for (uint32_t base = 0; base < ntiles; base += 256) {
-        const uint32_t k = base + t;
-        const uint32_t c = k < ntiles ? b.tile_keep[fr.tile_base + k] : 0u;
-        cands += k < ntiles ? b.tile_count[fr.tile_base + k] : 0u;
-        const uint32_t inc = wave_incl_scan(c, lane);
-        if (lane == 63) s_part[wave] = inc;
-        __syncthreads();
-        uint32_t before = carry;
-        for (int w = 0; w < wave; ++w) before += s_part[w];
-        if (k < ntiles) b.tile_row_off[fr.tile_base + k] = before + inc - c;
-        carry += s_part[0] + s_part[1] + s_part[2] + s_part[3];
-        __syncthreads();
-    }
-    cands = wave_sum_u(cands);
-    if (lane == 0) s_cand[wave] = cands;
-    __syncthreads();
-    if (t == 0) {
-        b.frame_rows[f] = carry;
-        b.frame_cands[f] = s_cand[0] + s_cand[1] + s_cand[2] + s_cand[3];
-    }
-}
-
+// scan: row offsets.  One launch of (frame, four tile rows); every wave adds
+// up what precedes its own tile row, so nothing waits for another workgroup.
+//
 // Raster order within a frame (get_work scans masses in raster order,
 // execute_gpu.rs:108-195): a kept row at pixel row r of tile t in tile row tr
 // comes after every kept row of the earlier tile rows, of tiles left of t in
@@ -921,16 +848,49 @@ __global__ __launch_bounds__(256) void k_tile_scan(Batch b) {
 // One wave per tile row, lane = pixel row.  Tile rows of up to 48 tiles
 // (frames up to 2304 columns) load every K once, in one round, and take
 // K[t][r - 1] from the lane below; wider ones load in chunks of 32 tiles.
-__global__ __launch_bounds__(256) void k_row_scan(Batch b) {
+//
+// The first workgroup of a frame also writes the frame's rows (counted by
+// dedup) and their base (the rows of the batches before, `carry_in`, and of the
+// frames before), that of the last frame the running totals (`carry_out`).
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_scan(Batch b) {
     constexpr int CH = 32;
     constexpr int C1 = 48;
+    __shared__ uint64_t s_rows[4], s_cands[4];
     const uint32_t f = blockIdx.x;
     const Frame fr = b.frames[f];
-    const int lane = threadIdx.x & 63;
-    const uint32_t tr = blockIdx.y * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (blockIdx.y == 0) {
+        const bool last = f + 1 == b.nframes;
+        uint64_t rows = 0, cands = 0;
+        for (uint32_t i = threadIdx.x; i < f + (last ? 1u : 0u); i += 256) {
+            const uint64_t n = b.counts[(size_t)i * b.count_stride];
+            rows += i < f ? n & 0xffffffffu : 0u;
+            cands += n >> 32;
+        }
+        for (int d = 32; d > 0; d >>= 1) {
+            rows += __shfl_xor(rows, d, 64);
+            cands += __shfl_xor(cands, d, 64);
+        }
+        if (lane == 0) { s_rows[wave] = rows; s_cands[wave] = cands; }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const uint64_t base = b.carry_in[0] + s_rows[0] + s_rows[1] + s_rows[2] + s_rows[3];
+            const uint32_t own = (uint32_t)b.counts[(size_t)f * b.count_stride];
+            b.frame_row_base[f] = base;
+            b.frame_rows[f] = own;
+            if (last) {
+                b.carry_out[0] = base + own;
+                b.carry_out[1] = b.carry_in[1] + s_cands[0] + s_cands[1] + s_cands[2] + s_cands[3];
+            }
+        }
+    }
+    const uint32_t tr = blockIdx.y * 4 + (uint32_t)wave;
     if (tr >= fr.ty) return;
     const uint32_t t0 = fr.tile_base + tr * fr.tx;
-    const uint32_t base = b.tile_row_off[t0];
+    uint32_t base = 0;   // kept rows of the tile rows above
+    for (uint32_t i = (uint32_t)lane; i < tr * fr.tx; i += 64) base += b.tile_keep[fr.tile_base + i];
+    base = wave_sum_u(base);
     const uint32_t* K = b.rowk + (size_t)t0 * TILE_H + lane;
     if (fr.tx <= C1) {  // wave-uniform
         uint32_t kle[C1], klt[C1];
@@ -983,60 +943,14 @@ __global__ __launch_bounds__(256) void k_row_scan(Batch b) {
     }
 }
 
-hipError_t launch_tile_scan(const Batch& b, uint32_t max_ty, hipStream_t s) {
-    hipLaunchKernelGGL(k_tile_scan, dim3(b.nframes), dim3(256), 0, s, b);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_row_scan, dim3(b.nframes, (max_ty + 3) / 4), dim3(256), 0, s, b);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// fscan: frame row bases (continuing the running count across batches)
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_frame_scan(Batch b) {
-    __shared__ uint64_t s_part[256];
-    __shared__ uint64_t s_cand[256];
-    const int t = threadIdx.x;
-    const uint32_t n = b.nframes;
-    const uint32_t per = (n + 255) / 256;
-    uint64_t sum = 0, cs = 0;
-    for (uint32_t i = 0; i < per; ++i) {
-        const uint32_t k = t * per + i;
-        if (k < n) {
-            sum += b.frame_rows[k];
-            cs += b.frame_cands[k];
-        }
-    }
-    s_part[t] = sum;
-    s_cand[t] = cs;
-    __syncthreads();
-    uint64_t before = *b.row_carry;
-    for (int i = 0; i < t; ++i) before += s_part[i];
-    for (uint32_t i = 0; i < per; ++i) {
-        const uint32_t k = t * per + i;
-        if (k < n) {
-            b.frame_row_base[k] = before;
-            before += b.frame_rows[k];
-        }
-    }
-    __syncthreads();
-    if (t == 255) {
-        *b.row_carry = before;
-        uint64_t c = 0;
-        for (int i = 0; i < 256; ++i) c += s_cand[i];
-        *b.cand_total += c;
-    }
-}
-
-hipError_t launch_frame_scan(const Batch& b, hipStream_t s) {
-    hipLaunchKernelGGL(k_frame_scan, dim3(1), dim3(256), 0, s, b);
+hipError_t launch_scan(const Batch& b, uint32_t max_ty, hipStream_t s) {
+    hipLaunchKernelGGL(k_scan, dim3(b.nframes, (max_ty + 3) / 4), dim3(256), 0, s, b);
     return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
 // K5 emit: rows [frame, mass, y, x, ...] in frame order, raster order of the
-// candidate pixel within a frame (row positions from k_tile_scan).  The columns
+// candidate pixel within a frame (row positions from k_scan).  The columns
 // after x (characterisation, raw signal) are left for k_char and k_raw.
 // ---------------------------------------------------------------------------
 // EMIT_TPW tiles per wave, EMIT_LPT lanes each: a tile holds about a dozen

@@ -8,6 +8,7 @@
 #include <atomic>
 #include <chrono>
 #include <cmath>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -91,6 +92,12 @@ bool injected_failure(int kind) {
     return false;
 }
 
+// Live contexts: the block caches below keep memory only while there is one.
+std::atomic<int> g_contexts{0};
+
+// Returns the device blocks that are kept for later calls; true if there were any.
+bool drop_kept_device_blocks();
+
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
@@ -103,6 +110,10 @@ struct DevBuf {
         n = (n + 255) & ~(size_t)255;
         if (injected_failure(0)) return hipErrorOutOfMemory;
         hipError_t e = hipMalloc(&p, n);
+        if (e == hipErrorOutOfMemory && drop_kept_device_blocks()) {
+            (void)hipGetLastError();
+            e = hipMalloc(&p, n);
+        }
         if (e == hipSuccess) bytes = n;
         else p = nullptr;
         return e;
@@ -114,6 +125,106 @@ struct DevBuf {
     }
     template <class T> T* as() const { return (T*)p; }
 };
+
+// Pinned host memory of a context, grown on demand.
+struct PinBuf {
+    void* p = nullptr;
+    size_t bytes = 0;
+    hipError_t ensure(size_t n) {
+        if (p && n <= bytes) return hipSuccess;
+        release();
+        n = std::max<size_t>((n + 4095) & ~(size_t)4095, 65536);
+        if (injected_failure(0)) return hipErrorOutOfMemory;
+        const hipError_t e = hipHostMalloc(&p, n, hipHostMallocDefault);
+        if (e == hipSuccess) bytes = n;
+        else p = nullptr;
+        return e;
+    }
+    void release() {
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        bytes = 0;
+    }
+    template <class T> T* as() const { return (T*)p; }
+};
+
+// Device blocks that outlive a call (an adjoint's Jacobian patches): freed ones
+// are kept for the next adjoint on the same device, at most 1 GiB in all, and
+// handed back with the last context or when an allocation fails.  Every call
+// that uses a block waits for the device before it returns, so a freed one may
+// go to another stream or thread at once.
+class DeviceBlockCache {
+  public:
+    struct Block {
+        void* p = nullptr;
+        size_t bytes = 0;
+        int device = 0;
+        template <class T> T* as() const { return (T*)p; }
+    };
+    static hipError_t get(int device, size_t n, Block& out) {   // `device` is current
+        n = (std::max<size_t>(n, 256) + 255) & ~(size_t)255;
+        {
+            std::lock_guard<std::mutex> lk(mu());
+            auto& v = blocks();
+            size_t best = v.size();
+            for (size_t i = 0; i < v.size(); ++i)
+                if (v[i].device == device && v[i].bytes >= n && v[i].bytes <= 2 * n &&
+                    (best == v.size() || v[i].bytes < v[best].bytes))
+                    best = i;
+            if (best != v.size()) {
+                out = v[best];
+                total() -= out.bytes;
+                v.erase(v.begin() + (std::ptrdiff_t)best);
+                return hipSuccess;
+            }
+        }
+        out = Block{};
+        DevBuf fresh;
+        const hipError_t e = fresh.ensure(n);
+        if (e == hipSuccess) out = Block{fresh.p, fresh.bytes, device};
+        return e;
+    }
+    static void put(Block& b) {
+        if (!b.p) return;
+        std::vector<void*> drop;
+        {
+            std::lock_guard<std::mutex> lk(mu());
+            if (b.bytes > kMax || g_contexts.load() <= 0) {
+                drop.push_back(b.p);
+            } else {
+                auto& v = blocks();
+                v.push_back(b);
+                total() += b.bytes;
+                while (total() > kMax) {   // the oldest
+                    total() -= v.front().bytes;
+                    drop.push_back(v.front().p);
+                    v.erase(v.begin());
+                }
+            }
+        }
+        for (void* p : drop) (void)hipFree(p);
+        b = Block{};
+    }
+    static bool drain() {
+        std::vector<Block> drop;
+        {
+            std::lock_guard<std::mutex> lk(mu());
+            drop.swap(blocks());
+            total() = 0;
+        }
+        for (auto& b : drop) (void)hipFree(b.p);
+        return !drop.empty();
+    }
+
+  private:
+    static constexpr size_t kMax = (size_t)1 << 30;
+    // never destroyed: adjoints may be freed during process teardown
+    static std::mutex& mu() { static std::mutex* m = new std::mutex; return *m; }
+    static std::vector<Block>& blocks() { static auto* v = new std::vector<Block>; return *v; }
+    static size_t& total() { static size_t t = 0; return t; }
+};
+
+bool drop_kept_device_blocks() { return DeviceBlockCache::drain(); }
 
 // ---- exact division check -------------------------------------------------
 
@@ -332,10 +443,12 @@ gt_status make_geom(const gt_params* p, bool integer_input, Geom& g) {
         for (int j = -g.rint; j <= g.rint; ++j) {
             if (i * i + j * j > g.rint * g.rint) continue;
             if (t >= 1024) return fail(GT_E_INVALID, "diameter too large for characterisation");
-            const float a = 2.0f * atan2f((float)j, (float)i);
-            g.r2_gpu[t] = (float)(i * i + j * j);
-            g.sin2_gpu[t] = sinf(a);
-            g.cos2_gpu[t] = cosf(a);
+            if (g.characterize) {
+                const float a = 2.0f * atan2f((float)j, (float)i);
+                g.r2_gpu[t] = (float)(i * i + j * j);
+                g.sin2_gpu[t] = sinf(a);
+                g.cos2_gpu[t] = cosf(a);
+            }
             ++t;
         }
     g.ntap_gpu = t;
@@ -345,14 +458,22 @@ gt_status make_geom(const gt_params* p, bool integer_input, Geom& g) {
         for (int j = -g.band; j <= g.band; ++j) {
             if (i * i + j * j > g.band * g.band) continue;
             if (t >= 1024) return fail(GT_E_INVALID, "diameter too large for characterisation");
-            const float a = 2.0f * atan2f((float)j, (float)i);
-            g.r2_cpu[t] = (float)(i * i + j * j);
-            g.sin_cpu[t] = sinf(a);
-            g.cos_cpu[t] = cosf(a);
+            if (g.cpu_processed) {
+                const float a = 2.0f * atan2f((float)j, (float)i);
+                g.r2_cpu[t] = (float)(i * i + j * j);
+                g.sin_cpu[t] = sinf(a);
+                g.cos_cpu[t] = cosf(a);
+            }
             ++t;
         }
     g.ntap_cpu = t;
     return GT_OK;
+}
+
+// Bytes of the parameter block that a call's kernels read: the tap tables at
+// its end only where there are columns that use them.
+size_t geom_bytes(const Geom& g) {
+    return g.raw_cols || g.characterize || g.cpu_processed ? sizeof(Geom) : offsetof(Geom, raw_tap);
 }
 
 const char* const kColFrame = "frame";
@@ -373,6 +494,9 @@ struct Workspace {
 };
 
 constexpr int kStreams = 2;
+// Result bytes that a call writes to pinned memory before it knows their
+// number: about 9000 rows, 5 us over the bus; more are copied by the engine.
+constexpr size_t kFewBytes = (size_t)256 << 10;
 
 struct gt_context {
     int device = 0;
@@ -418,7 +542,11 @@ struct gt_context {
     std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> ev_used;
     double stage_ms[GT_NSTAGES] = {0};
     uint64_t stage_launches[GT_NSTAGES] = {0};
-    DevBuf geom, frames_tab, bases, rows, rows_cand, counters;
+    // tables: the parameter block, the frame table and the batches' bases of a
+    // call, uploaded together from `up`; then the tables expanded from them
+    DevBuf tables, rows, rows_cand, counters;
+    DevBuf adj_sigma, adj_origin, adj_rowpos;   // adjoint outputs of a call
+    PinBuf up, down;   // down: a call's totals, then its rows where they are few
     Workspace ws[kStreams];
     LinkStats last_link;
     LinkCache* link_cache = nullptr;   // linker buffers, created on first use
@@ -435,16 +563,17 @@ struct gt_context {
     hipEvent_t ev_na = nullptr;
 };
 
-// Host result buffers.  Blocks of 1 MiB and more are kept when a result is
-// freed (up to 256 MiB in all) and handed to the next result that fits, so
-// calls in a loop write their rows into memory whose pages are already
-// mapped instead of faulting in fresh pages on every call.
+// Host result buffers.  Blocks of 256 KiB and more are pinned (a copy from the
+// device goes straight into them) while the pinned ones, in use or kept, stay
+// below 256 MiB, and are kept when a result is freed: the next result that fits
+// takes one, so calls in a loop write their rows into memory whose pages are
+// mapped already.  What is kept goes back when the last context is destroyed.
 class HostBlockCache {
   public:
     static void* get(size_t bytes) {
         if (bytes >= kMin) {
             std::lock_guard<std::mutex> lk(mu());
-            auto& v = blocks();
+            auto& v = kept();
             size_t best = v.size();
             for (size_t i = 0; i < v.size(); ++i)
                 if (v[i].second >= bytes && v[i].second <= 2 * bytes &&
@@ -452,42 +581,87 @@ class HostBlockCache {
                     best = i;
             if (best != v.size()) {
                 void* p = v[best].first;
-                total() -= v[best].second;
                 v.erase(v.begin() + (std::ptrdiff_t)best);
                 return p;
             }
         }
         if (injected_failure(1)) throw std::bad_alloc();
+        if (bytes >= kMin && bytes <= kMax) {
+            const size_t n = (bytes + 65535) & ~(size_t)65535;
+            std::vector<void*> drop;
+            bool room;
+            {
+                std::lock_guard<std::mutex> lk(mu());
+                auto& v = kept();
+                while (total() + n > kMax && !v.empty()) {   // the oldest kept ones make room
+                    total() -= v.front().second;
+                    pinned().erase(v.front().first);
+                    drop.push_back(v.front().first);
+                    v.erase(v.begin());
+                }
+                room = g_contexts.load() > 0 && total() + n <= kMax;
+                if (room) total() += n;
+            }
+            for (void* p : drop) (void)hipHostFree(p);
+            if (room) {
+                void* p = nullptr;
+                const bool ok = hipHostMalloc(&p, n, hipHostMallocPortable) == hipSuccess && p;
+                if (!ok) (void)hipGetLastError();
+                std::lock_guard<std::mutex> lk(mu());
+                if (ok) {
+                    pinned()[p] = n;
+                    return p;
+                }
+                total() -= n;
+            }
+        }
         void* p = std::malloc(bytes ? bytes : 1);
         if (!p) throw std::bad_alloc();
         return p;
     }
-    // bytes: the size the block was requested with (a reused block may be larger)
-    static void put(void* p, size_t bytes) {
+    static void put(void* p) {
         if (!p) return;
-        if (bytes < kMin || bytes > kMax) {
-            std::free(p);
-            return;
+        bool free_pinned = false;
+        {
+            std::lock_guard<std::mutex> lk(mu());
+            auto it = pinned().find(p);
+            if (it != pinned().end()) {
+                if (g_contexts.load() > 0) {
+                    kept().emplace_back(p, it->second);
+                    return;
+                }
+                total() -= it->second;   // nobody left who would take it
+                pinned().erase(it);
+                free_pinned = true;
+            }
         }
-        std::lock_guard<std::mutex> lk(mu());
-        auto& v = blocks();
-        v.emplace_back(p, bytes);
-        total() += bytes;
-        while (total() > kMax) {   // drop the oldest
-            total() -= v.front().second;
-            std::free(v.front().first);
-            v.erase(v.begin());
+        if (free_pinned) (void)hipHostFree(p);
+        else std::free(p);
+    }
+    static void drain() {
+        std::vector<void*> drop;
+        {
+            std::lock_guard<std::mutex> lk(mu());
+            for (auto& b : kept()) {
+                total() -= b.second;
+                pinned().erase(b.first);
+                drop.push_back(b.first);
+            }
+            kept().clear();
         }
+        for (void* p : drop) (void)hipHostFree(p);
     }
 
   private:
-    static constexpr size_t kMin = (size_t)1 << 20, kMax = (size_t)256 << 20;
+    static constexpr size_t kMin = (size_t)256 << 10, kMax = (size_t)256 << 20;
     // never destroyed: results may be freed during process teardown
     static std::mutex& mu() { static std::mutex* m = new std::mutex; return *m; }
-    static std::vector<std::pair<void*, size_t>>& blocks() {
+    static std::vector<std::pair<void*, size_t>>& kept() {
         static auto* v = new std::vector<std::pair<void*, size_t>>;
         return *v;
     }
+    // every pinned block, in use or kept
+    static std::map<void*, size_t>& pinned() { static auto* v = new std::map<void*, size_t>; return *v; }
     static size_t& total() { static size_t t = 0; return t; }
 };
 
@@ -498,7 +672,12 @@ struct HostAlloc {
     template <class U>
     HostAlloc(const HostAlloc<U>&) {}
     T* allocate(size_t n) { return (T*)HostBlockCache::get(n * sizeof(T)); }
-    void deallocate(T* p, size_t n) { HostBlockCache::put(p, n * sizeof(T)); }
+    void deallocate(T* p, size_t) { HostBlockCache::put(p); }
+    // resize() leaves new elements uninitialised: they are copied over next
+    template <class U>
+    void construct(U* p) { ::new ((void*)p) U; }
+    template <class U, class... A>
+    void construct(U* p, A&&... a) { ::new ((void*)p) U(std::forward<A>(a)...); }
     template <class U>
     bool operator==(const HostAlloc<U>&) const { return true; }
     template <class U>
@@ -528,12 +707,12 @@ struct gt_adjoint {
     bool jacobian = false;
     HostVec<float> sigma;
     HostVec<int32_t> origin, rowpos;
-    DevBuf d_jac, d_origin, d_frame_rows;
+    DeviceBlockCache::Block d_jac, d_origin, d_frame_rows;
     ~gt_adjoint() {
         delete fwd;
-        d_jac.release();
-        d_origin.release();
-        d_frame_rows.release();
+        DeviceBlockCache::put(d_jac);
+        DeviceBlockCache::put(d_origin);
+        DeviceBlockCache::put(d_frame_rows);
     }
 };
 
@@ -681,15 +860,15 @@ void collect_stage_times(gt_context* ctx) {
     ctx->ev_used.clear();
 }
 
-// Device buffers an adjoint request fills while the batches' P is resident.
+// An adjoint request: its outputs are filled while the batches' P is resident
+// (the context's adj_* buffers and, for the Jacobian, blocks that the adjoint
+// takes over).
 struct AdjReq {
     bool jacobian = false;
-    DevBuf sigma, origin, rowpos, jac;
+    DeviceBlockCache::Block jac, origin;
     ~AdjReq() {
-        sigma.release();
-        origin.release();
-        rowpos.release();
-        jac.release();
+        DeviceBlockCache::put(jac);
+        DeviceBlockCache::put(origin);
     }
 };
 
@@ -825,9 +1004,12 @@ struct LinkPipeline {
     }
 };
 
+// Host frames that are still being written: waits until frame i is there.
+using FrameReady = std::function<gt_status(size_t)>;
+
 gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in_type,
                      const gt_params* p, uint32_t flags, gt_result** out,
-                     AdjReq* adj = nullptr) {
+                     AdjReq* adj = nullptr, const FrameReady* ready = nullptr) {
     const auto t_start = std::chrono::steady_clock::now();
     if (!ctx) return fail(GT_E_INVALID, "context is NULL");
     if (!out) return fail(GT_E_INVALID, "out is NULL");
@@ -914,6 +1096,9 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
 
     // ---- batch plan -------------------------------------------------------
     const size_t max_batch = plain ? 1 : (batch_frames ? batch_frames : 4096);
+    // host frames go up in pieces, so that one piece's kernels run beside the
+    // next one's upload (64 MiB: 1.2 ms of upload, some 0.5 ms of kernels)
+    const size_t host_piece = batch_frames || plain ? SIZE_MAX : (size_t)64 << 20;
     std::vector<BatchPlan> plan;
     Need maxneed;
     {
@@ -929,7 +1114,9 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
                 m.k1 += fs.k1_items;
                 m.in_bytes += on_device ? 0 : al256(fs.px * es);
                 m.nframes += 1;
-                if (b1 > b0 && workspace_bytes(m, g, tmp_planes) > ctx->workspace_limit) break;
+                if (b1 > b0 && (workspace_bytes(m, g, tmp_planes) > ctx->workspace_limit ||
+                                m.in_bytes > host_piece))
+                    break;
                 n = m;
                 ++b1;
             }
@@ -956,7 +1143,6 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     const size_t pf_count = count_bytes(nfb);
     const size_t pf_sel = al256(nfb * 16);
     const size_t pf_8 = al256(nfb * 8);
-    HIP_TRY(ctx->geom.ensure(sizeof(Geom)));
     for (int si = 0; si < nstreams; ++si) {
         Workspace& w = ctx->ws[si];
         HIP_TRY(w.P.ensure(maxneed.px * 4));
@@ -974,7 +1160,8 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     // rows capacity: one row per 16 pixels (per 256 when Jacobian patches
     // ride along), grown on overflow
     uint64_t rows_cap = std::max<uint64_t>(4096, total_px / (adj && adj->jacobian ? 256 : 16));
-    if (!(adj && adj->jacobian) && ctx->rows.bytes >= rows_cap * 4 * g.ncols &&
+    // (an adjoint has a buffer per row besides: it takes what its own frames ask for)
+    if (!adj && ctx->rows.bytes >= rows_cap * 4 * g.ncols &&
         ctx->rows_cand.bytes >= rows_cap * 8) {
         rows_cap = std::min<uint64_t>(ctx->rows.bytes / (4 * (uint64_t)g.ncols), ctx->rows_cand.bytes / 8);
     }
@@ -985,7 +1172,12 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     // 3 x (nb + 1) entries); k_begin expands them on the device into the
     // per-item tables (frame of every bandpass item and tile, top-left tile of
     // every dedup block), so a call uploads kilobytes, not megabytes.
-    std::vector<Frame> ftab(frames.size());
+    const size_t tab_ftab = al256(sizeof(Geom));
+    const size_t tab_small = tab_ftab + al256(frames.size() * sizeof(Frame));
+    const size_t tab_big = tab_small + al256(3 * (frames.size() + plan.size()) * 4);
+    HIP_TRY(ctx->up.ensure(tab_big));
+    std::memcpy(ctx->up.p, &g, geom_bytes(g));
+    Frame* const ftab = (Frame*)(ctx->up.as<char>() + tab_ftab);
     std::vector<uint32_t> small;              // per batch: k1, tile and dedup-block bases
     std::vector<size_t> small_off(plan.size());
     std::vector<uint64_t> big_off(plan.size());   // per batch: k1_frame, tile_frame, dblock_tile
@@ -1044,12 +1236,32 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         big_off[bi] = big_total;
         big_total += (uint64_t)k1b + tb + db;
     }
-    HIP_TRY(ctx->frames_tab.ensure(ftab.size() * sizeof(Frame)));
-    HIP_TRY(ctx->bases.ensure((small.size() + big_total) * 4));
-    HIP_TRY(hipMemcpy(ctx->frames_tab.p, ftab.data(), ftab.size() * sizeof(Frame), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(ctx->bases.p, small.data(), small.size() * 4, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(ctx->geom.p, &g, sizeof(Geom), hipMemcpyHostToDevice));
-    const Geom* d_geom = ctx->geom.as<const Geom>();
+    HIP_TRY(ctx->tables.ensure(tab_big + big_total * 4));
+    std::memcpy(ctx->up.as<char>() + tab_small, small.data(), small.size() * 4);
+    char* const tab = ctx->tables.as<char>();
+    const Geom* d_geom = (const Geom*)tab;
+    const uint32_t* d_small = (const uint32_t*)(tab + tab_small);
+    const uint32_t* d_big = (const uint32_t*)(tab + tab_big);
+    // an error return leaves nothing in flight: `up`, the staging buffers and
+    // the adjoint's blocks may be written or handed on right after it
+    struct Drain {
+        gt_context* ctx;
+        ~Drain() {
+            if (!ctx) return;
+            for (hipStream_t s : ctx->streams) (void)hipStreamSynchronize(s);
+            (void)hipGetLastError();
+        }
+    } drain{ctx};
+
+    // one upload from pinned memory, ahead of every launch of the call
+    // (without column tables the block's head and the rest of the tables)
+    if (geom_bytes(g) == sizeof(Geom)) {
+        HIP_TRY(hipMemcpyAsync(tab, ctx->up.p, tab_big, hipMemcpyHostToDevice, ctx->streams[0]));
+    } else {
+        HIP_TRY(hipMemcpyAsync(tab, ctx->up.p, geom_bytes(g), hipMemcpyHostToDevice, ctx->streams[0]));
+        HIP_TRY(hipMemcpyAsync(tab + tab_ftab, ctx->up.as<char>() + tab_ftab, tab_big - tab_ftab,
+                               hipMemcpyHostToDevice, ctx->streams[0]));
+    }
 
     uint64_t launches = 0;
     const int S = adjoint_patch(g);
@@ -1058,15 +1270,20 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         HIP_TRY(ctx->rows_cand.ensure(rows_cap * 8));
         AdjOut ao{};
         if (adj) {
-            HIP_TRY(adj->sigma.ensure(rows_cap * 12));
-            HIP_TRY(adj->origin.ensure(rows_cap * 8));
-            HIP_TRY(adj->rowpos.ensure(rows_cap * 4));
-            ao.sigma = adj->sigma.as<float>();
-            ao.origin = adj->origin.as<int32_t>();
-            ao.rowpos = adj->rowpos.as<int32_t>();
+            HIP_TRY(ctx->adj_sigma.ensure(rows_cap * 12));
+            HIP_TRY(ctx->adj_rowpos.ensure(rows_cap * 4));
+            ao.sigma = ctx->adj_sigma.as<float>();
+            ao.rowpos = ctx->adj_rowpos.as<int32_t>();
             if (adj->jacobian) {
-                HIP_TRY(adj->jac.ensure(rows_cap * 12 * (uint64_t)S * S));
+                DeviceBlockCache::put(adj->jac);      // too short, on a second attempt
+                DeviceBlockCache::put(adj->origin);
+                HIP_TRY(DeviceBlockCache::get(ctx->device, rows_cap * 12 * (uint64_t)S * S, adj->jac));
+                HIP_TRY(DeviceBlockCache::get(ctx->device, rows_cap * 8, adj->origin));
                 ao.jac = adj->jac.as<float>();
+                ao.origin = adj->origin.as<int32_t>();
+            } else {
+                HIP_TRY(ctx->adj_origin.ensure(rows_cap * 8));
+                ao.origin = ctx->adj_origin.as<int32_t>();
             }
         }
         // running (rows, candidates), two pairs that the batches alternate between
@@ -1091,14 +1308,14 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             const uint32_t nb = (uint32_t)(bp.b1 - bp.b0);
             Batch b;
             std::memset(&b, 0, sizeof(b));
-            b.frames = ctx->frames_tab.as<const Frame>() + bp.b0;
-            b.k1_bases = ctx->bases.as<const uint32_t>() + small_off[bi];
+            b.frames = (const Frame*)(tab + tab_ftab) + bp.b0;
+            b.k1_bases = d_small + small_off[bi];
             b.tile_bases = b.k1_bases + nb + 1;
             b.nframes = nb;
             b.k1_items = k1_items_of[bi];
             b.tiles = tiles_of[bi];
             const uint32_t* dblock_bases = b.tile_bases + nb + 1;
-            b.k1_frame = ctx->bases.as<const uint32_t>() + small.size() + big_off[bi];
+            b.k1_frame = d_big + big_off[bi];
             b.tile_frame = b.k1_frame + b.k1_items;
             b.dblock_tile = b.tile_frame + b.tiles;
             b.dblocks = dblocks_of[bi];
@@ -1131,12 +1348,25 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             b.rows_cap = rows_cap;
 
             if (!on_device) {
+                // staged frames, which lie as the device copy does, go up
+                // together, a few MiB at a time as they become ready
+                constexpr size_t kRun = (size_t)4 << 20;
                 size_t off = 0;
-                for (size_t fi = bp.b0; fi < bp.b1; ++fi) {
-                    const size_t nbytes = (size_t)frames[fi].h * frames[fi].w * es;
+                for (size_t fi = bp.b0; fi < bp.b1;) {
+                    size_t e = fi, len = 0;
+                    for (; e < bp.b1; ++e) {
+                        if (e > fi && (!ready || len >= kRun || (const char*)frames[e].ptr !=
+                                                          (const char*)frames[fi].ptr + len))
+                            break;
+                        if (ready) GT_TRY((*ready)(e));
+                        len += al256((size_t)frames[e].h * frames[e].w * es);
+                    }
+                    const size_t last = (size_t)frames[e - 1].h * frames[e - 1].w * es;
+                    const size_t nbytes = len - al256(last) + last;
                     HIP_TRY(hipMemcpyAsync((char*)w.in_stage.p + off, frames[fi].ptr, nbytes,
                                            hipMemcpyHostToDevice, st));
-                    off += al256(nbytes);
+                    off += len;
+                    fi = e;
                 }
             }
             HIP_TRY(stage(ctx, st, GT_STAGE_ZERO, [&] {
@@ -1170,7 +1400,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             HIP_TRY(stage(ctx, st, GT_STAGE_DEDUP, [&] { return launch_dedup(b, g, d_geom, st); }));
             uint32_t max_ty = 1;
             for (size_t fi = bp.b0; fi < bp.b1; ++fi)
-                max_ty = std::max(max_ty, ftab[fi].ty);
+                max_ty = std::max(max_ty, (uint32_t)((frames[fi].h + TILE_H - 1) / TILE_H));
             // row bases continue the previous batch's count: order the scans
             if (nstreams > 1 && bi > 0)
                 HIP_TRY(hipStreamWaitEvent(st, ctx->ev_scan[(bi - 1) % nstreams], 0));
@@ -1228,6 +1458,8 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         // directly and turns graphs off for the context.
         bool launched = false;
         if (ctx->graphs && !plain && !ctx->profiling && !adj) {
+            if (ready)   // a replay copies them without asking
+                for (size_t fi = 0; fi < frames.size(); ++fi) GT_TRY((*ready)(fi));
             std::vector<uint64_t> key;
             for (const auto& f : frames) {
                 key.push_back((uint64_t)(uintptr_t)f.ptr);
@@ -1240,8 +1472,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             key.push_back(rows_cap);
             key.push_back(((uint64_t)seg << 32) | (uint32_t)nstreams);
             key.push_back(((uint64_t)batch_frames << 32) | (uint32_t)g.walk_in_detect);
-            const DevBuf* bufs[] = {&ctx->geom, &ctx->frames_tab, &ctx->bases, &ctx->rows,
-                                    &ctx->rows_cand, &ctx->counters};
+            const DevBuf* bufs[] = {&ctx->tables, &ctx->rows, &ctx->rows_cand, &ctx->counters};
             for (const DevBuf* d : bufs) key.push_back((uint64_t)(uintptr_t)d->p);
             for (int si = 0; si < nstreams; ++si) {
                 const Workspace& w = ctx->ws[si];
@@ -1292,9 +1523,17 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             GT_TRY(enqueue());
         }
         HIP_TRY(hipEventRecord(ctx->ev1, s0));
-        uint64_t cnt[2] = {0, 0};
-        HIP_TRY(hipMemcpyAsync(cnt, totals, 16, hipMemcpyDeviceToHost, s0));
+        // totals, and the rows where they are few, straight into pinned memory
+        const bool to_host = !result_on_device && !plain;
+        const uint64_t few = to_host ? std::min<uint64_t>(kFewBytes / (4 * (uint64_t)g.ncols + 8), rows_cap) : 0;
+        const size_t down_cand = 64, down_rows = down_cand + al256(few * 8);
+        HIP_TRY(ctx->down.ensure(down_rows + few * 4 * (uint64_t)g.ncols));
+        char* const down = ctx->down.as<char>();
+        HIP_TRY(launch_export(totals, ctx->rows.as<float>(), ctx->rows_cand.as<int64_t>(),
+                              (uint32_t)g.ncols, few, (uint64_t*)down, (float*)(down + down_rows),
+                              (int64_t*)(down + down_cand), s0));
         HIP_TRY(hipStreamSynchronize(s0));
+        const uint64_t cnt[2] = {((const uint64_t*)down)[0], ((const uint64_t*)down)[1]};
         float ms = 0.f;
         HIP_TRY(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
         ctx->last.device_ms = ms;
@@ -1311,11 +1550,15 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         } else if (!plain) {
             res->data.resize(total_rows * g.ncols);
             res->cand.resize(total_rows);
-            if (total_rows) {
-                HIP_TRY(hipMemcpy(res->data.data(), ctx->rows.p, total_rows * g.ncols * 4,
-                                  hipMemcpyDeviceToHost));
-                HIP_TRY(hipMemcpy(res->cand.data(), ctx->rows_cand.p, total_rows * 8,
-                                  hipMemcpyDeviceToHost));
+            if (total_rows <= few) {
+                std::memcpy(res->data.data(), down + down_rows, total_rows * g.ncols * 4);
+                std::memcpy(res->cand.data(), down + down_cand, total_rows * 8);
+            } else {
+                HIP_TRY(hipMemcpyAsync(res->data.data(), ctx->rows.p, total_rows * g.ncols * 4,
+                                       hipMemcpyDeviceToHost, s0));
+                HIP_TRY(hipMemcpyAsync(res->cand.data(), ctx->rows_cand.p, total_rows * 8,
+                                       hipMemcpyDeviceToHost, s0));
+                HIP_TRY(hipStreamSynchronize(s0));
             }
         }
         break;
@@ -1325,6 +1568,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     ctx->last.launches = launches;
     ctx->last.total_ms =
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
+    drain.ctx = nullptr;
     *out = res.release();
     return GT_OK;
 }
@@ -1452,6 +1696,7 @@ gt_status gt_context_create(int device, gt_context** out) {
     HIP_TRY(hipSetDevice(device));
     gt_context* c = new gt_context();
     c->device = device;
+    ++g_contexts;
     bool ok = true;
     for (int i = 0; i < kStreams; ++i)
         ok = ok && hipStreamCreateWithFlags(&c->streams[i], hipStreamNonBlocking) == hipSuccess &&
@@ -1461,6 +1706,7 @@ gt_status gt_context_create(int device, gt_context** out) {
          hipEventCreateWithFlags(&c->ev_na, hipEventDisableTiming) == hipSuccess;
     if (!ok) {
         delete c;
+        --g_contexts;
         return fail(GT_E_HIP, "stream/event creation failed");
     }
     c->stream = c->streams[0];
@@ -1484,9 +1730,15 @@ gt_status gt_context_destroy(gt_context* ctx) {
     (void)hipSetDevice(ctx->device);
     for (int i = 0; i < kStreams; ++i) (void)hipStreamSynchronize(ctx->streams[i]);
     ctx->drop_graphs();
-    DevBuf* bufs[] = {&ctx->geom, &ctx->frames_tab, &ctx->bases, &ctx->rows, &ctx->rows_cand,
-                      &ctx->counters};
+    DevBuf* bufs[] = {&ctx->tables, &ctx->rows, &ctx->rows_cand, &ctx->counters,
+                      &ctx->adj_sigma, &ctx->adj_origin, &ctx->adj_rowpos};
     for (DevBuf* b : bufs) b->release();
+    ctx->up.release();
+    ctx->down.release();
+    if (--g_contexts == 0) {
+        DeviceBlockCache::drain();
+        HostBlockCache::drain();
+    }
     for (int i = 0; i < kStreams; ++i) ctx->ws[i].release();
     for (void* b : ctx->pinned)
         if (b) (void)hipHostFree(b);
@@ -1661,11 +1913,14 @@ gt_status gt_context_set_batch(gt_context* ctx, uint32_t frames_per_launch) {
 }
 
 // Frames located chunk by chunk (about 256 MiB of input each).  Host frames
-// (fill given) go through the context's two pinned buffers: while chunk c is
-// uploaded and located, up to 8 threads fill chunk c + 1 (fill(frame, dst)
-// copies or decodes one frame).  Device frames (fill empty) are used in
-// place.  With search_range each located chunk is linked on a worker thread
-// while the next one is located.
+// (fill given) go through the context's two pinned buffers: up to 8 threads
+// fill a chunk (fill(frame, dst) copies or decodes one frame), each frame goes
+// up as soon as it is there, and chunk c + 1 is filled while chunk c is
+// uploaded and located.  24 frames of 2048 x 2048 from host memory: 6.4 ms when
+// a chunk was filled before its upload began, 4.7 ms now, of which the
+// upload alone is 3.5.  Device frames (fill empty) are used in place.  With
+// search_range each located chunk is linked on a worker thread while the next
+// one is located.
 static gt_status locate_staged(gt_context* ctx, const std::vector<FrameIn>& frames, int in_type,
                                const gt_params* p, uint32_t flags,
                                const std::function<gt_status(size_t, void*)>& fill,
@@ -1674,7 +1929,14 @@ static gt_status locate_staged(gt_context* ctx, const std::vector<FrameIn>& fram
     const auto t_start = std::chrono::steady_clock::now();
     HIP_TRY(hipSetDevice(ctx->device));
     const size_t es = elem_size(in_type);
-    const size_t limit = (size_t)256 << 20;
+    // device frames are chunked to link one chunk while the next is located: a
+    // quarter of the movie each, where that is neither small nor large
+    size_t limit = (size_t)256 << 20;
+    if (!host && p->has_search_range) {
+        size_t all = 0;
+        for (const auto& f : frames) all += al256((size_t)f.h * f.w * es);
+        limit = std::min(limit, std::max<size_t>(all / 4, (size_t)16 << 20));
+    }
     std::vector<size_t> starts(1, 0), offs(frames.size());
     size_t cur = 0, max_chunk = 0;
     for (size_t i = 0; i < frames.size(); ++i) {
@@ -1705,27 +1967,54 @@ static gt_status locate_staged(gt_context* ctx, const std::vector<FrameIn>& fram
     char* const buf[2] = {(char*)ctx->pinned[0], (char*)ctx->pinned[1]};
     // (error messages are per thread: the filler's travels back with it)
     using Status = std::pair<gt_status, std::string>;
-    auto fill_chunk = [&](size_t c) -> Status {
-        const size_t a = starts[c], m = starts[c + 1] - a;
-        const size_t nt = std::min<size_t>(8, m), per = (m + nt - 1) / nt;
-        std::vector<std::future<Status>> parts;
-        for (size_t t = 0; t < nt; ++t) {
-            const size_t f0 = a + t * per, f1 = std::min(a + m, f0 + per);
-            if (f0 >= f1) break;
-            parts.push_back(std::async(std::launch::async, [&, f0, f1, c]() -> Status {
-                for (size_t fi = f0; fi < f1; ++fi) {
-                    const gt_status r = fill(fi, buf[c & 1] + offs[fi]);
-                    if (r != GT_OK) return {r, gt_last_error()};
-                }
-                return {GT_OK, {}};
-            }));
-        }
+    // One chunk's frames, handed out in order to up to 8 threads; frame_ready
+    // (called by the locate that uploads them) waits for one of them.  A chunk
+    // of less than 1 MiB is filled at once.
+    struct Filling {
+        std::mutex mu;
+        std::condition_variable cv;
+        std::vector<uint8_t> done;
+        std::atomic<size_t> next{0};
         Status st{GT_OK, {}};
-        for (auto& q : parts) {
-            Status r = q.get();
-            if (st.first == GT_OK) st = std::move(r);
+        std::vector<std::future<void>> threads;
+        ~Filling() {
+            for (auto& t : threads)
+                if (t.valid()) t.wait();
         }
-        return st;
+    };
+    auto start_fill = [&](size_t c, std::shared_ptr<Filling> after) {
+        auto fl = std::make_shared<Filling>();
+        const size_t a = starts[c], m = starts[c + 1] - a;
+        fl->done.assign(m, 0);
+        auto work = [&, a, m, c](Filling* f, Filling* prev) {
+            if (prev)   // the threads of the chunk before have the host first
+                for (auto& t : prev->threads) t.wait();
+            for (size_t i; (i = f->next.fetch_add(1)) < m;) {
+                const gt_status r = guarded([&] { return fill(a + i, buf[c & 1] + offs[a + i]); });
+                std::string msg = r == GT_OK ? "" : gt_last_error();
+                std::lock_guard<std::mutex> lk(f->mu);
+                f->done[i] = 1;
+                if (r != GT_OK && f->st.first == GT_OK) f->st = {r, std::move(msg)};
+                f->cv.notify_all();
+            }
+        };
+        size_t bytes = 0;
+        for (size_t i = a; i < a + m; ++i) bytes += al256((size_t)frames[i].h * frames[i].w * es);
+        if (bytes < ((size_t)1 << 20) && !after) {
+            work(fl.get(), nullptr);
+        } else {
+            const size_t nt = std::min<size_t>(8, m);
+            for (size_t t = 0; t < nt; ++t)
+                fl->threads.push_back(std::async(std::launch::async, [work, f = fl.get(), after] {
+                    work(f, after.get());
+                }));
+        }
+        return fl;
+    };
+    auto frame_ready = [](Filling& f, size_t i) -> Status {
+        std::unique_lock<std::mutex> lk(f.mu);
+        f.cv.wait(lk, [&] { return f.done[i] != 0; });
+        return f.st;
     };
     gt_params q = *p;
     q.has_search_range = 0;   // linked once over all frames below
@@ -1746,22 +2035,26 @@ static gt_status locate_staged(gt_context* ctx, const std::vector<FrameIn>& fram
     std::unique_ptr<LinkPipeline> lp;
     if (p->has_search_range)
         lp.reset(new LinkPipeline(ctx, p, frames.size(), &res->data, &data_mu, stride));
-    if (host && nchunks) {
-        const Status r0 = fill_chunk(0);
-        if (r0.first != GT_OK) return fail(r0.first, "%s", r0.second.c_str());
-    }
+    std::shared_ptr<Filling> filling, next;
+    if (host && nchunks) filling = start_fill(0, nullptr);
     for (size_t c = 0; c < nchunks; ++c) {
-        std::future<Status> next;
-        if (host && c + 1 < nchunks) next = std::async(std::launch::async, fill_chunk, c + 1);
+        // (chunk c - 1, which used the other buffer, has been located)
+        if (host && c + 1 < nchunks) next = start_fill(c + 1, filling);
         std::vector<FrameIn> fr(frames.begin() + starts[c], frames.begin() + starts[c + 1]);
-        if (host)
+        FrameReady ready;
+        if (host) {
             for (size_t i = 0; i < fr.size(); ++i) fr[i].ptr = buf[c & 1] + offs[starts[c] + i];
+            ready = [&](size_t i) -> gt_status {
+                const Status r = frame_ready(*filling, i);
+                return r.first == GT_OK ? GT_OK : fail(r.first, "%s", r.second.c_str());
+            };
+        }
         gt_result* part = nullptr;
-        const gt_status st = run_locate(ctx, fr, in_type, &q, flags, &part);
-        const Status rs = next.valid() ? next.get() : Status{GT_OK, {}};
+        const gt_status st = run_locate(ctx, fr, in_type, &q, flags, &part, nullptr,
+                                        host ? &ready : nullptr);
         if (st != GT_OK) return st;
+        filling = std::move(next);
         std::unique_ptr<gt_result> partp(part);
-        if (rs.first != GT_OK) return fail(rs.first, "%s", rs.second.c_str());
         if (part->ncols + gap != stride) return fail(GT_E_INTERNAL, "locate: column count mismatch");
         const uint64_t r0 = res->rows;
         {
@@ -1771,7 +2064,9 @@ static gt_status locate_staged(gt_context* ctx, const std::vector<FrameIn>& fram
                 res->data.reserve(est * stride);
                 res->cand.reserve(est);
             }
-            if (!gap) {
+            if (!gap && nchunks == 1) {
+                res->data.swap(part->data);
+            } else if (!gap) {
                 res->data.insert(res->data.end(), part->data.begin(), part->data.end());
             } else {
                 const uint32_t nc = part->ncols;
@@ -1785,7 +2080,8 @@ static gt_status locate_staged(gt_context* ctx, const std::vector<FrameIn>& fram
                 }
             }
         }
-        res->cand.insert(res->cand.end(), part->cand.begin(), part->cand.end());
+        if (nchunks == 1) res->cand.swap(part->cand);
+        else res->cand.insert(res->cand.end(), part->cand.begin(), part->cand.end());
         res->rows += part->rows;
         if (lp) GT_TRY(lp->submit(fr, part->data.data(), part->rows, part->ncols, r0));
         total.device_ms += ctx->last.device_ms;
@@ -1946,7 +2242,7 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
     Geom* d_geom = (Geom*)(base + L.geom);
     uint64_t* counters = (uint64_t*)(base + L.counters);
     hipStream_t st = ctx->streams[0];
-    HIP_TRY(hipMemcpyAsync(d_geom, &g, sizeof(Geom), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(d_geom, &g, geom_bytes(g), hipMemcpyHostToDevice, st));
     uint64_t bi = 0;   // batches
     Frame* ftab = ctx->na_ftab.data();
     uint32_t* bases = ctx->na_bases.data();
@@ -2201,22 +2497,23 @@ gt_status gt_locate_adjoint(gt_context* ctx, const void* frames, int dtype, uint
         return fail(GT_E_HIP, "adjoint readback: %s", hipGetErrorString(e));
     };
     hipError_t e = hipSuccess;
+    hipStream_t st = ctx->streams[0];
+    const void* d_origin = req.jacobian ? req.origin.p : ctx->adj_origin.p;
     if (n) {
-        e = hipMemcpy(a->sigma.data(), req.sigma.p, n * 12, hipMemcpyDeviceToHost);
-        if (e == hipSuccess) e = hipMemcpy(a->origin.data(), req.origin.p, n * 8, hipMemcpyDeviceToHost);
-        if (e == hipSuccess) e = hipMemcpy(a->rowpos.data(), req.rowpos.p, n * 4, hipMemcpyDeviceToHost);
+        e = hipMemcpyAsync(a->sigma.data(), ctx->adj_sigma.p, n * 12, hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipMemcpyAsync(a->origin.data(), d_origin, n * 8, hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipMemcpyAsync(a->rowpos.data(), ctx->adj_rowpos.p, n * 4, hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
         if (e != hipSuccess) return cleanup(e);
     }
     if (req.jacobian) {
         // keep the patches and origins on the device; row range of every frame
-        std::swap(a->d_jac.p, req.jac.p);
-        std::swap(a->d_jac.bytes, req.jac.bytes);
-        std::swap(a->d_origin.p, req.origin.p);
-        std::swap(a->d_origin.bytes, req.origin.bytes);
+        std::swap(a->d_jac, req.jac);
+        std::swap(a->d_origin, req.origin);
         std::vector<uint64_t> fr(n_frames + 1, 0);
         for (uint64_t r = 0; r < n; ++r) fr[(size_t)a->rowpos[r] + 1] += 1;
         for (uint64_t f = 0; f < n_frames; ++f) fr[f + 1] += fr[f];
-        e = a->d_frame_rows.ensure(fr.size() * 8);
+        e = DeviceBlockCache::get(ctx->device, fr.size() * 8, a->d_frame_rows);
         if (e == hipSuccess) e = hipMemcpy(a->d_frame_rows.p, fr.data(), fr.size() * 8, hipMemcpyHostToDevice);
         if (e != hipSuccess) return cleanup(e);
     }

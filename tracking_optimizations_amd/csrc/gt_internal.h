@@ -184,6 +184,11 @@ hipError_t launch_dedup(const Batch& b, const Geom& g, const Geom* d_geom,
 hipError_t launch_scan(const Batch& b, uint32_t max_ty, hipStream_t s);
 hipError_t launch_emit(const Batch& b, const Geom& g, const Geom* d_geom,
                        hipStream_t s);
+// The call's totals to h_totals and, where it has at most `few` rows, those to
+// h_rows and h_cand (pinned host memory).
+hipError_t launch_export(const uint64_t* totals, const float* rows, const int64_t* cand,
+                         uint32_t ncols, uint64_t few, uint64_t* h_totals, float* h_rows,
+                         int64_t* h_cand, hipStream_t s);
 hipError_t launch_copy(void* dst, const void* src, uint64_t bytes, hipStream_t s);
 
 // Characterisation columns of every output row (gt_char.hip).

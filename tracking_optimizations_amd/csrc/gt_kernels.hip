@@ -76,6 +76,33 @@ hipError_t launch_begin(const Batch& b, const uint32_t* dblock_bases, uint32_t m
     return hipGetLastError();
 }
 
+// The end of a call: its totals and, where they are few, its rows written
+// straight to pinned host memory, so that the host waits once instead of once
+// for the totals and again for each copy.  Latency bound (about 5 us): with the
+// tables' single upload a 512 x 512 call went from 220 to 127 us.
+__global__ __launch_bounds__(256) void k_export(const uint64_t* __restrict__ totals,
+                                                const float* __restrict__ rows,
+                                                const int64_t* __restrict__ cand, uint32_t ncols,
+                                                uint64_t few, uint64_t* __restrict__ h_totals,
+                                                float* __restrict__ h_rows,
+                                                int64_t* __restrict__ h_cand) {
+    const uint64_t n = totals[0];
+    const uint64_t t0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
+    if (t0 < 2) h_totals[t0] = totals[t0];
+    if (n > few) return;
+    for (uint64_t i = t0; i < n * ncols; i += step) h_rows[i] = rows[i];
+    for (uint64_t i = t0; i < n; i += step) h_cand[i] = cand[i];
+}
+
+hipError_t launch_export(const uint64_t* totals, const float* rows, const int64_t* cand,
+                         uint32_t ncols, uint64_t few, uint64_t* h_totals, float* h_rows,
+                         int64_t* h_cand, hipStream_t s) {
+    hipLaunchKernelGGL(k_export, dim3(few ? 16 : 1), dim3(256), 0, s, totals, rows, cand, ncols, few,
+                       h_totals, h_rows, h_cand);
+    return hipGetLastError();
+}
+
 // Plain device copy: 16-byte vectors, grid-stride, byte tail.  Also the kernel
 // of known traffic (n bytes read, n written) for scaling byte counters.
 __global__ void k_copy(uint4* __restrict__ dst, const uint4* __restrict__ src, uint64_t n16,

@@ -198,8 +198,9 @@ def batch(video, diameter, minmass=None, maxsize=None, separation=None, noise_si
                               smoothing_size, threshold, invert, percentile, topn, preprocess,
                               max_iterations, characterize, filter_close, search_range, memory,
                               cpu_processed, sig_radius, bg_radius, gap_radius)
-    columns = {name: typ for name, typ in columns}
-    return pd.DataFrame(arr, columns=columns).astype(columns)
+    # a column at a time: one conversion each, no 2-d frame in between
+    return pd.DataFrame({name: arr[:, i].astype(typ) for i, (name, typ) in enumerate(columns)},
+                        copy=False)
 
 
 class MovieFile:
@@ -296,5 +297,6 @@ def batch_file(path, diameter, channel=None, minmass=None, maxsize=None, separat
                                    preprocess, max_iterations, characterize, filter_close,
                                    search_range, memory, cpu_processed, sig_radius, bg_radius,
                                    gap_radius)
-    columns = {name: typ for name, typ in columns}
-    return pd.DataFrame(arr, columns=columns).astype(columns)
+    # a column at a time: one conversion each, no 2-d frame in between
+    return pd.DataFrame({name: arr[:, i].astype(typ) for i, (name, typ) in enumerate(columns)},
+                        copy=False)

@@ -1,0 +1,36 @@
+"""Candidate slots and percentile lists of tiles that hold many: coarse levels
+and plateaus, so that windows tie and whole rows of a tile are candidates, and
+ranges of the percentile that hold a large part of the frame; partial tiles at
+both edges.  The oracle's candidates, whole numbers, are the same; bars on the
+rows as in test_gpu_parity."""
+import numpy as np
+import pytest
+
+from tests.test_gpu_parity import _check, _oracle_movie
+from tracking_optimizations_amd import _lib
+from tracking_optimizations_amd.gpu_tracking import locate, make_params
+
+pytestmark = pytest.mark.gpu
+
+
+def _coarse(h, w, seed):
+    rng = np.random.default_rng(seed)
+    blocks = rng.integers(0, 3, (2, (h + 5) // 6, (w + 8) // 9)) * 700
+    f = np.repeat(np.repeat(blocks, 6, 1), 9, 2)[:, :h, :w]
+    f[1] = (np.arange(w)[None, :] % 16 == 5) * 900 + (np.arange(h)[:, None] % 12 == 3) * 900
+    return f.astype(np.uint16)
+
+
+# one window of each kernel: by lanes (4 .. 16), by rows (18 .. 26), any size
+@pytest.mark.parametrize("diameter,separation", [(3, 3), (5, 4), (7, 6), (9, 9), (11, 11), (7, 13),
+                                                 (11, 18), (9, 20), (11, 30)])
+@pytest.mark.parametrize("percentile", [None, 10, 60, 99])
+def test_many_candidates(diameter, separation, percentile):
+    ctx = _lib.default_context(0)
+    for h, w in ((64, 48), (131, 149), (193, 97)):
+        frames = _coarse(h, w, 10 * diameter + separation)
+        kw = dict(diameter=diameter, separation=separation, percentile=percentile)
+        ref = _oracle_movie(frames, kw)
+        print(f"[detect] d={diameter} sep={separation} pct={percentile} {h}x{w}", flush=True)
+        rows, cand, _, _ = locate(frames, make_params(**kw), ctx=ctx)
+        _check(rows, cand, *ref, f"d={diameter}/sep={separation}/{percentile}/{h}x{w}")

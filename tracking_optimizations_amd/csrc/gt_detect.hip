@@ -162,6 +162,119 @@ __device__ __forceinline__ void pct_bin_range(int32_t k, uint32_t& base, uint32_
     width = (k >= HIST_BINS - 1) ? 0x80000000u - base : (1u << 19);
 }
 
+// The candidate test of a detect kernel: lane A + c of wave kw holds column c
+// of the tile (the other lanes none) in the rows kw * 16 .. + 15, `center` and
+// `cm` their values and window maxima.  Writes the tile's slots in raster
+// order, its percentile list and its counts; returns the tile's candidate
+// count, with the slots not yet visible to the other waves.
+//
+// Bound by vector instructions, so everything that is one per row is scalar:
+// the row's lanes are one compare into a scalar mask, counts and first ranks
+// are s_bcnt sums, and a store's lanes are the mask itself.  Per wave that is
+// four vector instructions a row and, where the row has an entry, six more
+// for the store, and one barrier; by per-lane bits, scans and conditional
+// stores it was 18 a row and two barriers.  40 frames of 2048 x 2048, window 15
+// with the walk: 321 us then, 289 now; 48 of 1024 x 1024: 85 and 74; window 19,
+// 96 of 517 x 663: 67 and 57; window 31, 24 of 1024 x 1024: 82 and 67.
+// s_cnt: eight counts, each wave's candidates and list entries.
+template <int A>
+__device__ __forceinline__ uint32_t row_candidates(const Batch& b, const DetParams& dp,
+                                                   const int32_t (&center)[16],
+                                                   const int32_t (&cm)[16], uint32_t item,
+                                                   uint32_t f, int H, int W, int x0, int y0,
+                                                   int tid, uint32_t* s_cnt) {
+    constexpr int N = 16;
+    const int c = tid & 63;
+    const int kw = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int v = x0 - A + c;
+    const uint64_t omask = ((1ull << TILE_W) - 1) << A;   // lanes with a column of the tile
+    const uint64_t colmask = omask & __builtin_amdgcn_ballot_w64((v < W) & (v - dp.band >= 0) &
+                                                                 (v + dp.band < W));
+    // where a disk inside the window cannot give a zero-valued maximum a row,
+    // a candidate is a positive value: values in the frame are >= +0
+    int32_t least = dp.diw != 0 ? 1 : INT32_MIN;
+    // rows m of the wave's run that can hold a candidate: band <= u0 + m <= H - 1 - band
+    const int u0 = y0 + kw * N;
+    const int rlo = max(dp.band - u0, 0), rhi = min(H - 1 - dp.band - u0, N - 1);
+    const uint32_t rowbits = rhi >= rlo ? ((2u << rhi) - (1u << rlo)) : 0u;
+    // values in the two histogram bins holding the order statistics go to
+    // the tile's list (any order), each pixel from the one tile whose
+    // output lanes hold it; out-of-frame centres are -inf and fall
+    // outside every range.  The two order statistics have adjacent
+    // ranks, so no value lies strictly between their bins: one range
+    // from the start of the lower bin to the end of the upper one holds
+    // exactly the two bins.
+    uint32_t lcnt = 0, base = 0, width = 0;
+    if (dp.has_pct) {
+        uint32_t lb, lw, hb, hw;
+        pct_bin_range(b.selstate[f * 4 + 0], lb, lw);
+        pct_bin_range(b.selstate[f * 4 + 2], hb, hw);
+        base = lw ? lb : hb;
+        width = hw ? (hb + hw - base) : lw;
+#pragma unroll
+        for (int m = 0; m < N; ++m)
+            lcnt += (uint32_t)__popcll(
+                omask & __builtin_amdgcn_ballot_w64((uint32_t)center[m] - base < width));
+    }
+    uint64_t bal[N];
+    uint32_t cnt = 0;
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        bal[m] = __builtin_amdgcn_ballot_w64(center[m] >= max(cm[m], least)) &
+                 ((rowbits >> m) & 1u ? colmask : 0ull);
+        cnt += (uint32_t)__popcll(bal[m]);
+    }
+    if (c == 0) {
+        s_cnt[kw] = cnt;
+        s_cnt[4 + kw] = lcnt;
+    }
+    __syncthreads();
+    uint32_t slot = 0, total = 0, entry = 0, ltotal = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const uint32_t n = __builtin_amdgcn_readfirstlane(s_cnt[w]);
+        slot += w < kw ? n : 0u;
+        total += n;
+        const uint32_t l = __builtin_amdgcn_readfirstlane(s_cnt[4 + w]);
+        entry += w < kw ? l : 0u;
+        ltotal += l;
+    }
+    if (tid == 0) {
+        b.tile_count[item] = total;
+        if (dp.has_pct) b.tile_lcount[item] = ltotal;
+    }
+    GLOBAL char* slots = (GLOBAL char*)(b.slots + (size_t)item * TILE_PX);
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        if (bal[m] == 0) continue;  // wave-uniform: most rows hold no candidate
+        if (__builtin_amdgcn_inverse_ballot_w64(bal[m])) {
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+                (uint32_t)(bal[m] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal[m], slot));
+            *(GLOBAL uint16_t*)(slots + (uint32_t)(2u * rank)) =
+                (uint16_t)((kw * N + m) * TILE_W + (c - A));
+        }
+        slot += (uint32_t)__popcll(bal[m]);
+    }
+    if (dp.has_pct && lcnt) {
+        GLOBAL char* list = (GLOBAL char*)(b.list + (size_t)item * TILE_PX);
+        // the rows' masks again: kept from the count they would not fit the
+        // scalar registers beside the candidates'
+        asm volatile("" : "+s"(base));
+#pragma unroll
+        for (int m = 0; m < N; ++m) {
+            const uint64_t in = omask & __builtin_amdgcn_ballot_w64((uint32_t)center[m] - base < width);
+            if (in == 0) continue;
+            if (__builtin_amdgcn_inverse_ballot_w64(in)) {
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(in >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)in, entry));
+                *(GLOBAL uint32_t*)(list + (uint32_t)(4u * rank)) = (uint32_t)center[m];
+            }
+            entry += (uint32_t)__popcll(in);
+        }
+    }
+    return total;
+}
+
 // One workgroup per 48x64 tile (TILE_W x TILE_H).  Lane c of every wave owns
 // staged column c, frame column x0 - a + c: the 64 lanes hold the tile's 48
 // columns and the dilation window's halo (KD - 1 <= 16 columns), so the
@@ -169,8 +282,8 @@ __device__ __forceinline__ void pct_bin_range(int32_t k, uint32_t& base, uint32_
 // window over them is formed by lane shifts (DPP and ds_bpermute).  The
 // staged tile ((64 + KD - 1) x 64 floats: 19.5 KB for KD = 15) is never
 // overwritten, so the walk reads it as staged; wave w tests output rows
-// 16w .. 16w + 15.  With about 20 KB of LDS and 59 VGPRs, seven workgroups
-// share a CU (the row ballots' scalar registers set that).
+// 16w .. 16w + 15.  With about 20 KB of LDS and 64 VGPRs, eight workgroups
+// share a CU.
 //
 // RI > 0: the centroid walk of every candidate (refine) runs here too, on
 // the staged tile: each candidate walks in one lane, reading its disk from
@@ -188,9 +301,7 @@ __global__ __launch_bounds__(256) void k_detect(Batch b, DetParams dp) {
     constexpr int P2 = KD >= 16 ? 16 : KD >= 8 ? 8 : KD >= 4 ? 4 : KD >= 2 ? 2 : 1;
     static_assert(TILE_W + KD - 1 <= LS, "tile and window halo must fit the 64 lanes");
     __shared__ __attribute__((aligned(16))) float L[LR * LS];
-    // candidates per tile row, then (in place) the row's first slot
-    __shared__ uint32_t s_rowcnt[TILE_H];
-    __shared__ uint32_t s_lcnt, s_total;
+    __shared__ uint32_t s_cnt[8];
 
     const int tid = threadIdx.x;
     const int c = tid & 63;
@@ -204,7 +315,6 @@ __global__ __launch_bounds__(256) void k_detect(Batch b, DetParams dp) {
     const int y0 = (int)(local / fr.tx) * TILE_H;
     const int v = x0 - A + c;         // this lane's frame column
     const GLOBAL float* P = (const GLOBAL float*)fr.P;
-    if (tid == 0) s_lcnt = 0;
 
     // Staging: wave kw fills rows kw, kw + 4, ...; every row is one 256-byte
     // load across the wave.  Tiles whose staged area lies inside the frame
@@ -300,186 +410,16 @@ __global__ __launch_bounds__(256) void k_detect(Batch b, DetParams dp) {
         }
     }
 
-    // candidates: the ballots of the wave's 16 rows stay in scalar registers
-    // (bitwise tests: no short-circuit branches); output lanes are
-    // A .. A + TILE_W - 1
-    const bool olane = (c >= A) & (c < A + TILE_W);
-    const uint64_t colmask = __builtin_amdgcn_ballot_w64(olane & (v < W) & (v - dp.band >= 0) &
-                                                         (v + dp.band < W));
-    const bool diw = dp.diw != 0;
-    // rows m of the wave's run that can hold a candidate: band <= u0 + m <= H - 1 - band
-    const int u0 = y0 + kw * N;
-    const int rlo = max(dp.band - u0, 0), rhi = min(H - 1 - dp.band - u0, N - 1);
-    const uint32_t rowbits = rhi >= rlo ? ((2u << rhi) - (1u << rlo)) : 0u;
-    uint64_t bal[N];
-    uint32_t mycnt = 0;
+    int32_t center[N];
 #pragma unroll
-    for (int m = 0; m < N; ++m) {
-        const uint64_t ge = __builtin_amdgcn_ballot_w64(x[m + A] >= wm[m]);
-        const uint64_t nz = diw ? __builtin_amdgcn_ballot_w64(x[m + A] != 0) : ~0ull;
-        bal[m] = (rowbits >> m) & 1u ? (colmask & ge & nz) : 0ull;
-        mycnt = (c == m) ? (uint32_t)__popcll(bal[m]) : mycnt;
-    }
-    if (c < N) s_rowcnt[kw * N + c] = mycnt;
-
-    if (dp.has_pct) {
-        // values in the two histogram bins holding the order statistics go to
-        // the tile's list (any order), each pixel from the one tile whose
-        // output lanes hold it; out-of-frame centres are -inf and fall
-        // outside every range.  The two order statistics have adjacent
-        // ranks, so no value lies strictly between their bins: one range
-        // from the start of the lower bin to the end of the upper one holds
-        // exactly the two bins.
-        uint32_t lb, lw, hb, hw;
-        pct_bin_range(b.selstate[f * 4 + 0], lb, lw);
-        pct_bin_range(b.selstate[f * 4 + 2], hb, hw);
-        const uint32_t base = lw ? lb : hb;
-        const uint32_t width = olane ? (hw ? (hb + hw - base) : lw) : 0u;
-        uint32_t mbits = 0;
-#pragma unroll
-        for (int m = N - 1; m >= 0; --m) {
-            const uint32_t bits = (uint32_t)x[m + A];
-            mbits = 2u * mbits + ((bits - base < width) ? 1u : 0u);
-        }
-        if (__ballot(mbits != 0u)) {  // wave-uniform
-            const uint32_t n = (uint32_t)__popc(mbits);
-            const uint32_t inc = wave_incl_scan(n, c);
-            const uint32_t tot = __shfl(inc, 63, 64);
-            uint32_t lbase = 0;
-            if (c == 0) lbase = atomicAdd(&s_lcnt, tot);
-            lbase = __builtin_amdgcn_readfirstlane(lbase);
-            uint32_t j = lbase + inc - n;
-            GLOBAL uint32_t* list = (GLOBAL uint32_t*)b.list + (size_t)item * TILE_PX;
-#pragma unroll
-            for (int m = 0; m < N; ++m) {
-                if (mbits & (1u << m)) list[j++] = (uint32_t)x[m + A];
-            }
-        }
-    }
-    __syncthreads();
-    if (tid < 64) {
-        const uint32_t cnt = s_rowcnt[tid];
-        const uint32_t inc = wave_incl_scan(cnt, tid);
-        s_rowcnt[tid] = inc - cnt;
-        if (tid == 63) {
-            b.tile_count[item] = inc;
-            s_total = inc;
-            if (dp.has_pct) b.tile_lcount[item] = s_lcnt;
-        }
-    }
-    __syncthreads();
-    GLOBAL uint16_t* slots = (GLOBAL uint16_t*)b.slots + (size_t)item * TILE_PX;
-#pragma unroll
-    for (int m = 0; m < N; ++m) {
-        if (bal[m] == 0) continue;  // wave-uniform: most row pieces hold no candidate
-        const int r = kw * N + m;
-        if ((bal[m] >> c) & 1ull) {
-            const uint32_t rank =
-                s_rowcnt[r] + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal[m] >> 32),
-                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)bal[m], 0u));
-            slots[rank] = (uint16_t)(r * TILE_W + (c - A));
-        }
-    }
+    for (int m = 0; m < N; ++m) center[m] = x[m + A];
+    const uint32_t total = row_candidates<A>(b, dp, center, wm, item, f, H, W, x0, y0, tid, s_cnt);
 
     if constexpr (RI > 0) {
-        const uint32_t total = s_total;
         if (total == 0) return;  // workgroup-uniform
+        const GLOBAL uint16_t* slots = (const GLOBAL uint16_t*)b.slots + (size_t)item * TILE_PX;
         __syncthreads();         // slots visible
         walk_tile<RI>(b, dp, L, LR, LS, LS, slots, total, item, P, H, W, x0, y0, A, tid);
-    }
-}
-
-// The candidate test of a row-first detect kernel: lane c holds output column c
-// (lanes TILE_W .. 63 none), wave kw output rows kw * 16 .. + 15, `center` and
-// `cm` their values and window maxima.  Writes the tile's slots in raster
-// order, its percentile list and its counts; returns with the tile's candidate
-// count in s_total, the slots not yet visible to the other waves.
-__device__ __forceinline__ void row_candidates(const Batch& b, const DetParams& dp,
-                                               const int32_t (&center)[16], const int32_t (&cm)[16],
-                                               uint32_t item, uint32_t f, int H, int W, int x0,
-                                               int y0, int tid, uint32_t* s_rowcnt,
-                                               uint32_t& s_lcnt, uint32_t& s_total) {
-    constexpr int N = 16;
-    const int c = tid & 63;
-    const int kw = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int v = x0 + c;
-    // candidates: the ballots of the wave's 16 rows stay in scalar registers
-    // (bitwise tests: no short-circuit branches)
-    // (lane masks combined in scalar registers: one vector compare each)
-    const uint64_t colmask = __builtin_amdgcn_ballot_w64((c < TILE_W) & (v < W) &
-                                                         (v - dp.band >= 0) & (v + dp.band < W));
-    const bool diw = dp.diw != 0;
-    // rows m of the wave's run that can hold a candidate: band <= u0 + m <= H - 1 - band
-    const int u0 = y0 + kw * N;
-    const int rlo = max(dp.band - u0, 0), rhi = min(H - 1 - dp.band - u0, N - 1);
-    const uint32_t rowbits = rhi >= rlo ? ((2u << rhi) - (1u << rlo)) : 0u;
-    uint64_t bal[N];
-    uint32_t mycnt = 0;
-#pragma unroll
-    for (int m = 0; m < N; ++m) {
-        const uint64_t ge = __builtin_amdgcn_ballot_w64(center[m] >= cm[m]);
-        const uint64_t nz = diw ? __builtin_amdgcn_ballot_w64(center[m] != 0) : ~0ull;
-        bal[m] = (rowbits >> m) & 1u ? (colmask & ge & nz) : 0ull;
-        mycnt = (c == m) ? (uint32_t)__popcll(bal[m]) : mycnt;
-    }
-    if (c < N) s_rowcnt[kw * N + c] = mycnt;
-
-    if (dp.has_pct) {
-        // values in the two histogram bins holding the order statistics go to
-        // the tile's list (any order); out-of-frame centres are -inf and
-        // fall outside every range
-        // The two order statistics have adjacent ranks, so no value lies
-        // strictly between their bins: one range from the start of the lower
-        // bin to the end of the upper one holds exactly the two bins.
-        uint32_t lb, lw, hb, hw;
-        pct_bin_range(b.selstate[f * 4 + 0], lb, lw);
-        pct_bin_range(b.selstate[f * 4 + 2], hb, hw);
-        const uint32_t base = lw ? lb : hb;
-        const uint32_t width = c < TILE_W ? (hw ? (hb + hw - base) : lw) : 0u;
-        uint32_t mbits = 0;
-#pragma unroll
-        for (int m = N - 1; m >= 0; --m) {
-            const uint32_t bits = (uint32_t)center[m];
-            mbits = 2u * mbits + ((bits - base < width) ? 1u : 0u);
-        }
-        if (__ballot(mbits != 0u)) {  // wave-uniform
-            const uint32_t n = (uint32_t)__popc(mbits);
-            const uint32_t inc = wave_incl_scan(n, c);
-            const uint32_t tot = __shfl(inc, 63, 64);
-            uint32_t base = 0;
-            if (c == 0) base = atomicAdd(&s_lcnt, tot);
-            base = __builtin_amdgcn_readfirstlane(base);
-            uint32_t j = base + inc - n;
-            GLOBAL uint32_t* list = (GLOBAL uint32_t*)b.list + (size_t)item * TILE_PX;
-#pragma unroll
-            for (int m = 0; m < N; ++m) {
-                if (mbits & (1u << m)) list[j++] = (uint32_t)center[m];
-            }
-        }
-    }
-    __syncthreads();
-    if (tid < 64) {
-        const uint32_t cnt = s_rowcnt[tid];
-        const uint32_t inc = wave_incl_scan(cnt, tid);
-        s_rowcnt[tid] = inc - cnt;
-        if (tid == 63) {
-            b.tile_count[item] = inc;
-            s_total = inc;
-            if (dp.has_pct) b.tile_lcount[item] = s_lcnt;
-        }
-    }
-    __syncthreads();
-    GLOBAL uint16_t* slots = (GLOBAL uint16_t*)b.slots + (size_t)item * TILE_PX;
-#pragma unroll
-    for (int m = 0; m < N; ++m) {
-        if (bal[m] == 0) continue;  // wave-uniform: most 64-pixel row pieces hold no candidate
-        const int r = kw * N + m;
-        if ((bal[m] >> c) & 1ull) {
-            const uint32_t rank =
-                s_rowcnt[r] + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal[m] >> 32),
-                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)bal[m], 0u));
-            slots[rank] = (uint16_t)(r * TILE_W + c);
-        }
     }
 }
 
@@ -510,9 +450,7 @@ __global__ __launch_bounds__(256) void k_detect_rows(Batch b, DetParams dp) {
     static_assert(LC - 64 <= 64, "halo wider than one extra column pass");
     static_assert(LC >= 64, "the first staging pass fills 64 columns");
     __shared__ __attribute__((aligned(16))) float L[LR * LS];
-    // candidates per tile row, then (in place) the row's first slot
-    __shared__ uint32_t s_rowcnt[TILE_H];
-    __shared__ uint32_t s_lcnt, s_total;
+    __shared__ uint32_t s_cnt[8];
 
     const int tid = threadIdx.x;
     const int a = dp.a;
@@ -524,7 +462,6 @@ __global__ __launch_bounds__(256) void k_detect_rows(Batch b, DetParams dp) {
     const int x0 = (int)(local % fr.tx) * TILE_W;
     const int y0 = (int)(local / fr.tx) * TILE_H;
     const GLOBAL float* P = (const GLOBAL float*)fr.P;
-    if (tid == 0) s_lcnt = 0;
 
     // Staging: wave w fills rows w, w+4, ...: lane = column (plus a second
     // pass over the KD-1 halo columns).  Indices are clamped into the frame
@@ -651,11 +588,14 @@ __global__ __launch_bounds__(256) void k_detect_rows(Batch b, DetParams dp) {
         sliding_max<N, KD>(x, cm);
     }
 
-    row_candidates(b, dp, center, cm, item, f, H, W, x0, y0, tid, s_rowcnt, s_lcnt, s_total);
+    // the maxima are finished here, not after the list's branch, where their
+    // two operands would be kept instead (146 registers for 77)
+#pragma unroll
+    for (int m = 0; m < N; ++m) asm volatile("" : "+v"(cm[m]));
+    const uint32_t total = row_candidates<0>(b, dp, center, cm, item, f, H, W, x0, y0, tid, s_cnt);
 
     if constexpr (RI > 0) {
         const GLOBAL uint16_t* slots = (const GLOBAL uint16_t*)b.slots + (size_t)item * TILE_PX;
-        const uint32_t total = s_total;
         if (total == 0) return;  // workgroup-uniform
         __syncthreads();         // column pass done with L; slots visible
         stage_tile(false);       // columns 0..63 again hold P
@@ -680,7 +620,7 @@ constexpr size_t wide_lds(int kd) {
 // two places of a row and of a column.
 //
 // Bound by latency and LDS (32 KB at KD = 31, 59 KB at 63: five to two
-// workgroups per CU).  24 frames of 1024^2 at diameter 21 (KD = 31): 80 us
+// workgroups per CU).  24 frames of 1024^2 at diameter 21 (KD = 31): 67 us
 // without the walk, where the straightforward window loops took 353 us.
 template <int P2, int RI>
 __global__ __launch_bounds__(256) void k_detect_wide(Batch b, DetParams dp) {
@@ -688,9 +628,7 @@ __global__ __launch_bounds__(256) void k_detect_wide(Batch b, DetParams dp) {
     constexpr int MAXRUNS = (TILE_W + P2 - 1 + N - 1) / N;            // 16-column runs of a row
     constexpr int NRUN = ((TILE_H + 2 * P2 - 2) * MAXRUNS + 255) / 256;   // of a thread
     extern __shared__ __attribute__((aligned(16))) float L[];
-    // candidates per tile row, then (in place) the row's first slot
-    __shared__ uint32_t s_rowcnt[TILE_H];
-    __shared__ uint32_t s_lcnt, s_total;
+    __shared__ uint32_t s_cnt[8];
 
     const int tid = threadIdx.x;
     const int a = dp.a, KD = dp.kd, off = KD - P2;
@@ -705,7 +643,6 @@ __global__ __launch_bounds__(256) void k_detect_wide(Batch b, DetParams dp) {
     const int y0 = (int)(local / fr.tx) * TILE_H;
     const GLOBAL float* P = (const GLOBAL float*)fr.P;
     const GLOBAL char* Pb = (const GLOBAL char*)P;
-    if (tid == 0) s_lcnt = 0;
 
     // Staging: wave w fills rows w, w + 4, ...; lane = column, then column
     // 64 + lane.  Indices are clamped into the frame so every load is in
@@ -806,11 +743,14 @@ __global__ __launch_bounds__(256) void k_detect_wide(Batch b, DetParams dp) {
 #pragma unroll
         for (int m = 0; m < N; ++m) cm[m] = max(cm[m], w2[m]);
     }
-    row_candidates(b, dp, center, cm, item, f, H, W, x0, y0, tid, s_rowcnt, s_lcnt, s_total);
+    // the maxima are finished here, not after the list's branch, where their
+    // two operands would be kept instead (146 registers for 77)
+#pragma unroll
+    for (int m = 0; m < N; ++m) asm volatile("" : "+v"(cm[m]));
+    const uint32_t total = row_candidates<0>(b, dp, center, cm, item, f, H, W, x0, y0, tid, s_cnt);
 
     if constexpr (RI > 0) {
         const GLOBAL uint16_t* slots = (const GLOBAL uint16_t*)b.slots + (size_t)item * TILE_PX;
-        const uint32_t total = s_total;
         if (total == 0) return;  // workgroup-uniform
         __syncthreads();         // column pass done with L; slots visible
         stage_tile();            // P again

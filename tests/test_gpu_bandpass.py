@@ -33,6 +33,7 @@ def _noise(shape, dtype, seed):
 @pytest.mark.parametrize("k", [2, 3, 5, 8, 9, 11, 13, 15, 16, 17, 19, 21, 23, 25, 27, 29, 31, 33])
 def test_radii_and_widths(dtype, k):
     import torch
+    torch.cuda.init()   # before the first context of a process
     ctx = _lib.default_context(0)
     r = k // 2
     for n, (h, w) in enumerate([(max(r, 9), max(r, 2)), (29, 17), (37, 127), (31, 128), (33, 129),
@@ -68,3 +69,48 @@ def test_long_segments_and_narrow_frames():
         rows, cand, _, _ = locate(frames, make_params(**kw), ctx=ctx)
         _check(rows, cand, *_oracle_movie(frames, kw), f"width {w}")
     ctx.close()
+
+
+def _blocks_of_zeros(h, w, seed):
+    # whole numbers: what is rounded stays above the denormals after scaling
+    f = np.random.default_rng(seed).integers(-300, 700, (2, h, w)).astype(np.float32)
+    f[:, 20:60, 30:90] = 0
+    f[1, :, w - 40:] = 0
+    return f
+
+
+# float quotients come from a reciprocal where every lane's is in range, else
+# from the division: zeros, values whose products with the reciprocal's low part
+# are denormal (2^-100 and below), large ones.  A power of two scales every
+# exact and every rounded step, so the rows are the same and the masses scale.
+@pytest.mark.parametrize("exponent", [-110, -100, -92, -60, 60])
+def test_float_range(exponent):
+    ctx = _lib.default_context(0)
+    frames = _blocks_of_zeros(131, 281, 5)
+    kw = dict(diameter=5, separation=6, smoothing_size=5)
+    ref = locate(frames, make_params(**kw), ctx=ctx)
+    _check(ref[0], ref[1], *_oracle_movie(frames, kw), "zeros")
+    scale = np.float32(2.0 ** exponent)
+    got = locate(frames * scale, make_params(**kw), ctx=ctx)
+    assert np.array_equal(got[1], ref[1])
+    mass = [c[0] for c in ref[2]].index("mass")
+    keep = [i for i in range(ref[0].shape[1]) if i != mass]
+    assert np.array_equal(got[0][:, keep], ref[0][:, keep])
+    assert np.array_equal(got[0][:, mass], ref[0][:, mass] * scale)
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_float_not_finite(value):
+    """One pixel that is not finite: rows out of its reach are untouched."""
+    ctx = _lib.default_context(0)
+    frames = _blocks_of_zeros(131, 281, 6)
+    p = make_params(diameter=5, separation=6, smoothing_size=5)
+    ref = locate(frames, p, ctx=ctx)
+    frames[0, 90, 150] = value
+    got = locate(frames, p, ctx=ctx)
+
+    def far(r):
+        away = (r[0][:, 0] != 0) | (np.abs(r[0][:, 2] - 90) > 40) | (np.abs(r[0][:, 3] - 150) > 40)
+        return r[0][away], r[1][away]
+
+    assert all(np.array_equal(a, b) for a, b in zip(far(got), far(ref)))

@@ -228,54 +228,60 @@ bool drop_kept_device_blocks() { return DeviceBlockCache::drain(); }
 
 // ---- exact division check -------------------------------------------------
 
-__attribute__((target("fma"))) bool corrected_div_exact_fma(float d) {
-    const float rd = 1.0f / d;
+// Whether fma(x, hi, x * lo) is the rounded x / d for every significand in
+// [1, 2), and with it for every x whose x * lo is a normal number (all three
+// then scale by powers of two).
+__attribute__((target("fma"))) bool two_part_div_exact_fma(float d, float hi, float lo) {
     for (uint32_t m = 0; m < (1u << 23); ++m) {
         const uint32_t bits = 0x3f800000u | m;
         float x;
         std::memcpy(&x, &bits, 4);
-        const float q = x * rd;
-        const float r = __builtin_fmaf(-q, d, x);
-        const float q2 = __builtin_fmaf(r, rd, q);
-        if (q2 != x / d) return false;
+        if (__builtin_fmaf(x, hi, x * lo) != x / d) return false;
     }
     return true;
 }
 
-bool corrected_div_exact_soft(float d) {
-    const float rd = 1.0f / d;
+bool two_part_div_exact_soft(float d, float hi, float lo) {
     for (uint32_t m = 0; m < (1u << 23); ++m) {
         const uint32_t bits = 0x3f800000u | m;
         float x;
         std::memcpy(&x, &bits, 4);
-        const float q = x * rd;
-        const float r = std::fma(-q, d, x);
-        const float q2 = std::fma(r, rd, q);
-        if (q2 != x / d) return false;
+        if (std::fma(x, hi, x * lo) != x / d) return false;
     }
     return true;
 }
 
-// Division x / d replaced by q = x*rd; r = fma(-q, d, x); q' = fma(r, rd, q)
-// with rd = RN(1/d) is correctly rounded for every x exactly when it is for
-// every significand in [1, 2) (the three steps commute with scaling by powers
-// of two while no result leaves the normal range).  Checked exhaustively,
-// cached per divisor.
-bool corrected_div_exact(float d) {
+// A two-part reciprocal of d that divides as above: hi = RN(1 / d) and lo near
+// 1 / d - hi.  The rounded difference misses a significand for one divisor in
+// 200; a neighbour of it has served for each of those (1500 random divisors).
+// Checked exhaustively, kept per divisor.
+bool two_part_reciprocal(float d, float& hi, float& lo) {
     static std::mutex mu;
-    static std::map<uint32_t, bool> cache;
+    static std::map<uint32_t, std::pair<bool, float>> cache;
+    if (!(d > 0.f) || !std::isfinite(d) || !std::isnormal(d)) return false;
+    hi = 1.0f / d;
     uint32_t key;
     std::memcpy(&key, &d, 4);
     {
         std::lock_guard<std::mutex> lk(mu);
         auto it = cache.find(key);
-        if (it != cache.end()) return it->second;
+        if (it != cache.end()) {
+            lo = it->second.second;
+            return it->second.first;
+        }
     }
-    if (!(d > 0.f) || !std::isfinite(d) || !std::isnormal(d)) return false;
-    const bool ok = __builtin_cpu_supports("fma") ? corrected_div_exact_fma(d)
-                                                  : corrected_div_exact_soft(d);
+    const bool hw = __builtin_cpu_supports("fma");
+    const float rest = (float)(1.0 / (double)d - (double)hi);
+    bool ok = false;
+    lo = rest;
+    for (int k = 0; k < 9 && !ok; ++k) {   // rest, then 8, 32, 72, 128 steps of 1 ulp to either side
+        const int step = 8 * ((k + 1) / 2) * ((k + 1) / 2);
+        lo = rest;
+        for (int i = 0; i < step; ++i) lo = std::nextafterf(lo, k & 1 ? INFINITY : -INFINITY);
+        ok = hw ? two_part_div_exact_fma(d, hi, lo) : two_part_div_exact_soft(d, hi, lo);
+    }
     std::lock_guard<std::mutex> lk(mu);
-    cache[key] = ok;
+    cache[key] = {ok, lo};
     return ok;
 }
 
@@ -354,7 +360,7 @@ void annulus_taps(float outer, float inner, std::vector<std::pair<int, int>>& ou
 }
 
 // Derived geometry and host tables (gpu_setup.rs:45-60, kernels.rs:134-205).
-gt_status make_geom(const gt_params* p, bool integer_input, Geom& g) {
+gt_status make_geom(const gt_params* p, Geom& g) {
     std::memset(&g, 0, sizeof(g));
     g.k = (int32_t)p->smoothing_size;
     g.R = g.k / 2;
@@ -418,17 +424,15 @@ gt_status make_geom(const gt_params* p, bool integer_input, Geom& g) {
         gn = gn + wi;
     }
     g.gn = gn;
-    g.rgn = 1.0f / gn;
     g.kk = (float)(g.k * g.k);
-    g.rkk = 1.0f / g.kk;
-    // Integer frames only.  Where weights are so small that a quotient leaves
-    // the normal range, the exact and the corrected quotient may differ in
-    // their last bits, below 2^-100; that cannot show: a nonzero pixel puts at
-    // least 1 / k^2 into the boxcar term, so an output whose Gaussian term is
-    // below 2^-60 is clamped to zero either way, and a larger one does not
-    // change when a term below 2^-100 does in its last bits.
-    g.fastdiv_gn = integer_input && corrected_div_exact(gn);
-    g.fastdiv_kk = integer_input && corrected_div_exact(g.kk);
+    // Integer frames use the quotients unchecked.  Where weights are so small
+    // that x * lo leaves the normal range, the exact and the two-part quotient
+    // may differ in their last bits, below 2^-100; that cannot show: a nonzero
+    // pixel puts at least 1 / k^2 into the boxcar term, so an output whose
+    // Gaussian term is below 2^-60 is clamped to zero either way, and a larger
+    // one does not change when a term below 2^-90 does in its last bits.
+    g.fastdiv = two_part_reciprocal(gn, g.rgn, g.rgn_lo) &&
+                two_part_reciprocal(g.kk, g.rkk, g.rkk_lo);
     // dedup neighbourhood in tiles: start pixels of two rows closer than
     // `separation` differ by less than sep + 2*(max_iterations + rint) per axis
     const double D = std::ceil((double)p->separation) + 2.0 * ((double)p->max_iterations + g.rint) + 1.0;
@@ -1023,10 +1027,9 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     const bool on_device = flags & GT_FRAMES_ON_DEVICE;
     const bool plain = flags & GT_PLAIN;
     const bool result_on_device = flags & GT_RESULT_ON_DEVICE;
-    const bool integer_input = in_type != IN_F32;
 
     Geom g;
-    GT_TRY(make_geom(p, integer_input, g));
+    GT_TRY(make_geom(p, g));
     uint64_t call_tiles = 0;
     for (const auto& f : frames) call_tiles += sizes_of(f.h, f.w, 1).tiles;
     g.walk_in_detect = ctx->fuse_walk && walk_in_detect_supported(g) &&
@@ -1810,7 +1813,7 @@ gt_status gt_context_autotune(gt_context* ctx, const gt_params* p, uint32_t h, u
     if (n_frames == 0) n_frames = 1;
     HIP_TRY(hipSetDevice(ctx->device));
     Geom g;
-    GT_TRY(make_geom(p, true, g));
+    GT_TRY(make_geom(p, g));
     // synthetic uint16 frames: background 100 + Poisson, one spot per 800 px^2
     const uint64_t npx = (uint64_t)h * w;
     struct ScopedBuf : DevBuf {
@@ -2164,9 +2167,8 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
         return fail(GT_E_HIP, "the no-allocation scratch has no device address on device %d",
                     ctx->device);
     HIP_TRY(hipSetDevice(ctx->device));
-    const bool integer_input = in_type != IN_F32;
     Geom g;
-    GT_TRY(make_geom(p, integer_input, g));
+    GT_TRY(make_geom(p, g));
     g.walk_in_detect = ctx->fuse_walk && walk_in_own_detect(g) ? 1 : 0;
     const size_t es = elem_size(in_type);
     const bool generic = !bandpass_fast_path(in_type, w, g);
@@ -2481,7 +2483,7 @@ gt_status gt_locate_adjoint(gt_context* ctx, const void* frames, int dtype, uint
     a->device = ctx->device;
     {
         Geom g;
-        make_geom(p, in_type != IN_F32, g);
+        make_geom(p, g);
         a->S = (uint32_t)adjoint_patch(g);
     }
     a->nframes = n_frames;

@@ -39,22 +39,24 @@ namespace gt {
 // uint16 filters it is kept as an integer, and where one of the wave's sums
 // reaches 2^24 the row sums are added in the shader's order instead (its
 // partial sums may round there).  Float input sums tap by tap from +0.
-// FAST selects the corrected-reciprocal division by the two per-call divisors
+// FAST selects the two-part-reciprocal division by the two per-call divisors
 // (host-verified to equal IEEE division).
 //
-// Bound by issued vector instructions: 47 per pixel at R = 5 (uint16 with a
-// histogram), of which 22 are the Gaussian's FMAs, 9 the three divisions and
-// 6 the boxcar; 40 frames of 2048^2 in 264 us, 3.8 TB/s of input and output
+// Bound by issued vector instructions (the units that carry them are never
+// idle at 40 frames of 2048^2): 43 per pixel at R = 5 (uint16 with a
+// histogram), of which 22 are the Gaussian's FMAs, 6 the three divisions and
+// 5.5 the boxcar; those frames in 267 us, 3.8 TB/s of input and output, where
+// corrected single reciprocals (nine for the divisions) took 278 beside it
 // (four columns per lane on 240-column strips, where four lanes only carry
 // halos: 301 us).  Two columns per lane halve the ring, so four waves share a
 // SIMD where three did, and leave room for R up to 16 (24 frames of 1024^2 at
-// k = 21: 80 us; two passes through a temporary plane: 1008 us) and for any
-// width and alignment (96 float32 frames of 517 x 663 at k = 13: 121 us
-// against 1032 us).
+// k = 21: 78 us; two passes through a temporary plane: 1008 us) and for any
+// width and alignment (96 float32 frames of 517 x 663 at k = 13: 105 us, 121
+// with a division for each quotient; in two passes 1032 us).
 // ---------------------------------------------------------------------------
 struct K1Params {
     float w[17];   // Gaussian weights of offsets 0 .. R (they are symmetric)
-    float gn, rgn, kk, rkk;
+    float gn, rgn, rgn_lo, kk, rkk, rkk_lo;
     int seg;
     int hist;
 };
@@ -112,13 +114,32 @@ __device__ __forceinline__ f2v unpack_pair(const Pair<T>& c, int i0, int i1) {
     return r;
 }
 
-__device__ __forceinline__ float cdiv_t(float x, float d, float rd, bool fast) {
-    if (fast) {
-        const float q = x * rd;
-        const float r = __builtin_fmaf(-q, d, x);
-        return __builtin_fmaf(r, rd, q);
+// r = x / d, correctly rounded, for a lane's two values.  FAST: by the two-part
+// reciprocal hi + lo, which the host has checked to give the rounded quotient
+// of every significand; that holds while x * lo is a normal number.  Integer
+// pixels (gt_api.hip says why) need no test of it; float pixels divide where a
+// lane's is not one (a zero, a value beyond 2^-95, infinities and NaN).
+// Two instructions a quotient where the corrected one of a single reciprocal
+// takes three and the division eleven.
+template <bool FAST, bool CHECK>
+__device__ __forceinline__ void div_pair(const float (&x)[2], float d, float hi, float lo,
+                                         float (&r)[2]) {
+    if constexpr (FAST) {
+        const float t0 = x[0] * lo, t1 = x[1] * lo;
+        r[0] = __builtin_fmaf(x[0], hi, t0);
+        r[1] = __builtin_fmaf(x[1], hi, t1);
+        if constexpr (CHECK) {
+            constexpr int NORMAL = 0x108;   // either sign
+            if (~(__builtin_amdgcn_ballot_w64(__builtin_amdgcn_classf(t0, NORMAL)) &
+                  __builtin_amdgcn_ballot_w64(__builtin_amdgcn_classf(t1, NORMAL)))) {
+                r[0] = x[0] / d;
+                r[1] = x[1] / d;
+            }
+        }
+    } else {
+        r[0] = x[0] / d;
+        r[1] = x[1] / d;
     }
-    return x / d;
 }
 
 // Order of a wave's own LDS operations: the hardware keeps it, the compiler
@@ -231,7 +252,7 @@ void k_bandpass(Batch b, K1Params kp) {
     // prefetch: row vr is loaded PF rows ahead into slot (vr - vr0) % NT, so
     // only PF + 1 slots are live at a time; as many as spill nothing (8 rows
     // ahead against 4: 264 against 272 us, 40 frames of 2048^2)
-    constexpr int PFMAX = FLT || R == 7 ? 4 : R == 4 ? 6 : 8;
+    constexpr int PFMAX = FLT ? (R == 3 ? 3 : 4) : R == 7 ? 4 : R == 4 ? 5 : R == 6 || R == 10 ? 7 : 8;
     constexpr int PF = NT < PFMAX ? NT : PFMAX;
     Pair<T> pm[NT], ph[NT];
 #pragma unroll
@@ -305,23 +326,29 @@ void k_bandpass(Batch b, K1Params kp) {
                         tb[q] = bx;
                     }
                 } else {
-                    float bx = v[HB - R];
+                    // whole numbers below 2^24, in any order: the taps that
+                    // the two columns share, then each one's own
+                    float bx = v[HB - R + 1];
 #pragma unroll
-                    for (int i = -R + 1; i <= R; ++i) bx = bx + v[HB + i];
-                    tb[0] = bx;
-                    tb[1] = (bx + v[HB + 1 + R]) - v[HB - R];
+                    for (int i = -R + 2; i <= R; ++i) bx = bx + v[HB + i];
+                    tb[0] = bx + v[HB - R];
+                    tb[1] = bx + v[HB + 1 + R];
                 }
                 // Gaussian row pass: zeros outside the frame (skipped taps).
                 // A row outside the frame sums to +0 (FMAs of +0 into +0)
                 // and so divides to +0: interior strips take that zero.
+                // (by a reciprocal of 0: the sums of integer pixels are finite)
+                constexpr bool ZERO_BY_HI = FAST && !FLT && !BORDER;
+                const float ghi = ZERO_BY_HI && !row_in ? 0.f : kp.rgn;
+                const float glo = ZERO_BY_HI && !row_in ? 0.f : kp.rgn_lo;
                 auto gauss = [&](const float (&u)[2 * HB + 2], float (&tg)[2]) {
+                    float gs[2] = {0.f, 0.f};
 #pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        float gs = 0.f;
+                    for (int q = 0; q < 2; ++q)
 #pragma unroll
-                        for (int i = -R; i <= R; ++i) gs = __builtin_fmaf(w[i < 0 ? -i : i], u[HB + q + i], gs);
-                        tg[q] = cdiv_t(gs, kp.gn, kp.rgn, FAST);
-                    }
+                        for (int i = -R; i <= R; ++i)
+                            gs[q] = __builtin_fmaf(w[i < 0 ? -i : i], u[HB + q + i], gs[q]);
+                    div_pair<FAST, FLT>(gs, kp.gn, ghi, glo, tg);
                 };
                 float tg[2];
                 if constexpr (BORDER) {
@@ -335,8 +362,10 @@ void k_bandpass(Batch b, K1Params kp) {
                     gauss(u, tg);
                 } else {
                     gauss(v, tg);
-                    tg[0] = row_in ? tg[0] : 0.f;
-                    tg[1] = row_in ? tg[1] : 0.f;
+                    if constexpr (!ZERO_BY_HI) {
+                        tg[0] = row_in ? tg[0] : 0.f;
+                        tg[1] = row_in ? tg[1] : 0.f;
+                    }
                 }
                 wave_lds_order();   // the next row overwrites the staged one
 #pragma unroll
@@ -370,16 +399,19 @@ void k_bandpass(Batch b, K1Params kp) {
                         bsum[0] = vbox[0];
                         bsum[1] = vbox[1];
                     }
-                    float out[2];
+                    float gsum[2] = {0.f, 0.f};
 #pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        float gsum = 0.f;
+                    for (int q = 0; q < 2; ++q)
 #pragma unroll
                         for (int j = 0; j < NT; ++j)
-                            gsum = __builtin_fmaf(w[j < R ? R - j : j - R], rg[(s + 1 + j) % NT][q],
-                                                  gsum);
-                        const float res = cdiv_t(gsum, kp.gn, kp.rgn, FAST) -
-                                          cdiv_t(bsum[q], kp.kk, kp.rkk, FAST);
+                            gsum[q] = __builtin_fmaf(w[j < R ? R - j : j - R],
+                                                     rg[(s + 1 + j) % NT][q], gsum[q]);
+                    float gq[2], bq[2], out[2];
+                    div_pair<FAST, FLT>(gsum, kp.gn, kp.rgn, kp.rgn_lo, gq);
+                    div_pair<FAST, FLT>(bsum, kp.kk, kp.rkk, kp.rkk_lo, bq);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const float res = gq[q] - bq[q];
                         if constexpr (FLT) out[q] = res < 0.f ? 0.f : res;   // keeps NaN
                         else out[q] = __builtin_fmaxf(res, 0.f);   // res is finite, never -0
                     }
@@ -436,11 +468,9 @@ hipError_t launch_bp_t(const Batch& b, const K1Params& kp, bool fast, hipStream_
     const size_t lds = (kp.hist ? HIST_BINS * sizeof(uint32_t) : 0) +
                        K1_WAVES * K1Shape<R>::BUF * sizeof(float);
     const dim3 grid(b.k1_items), block(64 * K1_WAVES);
-    if constexpr (!IsFloat<T>::v) {   // float input always divides exactly
-        if (fast) {
-            hipLaunchKernelGGL((k_bandpass<R, T, true>), grid, block, lds, s, b, kp);
-            return hipGetLastError();
-        }
+    if (fast) {
+        hipLaunchKernelGGL((k_bandpass<R, T, true>), grid, block, lds, s, b, kp);
+        return hipGetLastError();
     }
     hipLaunchKernelGGL((k_bandpass<R, T, false>), grid, block, lds, s, b, kp);
     return hipGetLastError();

@@ -84,10 +84,11 @@ hipError_t launch_bandpass(const Batch& b, const Geom& g, const Geom* d_geom, in
     (void)d_geom;
     K1Params kp;
     for (int i = 0; i < 17; ++i) kp.w[i] = i <= g.R ? g.w[g.R + i] : 0.f;
-    kp.gn = g.gn; kp.rgn = g.rgn; kp.kk = g.kk; kp.rkk = g.rkk;
+    kp.gn = g.gn; kp.rgn = g.rgn; kp.rgn_lo = g.rgn_lo;
+    kp.kk = g.kk; kp.rkk = g.rkk; kp.rkk_lo = g.rkk_lo;
     kp.seg = seg_rows;
     kp.hist = b.hist1 != nullptr && g.has_pct;
-    const bool fast = g.fastdiv_gn && g.fastdiv_kk;
+    const bool fast = g.fastdiv != 0;
     if (b.in_type == IN_U16) return launch_bandpass_t<uint16_t>(g.R, b, kp, fast, s);
     if (b.in_type == IN_F32) return launch_bandpass_t<float>(g.R, b, kp, fast, s);
     return launch_bandpass_t<uint8_t>(g.R, b, kp, fast, s);

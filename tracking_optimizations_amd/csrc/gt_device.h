@@ -31,16 +31,6 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t bid, uint32_t n) {
     return xcd * q + min(xcd, r) + local;
 }
 
-
-__device__ __forceinline__ float cdiv(float x, float d, float rd, int fast) {
-    if (fast) {
-        const float q = x * rd;
-        const float r = __builtin_fmaf(-q, d, x);
-        return __builtin_fmaf(r, rd, q);
-    }
-    return x / d;
-}
-
 // Percentile histogram key of a non-negative float bit pattern.
 __device__ __forceinline__ uint32_t pct_key(uint32_t bits) {
     if (bits == 0) return 0;

@@ -77,11 +77,10 @@ struct Geom {
     int32_t characterize;
     int32_t cpu_processed;
     int32_t disk_in_window;
-    int32_t fastdiv_gn;    // division by gauss_norm via corrected reciprocal
-    int32_t fastdiv_kk;    // division by k*k via corrected reciprocal
+    int32_t fastdiv;       // both divisions below by a two-part reciprocal
     float w[33];           // Gaussian weights, taps -R..R (R <= 16)
-    float gn, rgn;         // gauss_norm and its rounded reciprocal
-    float kk, rkk;         // float(k*k) and its rounded reciprocal
+    float gn, rgn, rgn_lo; // gauss_norm and its reciprocal, rounded, and the rest
+    float kk, rkk, rkk_lo; // float(k*k), likewise
     int32_t dedup_rty, dedup_rtx;  // tile radius of the dedup neighbourhood
     int32_t ncols;         // output columns
     int32_t ntap_gpu;      // disk taps (characterize tables)

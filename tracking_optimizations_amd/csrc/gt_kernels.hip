@@ -20,9 +20,9 @@
 // WGSL shader is one fused multiply-add, every other operation one binary32
 // operation in the shader's order; nothing else is contracted (this file is
 // compiled with contraction off).  Divisions by the two per-call constants
-// (gauss_norm, k*k) use a reciprocal with one residual correction only when
-// the host has verified, for every significand, that it rounds exactly like
-// IEEE division; otherwise they are IEEE divisions.
+// (gauss_norm, k*k) multiply by a two-part reciprocal only when the host has
+// verified, for every significand, that it rounds exactly like IEEE division;
+// otherwise they are IEEE divisions.
 #include <algorithm>
 #include <type_traits>
 

@@ -1175,12 +1175,12 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     // 3 x (nb + 1) entries); k_begin expands them on the device into the
     // per-item tables (frame of every bandpass item and tile, top-left tile of
     // every dedup block), so a call uploads kilobytes, not megabytes.
-    const size_t tab_ftab = al256(sizeof(Geom));
-    const size_t tab_small = tab_ftab + al256(frames.size() * sizeof(Frame));
-    const size_t tab_big = tab_small + al256(3 * (frames.size() + plan.size()) * 4);
+    const size_t tab_small = al256(frames.size() * sizeof(Frame));
+    const size_t tab_geom = tab_small + al256(3 * (frames.size() + plan.size()) * 4);
+    const size_t tab_big = tab_geom + al256(sizeof(Geom));
     HIP_TRY(ctx->up.ensure(tab_big));
-    std::memcpy(ctx->up.p, &g, geom_bytes(g));
-    Frame* const ftab = (Frame*)(ctx->up.as<char>() + tab_ftab);
+    std::memcpy(ctx->up.as<char>() + tab_geom, &g, geom_bytes(g));
+    Frame* const ftab = ctx->up.as<Frame>();
     std::vector<uint32_t> small;              // per batch: k1, tile and dedup-block bases
     std::vector<size_t> small_off(plan.size());
     std::vector<uint64_t> big_off(plan.size());   // per batch: k1_frame, tile_frame, dblock_tile
@@ -1242,7 +1242,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     HIP_TRY(ctx->tables.ensure(tab_big + big_total * 4));
     std::memcpy(ctx->up.as<char>() + tab_small, small.data(), small.size() * 4);
     char* const tab = ctx->tables.as<char>();
-    const Geom* d_geom = (const Geom*)tab;
+    const Geom* d_geom = (const Geom*)(tab + tab_geom);
     const uint32_t* d_small = (const uint32_t*)(tab + tab_small);
     const uint32_t* d_big = (const uint32_t*)(tab + tab_big);
     // an error return leaves nothing in flight: `up`, the staging buffers and
@@ -1256,15 +1256,10 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         }
     } drain{ctx};
 
-    // one upload from pinned memory, ahead of every launch of the call
-    // (without column tables the block's head and the rest of the tables)
-    if (geom_bytes(g) == sizeof(Geom)) {
-        HIP_TRY(hipMemcpyAsync(tab, ctx->up.p, tab_big, hipMemcpyHostToDevice, ctx->streams[0]));
-    } else {
-        HIP_TRY(hipMemcpyAsync(tab, ctx->up.p, geom_bytes(g), hipMemcpyHostToDevice, ctx->streams[0]));
-        HIP_TRY(hipMemcpyAsync(tab + tab_ftab, ctx->up.as<char>() + tab_ftab, tab_big - tab_ftab,
-                               hipMemcpyHostToDevice, ctx->streams[0]));
-    }
+    // one upload from pinned memory, ahead of every launch of the call, up to
+    // where the parameter block's column tables begin or end
+    HIP_TRY(hipMemcpyAsync(tab, ctx->up.p, tab_geom + geom_bytes(g), hipMemcpyHostToDevice,
+                           ctx->streams[0]));
 
     uint64_t launches = 0;
     const int S = adjoint_patch(g);
@@ -1311,7 +1306,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             const uint32_t nb = (uint32_t)(bp.b1 - bp.b0);
             Batch b;
             std::memset(&b, 0, sizeof(b));
-            b.frames = (const Frame*)(tab + tab_ftab) + bp.b0;
+            b.frames = (const Frame*)tab + bp.b0;
             b.k1_bases = d_small + small_off[bi];
             b.tile_bases = b.k1_bases + nb + 1;
             b.nframes = nb;

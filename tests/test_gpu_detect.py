@@ -34,3 +34,21 @@ def test_many_candidates(diameter, separation, percentile):
         print(f"[detect] d={diameter} sep={separation} pct={percentile} {h}x{w}", flush=True)
         rows, cand, _, _ = locate(frames, make_params(**kw), ctx=ctx)
         _check(rows, cand, *ref, f"d={diameter}/sep={separation}/{percentile}/{h}x{w}")
+
+
+@pytest.mark.parametrize("diameter,separation", [(3, 3), (9, 9), (7, 20), (11, 45)])
+def test_dedup_blocks(diameter, separation):
+    """81 frames of 9 x 9 tiles, more than have a wave each, are deduplicated
+    in blocks of 2x2 tiles; a frame at a time (the per-frame path) tile by
+    tile.  The rows are equal, and the first frame's are the oracle's."""
+    ctx = _lib.default_context(0)
+    rng = np.random.default_rng(separation)
+    frames = rng.integers(0, 400, (81, 520, 400)).astype(np.uint16)
+    frames[:, ::5, ::7] += 3      # ties in mass
+    kw = dict(diameter=diameter, separation=separation, percentile=30)
+    p = make_params(**kw)
+    got = locate(frames, p, ctx=ctx)
+    want = locate(frames, p, plain=True, ctx=ctx)
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    first = want[0][:, 0] == 0
+    _check(want[0][first], want[1][first], *_oracle_movie(frames[:1], kw), "one frame")

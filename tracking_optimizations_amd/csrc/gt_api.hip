@@ -801,6 +801,15 @@ FrameSizes sizes_of(uint32_t h, uint32_t w, int seg) {
 // 512^2 at KD = 31: 54 against 65 us).
 bool walk_apart(const Geom& g, uint64_t tiles) { return g.kd >= 18 && tiles > 1024; }
 
+// Tiles along a side of a dedup block, for a batch of `tiles`.  A block of 2x2
+// tiles stages its neighbourhood once for four tiles, but its wave works
+// through about five rounds of loads one after the other where a single tile's
+// takes three.  That is sooner done while every tile's wave is resident (24 on
+// each of 256 CUs): 18.7 -> 12.1 us for one frame of 512 x 512 (88 tiles),
+// 24.5 -> 20.4 for 64 of them (5632); past it the extra loads cost more
+// (8448 tiles, 24 frames of 1024 x 1024: 14.9 -> 22.3 us; 55040: 63 -> 164).
+uint32_t dedup_side(uint64_t tiles) { return tiles <= 256 * 24 ? 1 : 2; }
+
 int rec_planes(const Geom& g) {
     if (g.walk_in_detect && g.has_pct) return REC_CENTER + 1;
     return REC_X + 1;
@@ -1185,6 +1194,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     std::vector<size_t> small_off(plan.size());
     std::vector<uint64_t> big_off(plan.size());   // per batch: k1_frame, tile_frame, dblock_tile
     std::vector<uint32_t> k1_items_of(plan.size()), tiles_of(plan.size()), dblocks_of(plan.size());
+    std::vector<uint32_t> dside_of(plan.size());
     uint32_t max_frame_work = 1;              // largest bandpass items + tiles + blocks of a frame
     uint64_t big_total = 0;
     for (size_t bi = 0; bi < plan.size(); ++bi) {
@@ -1198,6 +1208,10 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         uint32_t* k1v = small.data() + small_off[bi];
         uint32_t* tbv = k1v + nb + 1;
         uint32_t* dbv = tbv + nb + 1;
+        uint64_t batch_tiles = 0;
+        for (size_t fi = bp.b0; fi < bp.b1; ++fi)
+            batch_tiles += sizes_of(frames[fi].h, frames[fi].w, seg).tiles;
+        const uint32_t ds = dside_of[bi] = dedup_side(batch_tiles);
         for (size_t fi = bp.b0; fi < bp.b1; ++fi) {
             const FrameSizes fs = sizes_of(frames[fi].h, frames[fi].w, seg);
             Frame& F = ftab[fi];
@@ -1220,7 +1234,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             F.k1_base = k1b;
             F.slot_base = (uint64_t)tb * TILE_PX;
             F.frame_index = frames[fi].fi;
-            const uint32_t nblk = ((fs.ty + 1) / 2) * ((fs.tx + 1) / 2);
+            const uint32_t nblk = ((fs.ty + ds - 1) / ds) * ((fs.tx + ds - 1) / ds);
             k1v[fi - bp.b0] = k1b;
             tbv[fi - bp.b0] = tb;
             dbv[fi - bp.b0] = db;
@@ -1317,6 +1331,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
             b.tile_frame = b.k1_frame + b.k1_items;
             b.dblock_tile = b.tile_frame + b.tiles;
             b.dblocks = dblocks_of[bi];
+            b.dblock_side = dside_of[bi];
             b.in_type = in_type;
             char* t3 = w.tile3.as<char>();
             const size_t t3s = al256(maxneed.tiles * 4);
@@ -2290,6 +2305,7 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
         b.tile_frame = b.k1_frame + (uint64_t)nb * fs.k1_items;
         b.dblock_tile = b.tile_frame + (uint64_t)nb * fs.tiles;
         b.dblocks = (uint32_t)(nb * dblocks_pf);
+        b.dblock_side = 2;   // a table of every tile could exceed the host tables' bound
         b.nframes = nb;
         b.k1_items = nb * fs.k1_items;
         b.tiles = nb * fs.tiles;

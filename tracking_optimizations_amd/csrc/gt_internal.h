@@ -101,11 +101,12 @@ struct Batch {
     const uint32_t* tile_bases; // [nframes + 1]
     const uint32_t* k1_frame;   // [k1_items] frame of each bandpass item
     const uint32_t* tile_frame; // [tiles] frame of each detect tile
-    const uint32_t* dblock_tile;  // [dblocks] top-left tile of each 2x2 block of tiles (dedup)
+    const uint32_t* dblock_tile;  // [dblocks] top-left tile of each block of tiles (dedup)
     uint32_t nframes;
     uint32_t k1_items;
     uint32_t tiles;
     uint32_t dblocks;
+    uint32_t dblock_side;         // tiles along a block's side: 1 or 2
     int in_type;           // InType
     // per-tile arrays [tiles]
     uint32_t* tile_count;

@@ -36,7 +36,7 @@ namespace gt {
 // begin: the first launch of a batch.  Clears the per-frame counters and
 // histograms, and expands the batch's bases into the per-item tables: frame
 // blockIdx.y writes the frame index of each of its bandpass items and tiles
-// and the top-left tile of each of its 2x2 dedup blocks (the frame's blocks in
+// and the top-left tile of each of its dedup blocks (the frame's blocks in
 // raster order).  The first batch of a call also clears the running totals
 // (`carry`, two pairs).
 // ---------------------------------------------------------------------------
@@ -47,7 +47,8 @@ __global__ __launch_bounds__(256) void k_begin(Batch b, const uint32_t* __restri
     const uint32_t ta = b.tile_bases[f], tn = b.tile_bases[f + 1] - ta;
     const uint32_t da = dbases[f], dn = dbases[f + 1] - da;
     const uint32_t tx = b.frames[f].tx;
-    const uint32_t bx = (tx + 1) / 2;   // dedup blocks per block row
+    const uint32_t ds = b.dblock_side;
+    const uint32_t bx = (tx + ds - 1) / ds;   // dedup blocks per block row
     uint32_t* k1f = (uint32_t*)b.k1_frame;
     uint32_t* tf = (uint32_t*)b.tile_frame;
     uint32_t* dt = (uint32_t*)b.dblock_tile;
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(256) void k_begin(Batch b, const uint32_t* __restri
             tf[ta + (i - k1n)] = f;
         } else {
             const uint32_t j = i - k1n - tn;
-            dt[da + j] = ta + 2 * (j / bx) * tx + 2 * (j % bx);
+            dt[da + j] = ta + ds * (j / bx) * tx + ds * (j % bx);
         }
     }
 }
@@ -542,7 +543,8 @@ hipError_t launch_refine(const Batch& b, const Geom& g, const Geom* d_geom, hipS
 
 // ---------------------------------------------------------------------------
 // K4 dedup: one wave per block of 2x2 tiles (the block's tiles share one
-// chain of dependent loads and one staged neighbourhood).  The valid records
+// chain of dependent loads and one staged neighbourhood), or per tile where a
+// batch has few (dblock_side).  The valid records
 // (mass != 0) of the tiles that can hold a neighbour, and that lie within
 // `separation` of the bounding box of the block's own valid positions, are
 // staged in LDS as 16-byte entries.  Each lane then tests its own candidate
@@ -588,7 +590,8 @@ void k_dedup(Batch b, const Geom* __restrict__ g) {
     const uint32_t local = top - fr.tile_base;
     const int W = (int)fr.W;
     const int tx = (int)(local % fr.tx), ty = (int)(local / fr.tx);
-    const bool hx = tx + 1 < (int)fr.tx, hy = ty + 1 < (int)fr.ty;
+    const int last = (int)b.dblock_side - 1;   // the block's last tile row and column
+    const bool hx = last && tx + 1 < (int)fr.tx, hy = last && ty + 1 < (int)fr.ty;
     // tile q = 2 dy + dx of the block (absent ones hold no candidate)
     const bool has[4] = {true, hx, hy, hx && hy};
     uint32_t tq[4], cq[4];
@@ -615,8 +618,8 @@ void k_dedup(Batch b, const Geom* __restrict__ g) {
     auto ok = [&](float mass, float cen) {
         return (mass != 0.f) & (!use_thr | ((double)cen > thr));
     };
-    const int y_lo = max(0, ty - rty), y_hi = min((int)fr.ty - 1, ty + 1 + rty);
-    const int x_lo = max(0, tx - rtx), x_hi = min((int)fr.tx - 1, tx + 1 + rtx);
+    const int y_lo = max(0, ty - rty), y_hi = min((int)fr.ty - 1, ty + last + rty);
+    const int x_lo = max(0, tx - rtx), x_hi = min((int)fr.tx - 1, tx + last + rtx);
     const int nxr = x_hi - x_lo + 1;
     const int ntl = (y_hi - y_lo + 1) * nxr;
 

@@ -42,11 +42,11 @@ namespace gt {
 // FAST selects the two-part-reciprocal division by the two per-call divisors
 // (host-verified to equal IEEE division).
 //
-// Bound by issued vector instructions (the units that carry them are never
-// idle at 40 frames of 2048^2): 43 per pixel at R = 5 (uint16 with a
-// histogram), of which 22 are the Gaussian's FMAs, 6 the three divisions and
-// 5.5 the boxcar; those frames in 267 us, 3.8 TB/s of input and output, where
-// corrected single reciprocals (nine for the divisions) took 278 beside it
+// Bound by issued vector instructions (the units that carry them are 80 %
+// busy): 50 per pixel at R = 5 (uint16 with a histogram, halo rows and frame
+// edges counted), of which 22 are the Gaussian's FMAs, 6 the three divisions
+// and 5.5 the boxcar; 40 frames of 2048^2 in 267 us, 3.8 TB/s of input and
+// output; corrected single reciprocals (nine for the divisions) took 278
 // (four columns per lane on 240-column strips, where four lanes only carry
 // halos: 301 us).  Two columns per lane halve the ring, so four waves share a
 // SIMD where three did, and leave room for R up to 16 (24 frames of 1024^2 at

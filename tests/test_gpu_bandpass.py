@@ -114,3 +114,16 @@ def test_float_not_finite(value):
         return r[0][away], r[1][away]
 
     assert all(np.array_equal(a, b) for a, b in zip(far(got), far(ref)))
+
+
+@pytest.mark.parametrize("dtype", ["u16", "f32"])
+@pytest.mark.parametrize("noise_size", [0.3, 1.0, 2.0, 7.5])
+def test_divisors(dtype, noise_size):
+    """Widths of the Gaussian, each a divisor of its own; with 11 taps 2.0 is
+    one whose rounded reciprocal misses a significand, so that a neighbour of
+    its low part serves."""
+    ctx = _lib.default_context(0)
+    frames = _noise((2, 90, 140), dtype, 9)
+    kw = dict(diameter=5, separation=5, smoothing_size=11, noise_size=noise_size)
+    rows, cand, _, _ = locate(frames, make_params(**kw), ctx=ctx)
+    _check(rows, cand, *_oracle_movie(frames, kw), f"{dtype}/noise={noise_size}")

@@ -120,3 +120,35 @@ def test_tap_counts(dtype, sig, bg, gap):
     names = [n for n, _ in cols]
     assert len(rows) > 60
     _check(v, rows, names, sig, bg, gap)
+
+
+@pytest.mark.parametrize("sig,bg,gap", [
+    (3.0, None, None),    # signal only
+    (3.0, 8.0, 1.0),      # background keys in registers
+    (3.0, 16.0, 1.0),     # background keys in LDS
+    (127.0 / 4, 35.0, 1.0),   # taps far from the centre
+])
+def test_infinite_positions(sig, bg, gap):
+    """Finite float32 frames near the binary32 limit: a disk's moment overflows
+    where its mass does not, so a row's y or x is infinite (the oracle's too).
+    Such a row's taps are all outside the frame: raw_mass 0, no median."""
+    from tests.test_gpu_parity import _oracle_movie
+    v = np.zeros((1, 60, 80), np.float32)
+    for i, j in ((4, 0), (3, -2), (3, 2), (3, 0), (0, 0)):
+        v[0, 20 + i, 20 + j] = v[0, 40 + j, 50 + i] = 4e37
+    v[0, 20, 20] *= 1.02
+    v[0, 40, 50] *= 1.02
+    v[0, 30, 10] = v[0, 12, 60] = 5.0
+    kw = dict(diameter=9, separation=4, smoothing_size=3, noise_size=0.05, max_iterations=1)
+    ref, cand = _oracle_movie(v, kw)[:2]
+    inf = np.isinf(ref[:, 2:4])
+    assert inf[:, 0].any() and inf[:, 1].any() and (~inf.any(axis=1)).any()
+    extra = {} if bg is None else dict(bg_radius=bg, gap_radius=gap)
+    rows, got_cand, cols, _ = locate(v, make_params(sig_radius=sig, **kw, **extra))
+    np.testing.assert_array_equal(got_cand, cand)
+    np.testing.assert_allclose(rows[:, :4], ref[:, :4], rtol=1e-5)
+    names = [n for n, _ in cols]
+    far = inf.any(axis=1)
+    _check(v, rows[~far], names, sig, bg, gap)
+    assert (rows[far, 4] == 0).all()
+    assert bg is None or np.isnan(rows[far, 5:7]).all()

@@ -110,7 +110,12 @@ __global__ __launch_bounds__(64) void k_raw(Batch b, const Geom* __restrict__ g)
         const int n = (int)min(per, nrows - q0);
         const uint64_t row = r0 + q0 + (uint32_t)min(lane, n - 1);
         float* const o = b.rows + row * (uint64_t)nc;
-        const int cy = (int)roundf(o[2]), cx = (int)roundf(o[3]);
+        // A walk over values near the binary32 limit ends at an infinite
+        // position (its moment overflows before its mass does).  No tap is
+        // more than 127 away, so a centre farther out than that reaches no
+        // pixel from wherever it is: clamped, its sums below cannot overflow.
+        const int cy = min(max((int)roundf(o[2]), -128), H + 127);
+        const int cx = min(max((int)roundf(o[3]), -128), W + 127);
         float sig = 0.f, med = 0.f;
         if constexpr (!SUM) {   // lane = row, taps in order
             const uint32_t at = index(cy, cx);

@@ -14,6 +14,12 @@
  *     use one context per host thread.
  *   - Frames are row-major H x W.  Host pointers are read during the call;
  *     device pointers (GT_FRAMES_ON_DEVICE) must stay valid until it returns.
+ *   - A locate call (gt_locate_u16/u8/f32/batch/file/adjoint) starts after the
+ *     work already queued on the device's default (null) stream, such as
+ *     kernels that write its frames or read an earlier call's device rows.
+ *     Work on non-blocking streams has to be finished by the caller.  So have
+ *     the inputs of gt_locate_noalloc and gt_adjoint_vjp, which wait for no
+ *     stream.  Every call's device work is done when it returns.
  *   - Results are float32 rows in the reference's column order
  *     (execute_gpu.rs:197-226), one row per located feature.
  */

@@ -34,6 +34,9 @@ def _adjoint(video, params, jacobian: bool, ctx=None, device: int = 0) -> Adjoin
     ctx = ctx or default_context(device)
     flags = (GT_FRAMES_ON_DEVICE if on_dev else 0) | (GT_ADJ_JACOBIAN if jacobian else 0)
     out = ctypes.c_void_p()
+    if on_dev:
+        import torch
+        torch.cuda.current_stream(video.device).synchronize()
     check(load().gt_locate_adjoint(ctx.handle, ctypes.c_void_p(ptr), _lib.DTYPE_CODES[dt], n, h, w,
                                    ctypes.byref(params), flags, ctypes.byref(out)))
     del keep

@@ -1273,6 +1273,13 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         }
     } drain{ctx};
 
+    // The call comes after what the caller has queued on the device's default
+    // stream: frames on the GPU may still be being computed there, and rows
+    // that an earlier call left on the GPU may still be being read.  (The
+    // context's streams are non-blocking: nothing else orders them.)  The host
+    // waits, which costs nothing measurable while that stream is idle; an event
+    // there that streams[0] waits for costs 14 us a call.
+    HIP_TRY(hipStreamSynchronize(nullptr));
     // one upload from pinned memory, ahead of every launch of the call, up to
     // where the parameter block's column tables begin or end
     HIP_TRY(hipMemcpyAsync(tab, ctx->up.p, tab_geom + geom_bytes(g), hipMemcpyHostToDevice,

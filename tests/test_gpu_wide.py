@@ -49,3 +49,41 @@ def test_windows_and_radii(diameter, separation):
                 finally:
                     ctx.set_fused_walk(True)
                 _check(rows, cand, *ref, f"d={diameter}/sep={separation}/{h}x{w}/{pct}/{fused}")
+
+
+def _spots_and_bad_pixels(value):
+    """Float32 spots on zeros, and a pixel of `value` 14 pixels from each: in its
+    window from separation 20 on, out of reach of its disk and of its filter."""
+    yy, xx = np.mgrid[:150, :203]
+    f = np.zeros((1, 150, 203), np.float32)
+    bad = []
+    for k, (y, x) in enumerate(((40, 40), (41, 95), (40, 150), (104, 70), (105, 131))):
+        r2 = (yy - y) ** 2 + (xx - x) ** 2
+        f[0] += np.where(r2 <= 16, (300 + 20 * k) * np.exp(-r2 / 6.0), 0).astype(np.float32)
+        bad.append((0, y + (0, 14, 0, -14, 10)[k], x + (14, 0, -14, 0, 10)[k]))
+    g = f.copy()
+    for b in bad:
+        g[b] = value
+    return f, g
+
+
+@pytest.mark.parametrize("separation", [20, 22, 23, 30, 44, 45, 46])   # windows 28 .. 63, 65
+@pytest.mark.parametrize("value", [np.nan, -np.nan, np.inf, -np.inf])
+def test_not_finite_pixels_hide_no_neighbour(separation, value):
+    """Windows without a kernel of their own skip NaN: the rows are those of the
+    frame without the pixels; a percentile that is NaN leaves none."""
+    ctx = _lib.default_context(0)
+    clean, frames = _spots_and_bad_pixels(np.float32(value))
+    for pct in (None, 60):
+        kw = dict(diameter=9, separation=separation, percentile=pct)
+        ref = _oracle_movie(clean, kw)
+        assert len(ref[0]) >= 3
+        for fused in (True, False):
+            ctx.set_fused_walk(fused)
+            try:
+                rows, cand, _, _ = locate(frames, make_params(**kw), ctx=ctx)
+                none, _, _, _ = locate(frames, make_params(**{**kw, "percentile": 99.5}), ctx=ctx)
+            finally:
+                ctx.set_fused_walk(True)
+            _check(rows, cand, *ref, f"sep={separation}/{value}/{pct}/{fused}")
+            assert len(none) == 0

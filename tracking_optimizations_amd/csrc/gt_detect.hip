@@ -21,6 +21,7 @@ struct DetParams {
     int diw;            // disk inside window (zero-valued maxima cannot yield rows)
     int has_pct;
     int walk_ri;        // disk radius of the walk run inside detect (0: none)
+    int nans;           // k_detect_wide: NaN values hide no neighbour
     uint32_t maxit;
     float minmass;
     uint64_t slot_cap;
@@ -619,6 +620,13 @@ constexpr size_t wide_lds(int kd) {
 // max(L[r][c .. c + P2 - 1]) over the staged tile, the column pass joins the
 // two places of a row and of a column.
 //
+// nans: windows of 28 and more skip NaN (P of float frames whose pixels are
+// not all finite), as the shader's compare does and as float maxima do: it is
+// staged as -inf for the maxima and is no candidate itself.  (Up to 26 a NaN
+// outranks its neighbours here as in the windows' own kernels, so that a call
+// may take either.)  The staged tile is gone over once more for it, so that
+// integer frames only skip three branches.
+//
 // Bound by latency and LDS (32 KB at KD = 31, 59 KB at 63: five to two
 // workgroups per CU).  24 frames of 1024^2 at diameter 21 (KD = 31): 67 us
 // without the walk, where the straightforward window loops took 353 us.
@@ -678,6 +686,13 @@ __global__ __launch_bounds__(256) void k_detect_wide(Batch b, DetParams dp) {
         }
     };
     stage_tile();
+    const int32_t inf = 0x7f800000;
+    if (dp.nans) {   // uniform; every thread over the cells it has stored
+        int32_t* cells = (int32_t*)L + (tid & 63);
+        for (int r = tid >> 6; r < LR; r += 4)
+            for (int j = 0; j + (tid & 63) < LC; j += 64)
+                if (cells[r * LS + j] > inf) cells[r * LS + j] = (int32_t)NEG_INF_BITS;
+    }
     __syncthreads();
 
     // the max filter works on the bit patterns (see sliding_max)
@@ -688,6 +703,16 @@ __global__ __launch_bounds__(256) void k_detect_wide(Batch b, DetParams dp) {
     int32_t center[N];
 #pragma unroll
     for (int m = 0; m < N; ++m) center[m] = Li[(kw * N + m + a) * LS + (cc + a)];
+    if (dp.nans) {   // the values themselves, for the percentile list
+#pragma unroll
+        for (int m = 0; m < N; ++m) {
+            const int u = y0 + kw * N + m, v = x0 + cc;
+            const uint32_t o = 4u * (uint32_t)(min(u, H - 1) * W + min(v, W - 1));
+            // patterns with the sign set (NaNs) count to the last bin
+            const uint32_t x = min(*(const GLOBAL uint32_t*)(Pb + o), (uint32_t)INT32_MAX - 1);
+            center[m] = u < H && v < W ? (int32_t)x : (int32_t)NEG_INF_BITS;
+        }
+    }
 
     // row pass: max(L[r][c .. c + P2 - 1]) for c < TILE_W + off, over L; the
     // last run of a row reads (but never uses) cells past it
@@ -742,6 +767,10 @@ __global__ __launch_bounds__(256) void k_detect_wide(Batch b, DetParams dp) {
         window(kw * N + off, w2);
 #pragma unroll
         for (int m = 0; m < N; ++m) cm[m] = max(cm[m], w2[m]);
+        if (dp.nans) {
+#pragma unroll
+            for (int m = 0; m < N; ++m) cm[m] = center[m] > inf ? INT32_MAX : cm[m];
+        }
     }
     // the maxima are finished here, not after the list's branch, where their
     // two operands would be kept instead (146 registers for 77)
@@ -854,9 +883,8 @@ __global__ __launch_bounds__(256) void k_detect_generic(Batch b, DetParams dp) {
     }
 }
 
-// Dilation windows too wide for the staged tile of k_detect_generic (its
-// (64 + kd - 1)^2 + (64 + kd - 1) * 64 floats exceed 60 KB from kd = 61, i.e.
-// separation 44): the row maxima of max_rows.wgsl are written to a plane
+// Dilation windows too wide for a staged tile (k_detect_wide's reaches 64 KB of
+// LDS past kd = 63, i.e. from separation 46 on): the row maxima of max_rows.wgsl are written to a plane
 // (the frame's tmp buffer) by one kernel, and the column test of
 // walk_cols.wgsl:23-34 reads that plane in a second.  Each output takes kd
 // loads (coalesced across the wave, reused through the caches), as the
@@ -1060,6 +1088,7 @@ hipError_t launch_detect(const Batch& b, const Geom& g, const Geom* d_geom, hipS
     dp.diw = g.disk_in_window;
     dp.has_pct = g.has_pct;
     dp.walk_ri = g.walk_in_detect ? g.rint : 0;
+    dp.nans = b.in_type == IN_F32 && !detect_specialised(g.kd);
     dp.maxit = g.max_iterations;
     dp.minmass = g.minmass;
     dp.slot_cap = b.slot_cap;

@@ -171,13 +171,16 @@ gt_status gt_context_set_graphs(gt_context* ctx, int enable);
 gt_status gt_context_set_launch_shape(gt_context* ctx, uint32_t seg_rows);
 
 /* Autotuner: times the batched path on n_frames synthetic uint16 frames of
- * h x w for every launch shape (rows per bandpass work item 64/128/256,
- * frames per launch automatic/16/32, the centroid walk inside detect or in
- * its own kernel where both are possible) and keeps the fastest in the
- * context for calls whose frames are all h x w with the same filter
- * geometry.  Results do not depend on the shape. */
+ * h x w for every launch shape (rows per bandpass work item chosen by the
+ * library or 64/128/256, frames per launch automatic/16/32, the centroid walk
+ * inside detect or in its own kernel where a call of this size chooses) and
+ * keeps the fastest in the context for calls whose frames are all h x w with
+ * the same filter geometry; its rows per work item for those among them that
+ * fill the device as the tuned call does (shorter calls keep the library's
+ * choice).  Results do not depend on the shape. */
 typedef struct gt_tuning {
-    uint32_t seg_rows;            /* rows per bandpass work item */
+    uint32_t seg_rows;            /* the fastest of 64/128/256; taken where it beats the
+                                     library's own choice */
     uint32_t frames_per_launch;   /* 0 = as many as the workspace holds */
     double device_ms_per_frame;   /* of the chosen shape */
     uint32_t fused_walk;          /* 1: walk inside detect, 0: separate refine kernel */

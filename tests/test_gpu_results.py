@@ -73,3 +73,39 @@ def test_results_and_adjoints_kept_while_others_are_made():
     assert not errors, errors
     assert np.array_equal(held.jacobian(), jac)
     assert np.array_equal(res[0], rows)
+
+
+def _stage_ms(ctx, frames, p, stage):
+    ms = []
+    for _ in range(30):
+        ctx.set_profiling(True)
+        locate(frames, p, ctx=ctx)
+        ms.append(ctx.stage_times()[stage][0])
+    ctx.set_profiling(False)
+    return min(ms)
+
+
+def test_tuning_on_a_movie_leaves_one_frame_its_short_segments():
+    """Tuned on 40 frames, whose bandpass runs in long segments, one frame of
+    the shape keeps the short ones of an untuned context (10 against 29 us; the
+    bar lies between)."""
+    p = make_params(diameter=9)
+    one = _noise(1, 512, 512, np.uint16, 5)
+    plain, tuned = _lib.Context(0), _lib.Context(0)
+    t = tuned.autotune(p, 512, 512, n_frames=40)
+    assert t["seg_rows"] in (64, 128, 256)
+    a, b = _stage_ms(plain, one, p, "bandpass"), _stage_ms(tuned, one, p, "bandpass")
+    print(f"[tune] {t} one frame {1000 * a:.1f} us untuned, {1000 * b:.1f} us tuned", flush=True)
+    assert b < 1.5 * a
+
+
+def test_tuning_reports_the_walk_that_runs():
+    """A window of 18 and more over more than 1024 tiles walks in a kernel of
+    its own whichever is asked for; fewer tiles walk inside detect or not as
+    measured."""
+    p = make_params(diameter=13)   # window 19
+    ctx = _lib.Context(0)
+    assert ctx.autotune(p, 512, 512, n_frames=16)["fused_walk"] is False   # 1408 tiles
+    ref = locate(_noise(1, 512, 512, np.uint16, 6), p, ctx=_lib.Context(0))
+    got = locate(_noise(1, 512, 512, np.uint16, 6), p, ctx=ctx)
+    assert all(np.array_equal(x, y) for x, y in zip(ref[:2], got[:2]))

@@ -535,10 +535,14 @@ struct gt_context {
         for (auto& e : gcache) (void)hipGraphExecDestroy(e.exec);
         gcache.clear();
     }
-    // autotuned (rows per bandpass work item, frames per launch) per frame
-    // shape and filter geometry
+    // autotuned (rows per bandpass work item, frames per launch, fused walk)
+    // per frame shape and filter geometry.  seg holds for calls of which
+    // bandpass_seg makes what it made of the tuned one (rule): a call with
+    // fewer rows to spread over the chip needs shorter segments, whatever the
+    // tuned call preferred (one frame of 512 x 512 at d = 9: 10 us at the
+    // rule's segment, 29 at the 64 rows that 40 frames are tuned to).
     struct Tuned {
-        int seg;
+        int seg, rule;
         uint32_t batch;
         int fuse;
     };
@@ -1046,18 +1050,16 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
     for (const auto& f : frames) call_tiles += sizes_of(f.h, f.w, 1).tiles;
     g.walk_in_detect = ctx->fuse_walk && walk_in_detect_supported(g) &&
                        !walk_apart(g, call_tiles) ? 1 : 0;
-    // autotuned launch shape for calls whose frames all share one shape
-    int seg = ctx->seg_rows;
-    if (!ctx->seg_set) {
-        uint64_t total = 0, largest = 0;
-        for (const auto& f : frames) {
-            const uint64_t r = strip_rows(f.h, f.w);
-            total += r;
-            largest = std::max(largest, r);
-        }
-        // on the per-frame path every frame is a launch of its own
-        seg = bandpass_seg(g, plain ? largest : total, largest);
+    uint64_t total_rows_in = 0, most_rows_in = 0;
+    for (const auto& f : frames) {
+        const uint64_t r = strip_rows(f.h, f.w);
+        total_rows_in += r;
+        most_rows_in = std::max(most_rows_in, r);
     }
+    // on the per-frame path every frame is a launch of its own
+    const int seg_rule = bandpass_seg(g, plain ? most_rows_in : total_rows_in, most_rows_in);
+    int seg = ctx->seg_set ? ctx->seg_rows : seg_rule;
+    // autotuned launch shape for calls whose frames all share one shape
     uint32_t batch_frames = ctx->batch_frames;
     if (!frames.empty() && ctx->batch_frames == 0 && !plain) {
         bool uniform = true;
@@ -1065,7 +1067,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         if (uniform) {
             auto it = ctx->tuned.find(tune_key(frames[0].h, frames[0].w, g));
             if (it != ctx->tuned.end()) {
-                seg = it->second.seg;
+                if (it->second.rule == seg_rule) seg = it->second.seg;
                 batch_frames = it->second.batch;
                 if (!it->second.fuse) g.walk_in_detect = 0;
             }
@@ -1871,12 +1873,16 @@ gt_status gt_context_autotune(gt_context* ctx, const gt_params* p, uint32_t h, u
     const int saved_fuse = ctx->fuse_walk;
     ctx->graphs = 0;
     ctx->tuned.erase(tune_key(h, w, g));
-    const int segs[] = {64, 128, 256};
+    const uint64_t rows = strip_rows(h, w);
+    const int rule = bandpass_seg(g, rows * n_frames, rows);
+    const int segs[] = {0, 64, 128, 256};   // 0: the rule's
     const uint32_t batches[] = {0, 16, 32};
-    // the walk inside detect or in its own kernel, where both are possible
-    const int nfuse = (saved_fuse && walk_in_detect_supported(g)) ? 2 : 1;
-    double best = 1e30;
-    int best_seg = saved_seg, best_fuse = saved_fuse;
+    // the walk inside detect or in its own kernel, where a call chooses
+    const bool can_fuse = saved_fuse && walk_in_detect_supported(g) &&
+                          !walk_apart(g, (uint64_t)sizes_of(h, w, 1).tiles * n_frames);
+    const int nfuse = can_fuse ? 2 : 1;
+    double best = 1e30, best_fixed = 1e30;
+    int best_seg = rule, fixed_seg = segs[1], best_fuse = saved_fuse;
     uint32_t best_batch = 0;
     gt_status st = GT_OK;
     for (int fz = 0; fz < nfuse && st == GT_OK; ++fz) {
@@ -1885,7 +1891,7 @@ gt_status gt_context_autotune(gt_context* ctx, const gt_params* p, uint32_t h, u
             for (uint32_t bf : batches) {
                 if (bf && bf >= n_frames) continue;
                 ctx->seg_rows = sg;
-                ctx->seg_set = true;
+                ctx->seg_set = sg != 0;
                 ctx->batch_frames = bf;
                 double ms = 1e30;
                 for (int rep = 0; rep < 3 && st == GT_OK; ++rep) {
@@ -1896,9 +1902,13 @@ gt_status gt_context_autotune(gt_context* ctx, const gt_params* p, uint32_t h, u
                     if (rep > 0) ms = std::min(ms, (double)ctx->last.device_ms);
                 }
                 if (st != GT_OK) break;
+                if (sg && ms < best_fixed) {
+                    best_fixed = ms;
+                    fixed_seg = sg;
+                }
                 if (ms < best) {
                     best = ms;
-                    best_seg = sg;
+                    best_seg = sg ? sg : rule;
                     best_batch = bf;
                     best_fuse = ctx->fuse_walk;
                 }
@@ -1912,12 +1922,12 @@ gt_status gt_context_autotune(gt_context* ctx, const gt_params* p, uint32_t h, u
     ctx->graphs = saved_graphs;
     ctx->fuse_walk = saved_fuse;
     if (st != GT_OK) return st;
-    ctx->tuned[tune_key(h, w, g)] = {best_seg, best_batch, best_fuse};
+    ctx->tuned[tune_key(h, w, g)] = {best_seg, rule, best_batch, best_fuse};
     if (out) {
-        out->seg_rows = (uint32_t)best_seg;
+        out->seg_rows = (uint32_t)fixed_seg;
         out->frames_per_launch = best_batch;
         out->device_ms_per_frame = best / n_frames;
-        out->fused_walk = (uint32_t)(best_fuse && walk_in_detect_supported(g));
+        out->fused_walk = can_fuse && best_fuse ? 1u : 0u;
     }
     return GT_OK;
     });

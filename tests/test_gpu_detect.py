@@ -52,3 +52,33 @@ def test_dedup_blocks(diameter, separation):
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
     first = want[0][:, 0] == 0
     _check(want[0][first], want[1][first], *_oracle_movie(frames[:1], kw), "one frame")
+
+
+@pytest.mark.parametrize("separation", [2, 4, 9, 14, 25])
+@pytest.mark.parametrize("spots", [(), ((30, 70), (110, 30)), ((20, 34),)])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_masses_beyond_binary32(separation, spots, transpose):
+    """Finite float32 pixels near the limit give disks of infinite mass and so a
+    NaN in y (or x): near no other record, such a row is kept wherever it
+    lies, alone in its tile or block or beside finite ones."""
+    f = np.zeros((1, 150, 170), np.float32)
+    for y, x in ((20, 20), (40, 60), (100, 100)):
+        for i, j in ((4, 0), (3, -2), (3, 2), (0, 0), (0, 4)):
+            f[0, y + i, x + j] = 8e37
+        f[0, y, x] *= 1.02
+    for y, x in spots:
+        f[0, y, x] = 50
+    if transpose:
+        f = np.ascontiguousarray(f.transpose(0, 2, 1))
+    kw = dict(diameter=9, separation=separation, smoothing_size=3, noise_size=0.05)
+    ref, ref_cand = _oracle_movie(f, kw)
+    assert np.isnan(ref[:, 2:4]).any(axis=1).sum() >= 3 and np.isinf(ref[:, 1]).any()
+    ctx = _lib.default_context(0)
+    for fused in (True, False):
+        ctx.set_fused_walk(fused)
+        try:
+            rows, cand, _, _ = locate(f, make_params(**kw), ctx=ctx)
+        finally:
+            ctx.set_fused_walk(True)
+        np.testing.assert_array_equal(cand, ref_cand)
+        np.testing.assert_allclose(rows, ref, rtol=1e-5, atol=1e-4)

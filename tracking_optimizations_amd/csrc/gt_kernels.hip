@@ -623,12 +623,16 @@ void k_dedup(Batch b, const Geom* __restrict__ g) {
     const int nxr = x_hi - x_lo + 1;
     const int ntl = (y_hi - y_lo + 1) * nxr;
 
-    // bounding box of the block's own valid positions
+    // bounding box of the block's own valid positions (a NaN, which a mass
+    // beyond binary32 gives, widens none: such a record is near no other, and
+    // an axis that has only those keeps an empty box, which takes no record)
+    bool some = false;
     float bymin = INFINITY, bymax = -INFINITY, bxmin = INFINITY, bxmax = -INFINITY;
     for (uint32_t j = lane; j < own_n; j += 64) {
         const size_t sl = own_slot(j, own_q(j));
         const float m0 = rmass[sl], c0 = cen_of(sl), y = ry[sl], x = rx[sl];
         if (ok(m0, c0)) {
+            some = true;
             bymin = fminf(bymin, y); bymax = fmaxf(bymax, y);
             bxmin = fminf(bxmin, x); bxmax = fmaxf(bxmax, x);
         }
@@ -645,7 +649,7 @@ void k_dedup(Batch b, const Geom* __restrict__ g) {
             atomicAdd((unsigned long long*)&b.counts[(size_t)f * b.count_stride],
                       (unsigned long long)kept_n | ((unsigned long long)own_n << 32));
     };
-    if (!(bymin <= bymax)) {  // no valid own record
+    if (!__ballot(some)) {  // no valid own record
         count(0);
         for (uint32_t j = lane; j < own_n; j += 64) b.keep[own_slot(j, own_q(j))] = 0;
 #pragma unroll
@@ -668,8 +672,8 @@ void k_dedup(Batch b, const Geom* __restrict__ g) {
     // (cell coordinates are monotone; their rounding is far below one cell)
     const float ch = fmaxf(rad + 1.0f, fmaxf(bymax - bymin, bxmax - bxmin) * (1.0f / 15.0f));
     const float cinv = uni(1.0f / ch);
-    const int ncy = min(DD_CELLS_1D, (int)((bymax - bymin) * cinv) + 1);
-    const int ncx = min(DD_CELLS_1D, (int)((bxmax - bxmin) * cinv) + 1);
+    const int ncy = max(1, min(DD_CELLS_1D, (int)((bymax - bymin) * cinv) + 1));
+    const int ncx = max(1, min(DD_CELLS_1D, (int)((bxmax - bxmin) * cinv) + 1));
     auto cell_y = [&](float yy) { return min(ncy - 1, max(0, (int)((yy - bymin) * cinv))); };
     auto cell_x = [&](float xx) { return min(ncx - 1, max(0, (int)((xx - bxmin) * cinv))); };
 

@@ -52,3 +52,19 @@ def test_host_library_under_asan():
         pytest.skip("clang's ASan runtime is not installed")
     lib = _build.build_asan()
     _pytest_under(rt, {"GT_TEST_LIB": lib}, ["test_abi.py", "test_ingest.py"])
+
+
+def test_kernel_objects_follow_their_headers(tmp_path):
+    """An object that the instrumented library links as it is must be as new as
+    every header, not as its own (possibly six-line) source only."""
+    from tracking_optimizations_amd import _build
+    src = "gt_bandpass_u16.hip"
+    obj = tmp_path / "gt_bandpass_u16.o"
+    assert _build._stale(str(obj), src)
+    obj.write_bytes(b"")
+    newest = max(os.path.getmtime(os.path.join(_build.CSRC, h))
+                 for h in ("gt_bandpass.h", "gt_internal.h"))
+    own = os.path.getmtime(os.path.join(_build.CSRC, src))
+    for at, stale in ((newest - 1, True), (max(newest, own) + 3600, False)):
+        os.utime(obj, (at, at))
+        assert _build._stale(str(obj), src) == stale

@@ -14,6 +14,7 @@ Every HIP source is compiled separately (in parallel) and linked into
 from __future__ import annotations
 
 import concurrent.futures as cf
+import glob
 import os
 import shutil
 import subprocess
@@ -73,6 +74,14 @@ def build(verbose: bool = True) -> str:
     return LIB
 
 
+def _stale(obj: str, src: str) -> bool:
+    """Whether `obj` is missing or older than `src` or any header: the headers
+    hold kernels and the structures that kernels and their callers share."""
+    deps = [os.path.join(CSRC, src), *glob.glob(os.path.join(CSRC, "*.h")),
+            *glob.glob(os.path.join(ROOT, "include", "*.h"))]
+    return not os.path.exists(obj) or os.path.getmtime(obj) < max(map(os.path.getmtime, deps))
+
+
 ASAN_DIR = os.path.join(HERE, "_build_asan")
 ASAN_LIB = os.path.join(ASAN_DIR, "libgpu_tracking_asan.so")
 
@@ -83,7 +92,7 @@ def build_asan(verbose: bool = False) -> str:
     host paths (parameters, column names, movie-file decoding, argument and
     error handling) under clang's ASan runtime.  The files in KERNEL_SOURCES,
     whose host code is kernel launchers only, are linked from the regular
-    build's objects (built first when missing)."""
+    build's objects (built first where missing or older than their sources)."""
     os.makedirs(ASAN_DIR, exist_ok=True)
     objdir = os.path.join(HERE, "_build")
     os.makedirs(objdir, exist_ok=True)
@@ -94,9 +103,8 @@ def build_asan(verbose: bool = False) -> str:
     for src in SOURCES:
         if src in KERNEL_SOURCES:
             obj = os.path.join(objdir, src.replace(".hip", ".o"))
-            srcp = os.path.join(CSRC, src)
-            if not os.path.exists(obj) or os.path.getmtime(obj) < os.path.getmtime(srcp):
-                jobs.append(([HIPCC, *FLAGS, "-c", srcp, "-o", obj], src))
+            if _stale(obj, src):
+                jobs.append(([HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj], src))
         else:
             obj = os.path.join(ASAN_DIR, src.replace(".hip", ".o"))
             jobs.append(([HIPCC, *flags, "-c", os.path.join(CSRC, src), "-o", obj], src))
@@ -124,7 +132,6 @@ def build_asan(verbose: bool = False) -> str:
 
 def asan_runtime() -> str:
     """clang's AddressSanitizer runtime matching hipcc (to preload)."""
-    import glob
     cands = sorted(glob.glob(os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "llvm", "lib",
                                           "clang", "*", "lib", "linux",
                                           "libclang_rt.asan-x86_64.so")))

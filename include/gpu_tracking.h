@@ -107,7 +107,10 @@ typedef struct gt_result gt_result;
 /* Per-call device timing of the last locate call on a context, measured with
  * HIP events on the context's stream. */
 typedef struct gt_timing {
-    double device_ms;       /* first kernel start .. last kernel end */
+    double device_ms;       /* first kernel start .. last kernel end; for frames in
+                               host memory or a file from the first upload on, with
+                               the waits for frames that are still being copied or
+                               decoded when their turn comes */
     double total_ms;        /* host wall time of the call */
     uint64_t frames;
     uint64_t pixels;

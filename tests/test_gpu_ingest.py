@@ -87,3 +87,23 @@ def test_batch_file_several_chunks_linked(tmp_path, ctx):
     ref, rc = batch_rust(v, 11, **kw)
     assert cols == rc and rows.shape[0] > 40 * 1000
     np.testing.assert_array_equal(rows, ref)
+
+
+def test_device_time_leaves_the_decoding_out(tmp_path):
+    """One frame that takes far longer to decode than to locate: device_ms
+    begins with its upload, not while it is being read."""
+    import time
+    from tracking_optimizations_amd.gpu_tracking import MovieFile
+    v = np.random.default_rng(4).integers(0, 400, (1, 2500, 2500)).astype(np.uint16)
+    f = tmp_path / "movie.tif"
+    write_tiff(f, list(v), compression=8)
+    with MovieFile(str(f)) as m:
+        t = time.perf_counter()
+        m.read()
+        decode_ms = 1e3 * (time.perf_counter() - t)
+    ctx = _lib.Context(0)
+    for _ in range(2):
+        batch_file_rust(str(f), 9, ctx=ctx, **KW)
+    t = ctx.timing()
+    print(f"[ingest] decode {decode_ms:.1f} ms, call {t['total_ms']:.1f}, device {t['device_ms']:.2f}", flush=True)
+    assert t["total_ms"] > decode_ms / 2 and t["device_ms"] < decode_ms / 4

@@ -1544,6 +1544,7 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         }
         if (!launched) {
             launches = 0;
+            if (ready) GT_TRY((*ready)(0));   // device time begins with the first upload
             HIP_TRY(hipEventRecord(ctx->ev0, s0));
             GT_TRY(enqueue());
         }

@@ -109,3 +109,31 @@ def test_tuning_reports_the_walk_that_runs():
     ref = locate(_noise(1, 512, 512, np.uint16, 6), p, ctx=_lib.Context(0))
     got = locate(_noise(1, 512, 512, np.uint16, 6), p, ctx=ctx)
     assert all(np.array_equal(x, y) for x, y in zip(ref[:2], got[:2]))
+
+
+def test_kept_blocks_go_back():
+    """An adjoint's patches are kept for the next one, and go back to the device
+    once calls without an adjoint follow; one that comes then allocates anew."""
+    torch = pytest.importorskip("torch")
+    torch.cuda.init()
+    ctx = _lib.Context(0)
+    video = _noise(32, 1024, 1024, np.uint16, 8)   # 131072 rows of patches: 127 MB
+    small = _noise(1, 64, 80, np.uint16, 9)
+    p = make_params(diameter=5, separation=5, minmass=30)
+    locate(video, p, ctx=ctx)   # the context's own buffers
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    def jac():
+        a = _adjoint(video, p, True, ctx=ctx)
+        return a.jacobian()
+
+    first = jac()
+    kept = free()
+    assert np.array_equal(jac(), first) and free() == kept
+    for _ in range(64):
+        locate(small, p, ctx=ctx)
+    assert free() - kept > 100e6
+    assert np.array_equal(jac(), first)

@@ -92,11 +92,12 @@ bool injected_failure(int kind) {
     return false;
 }
 
-// Live contexts: the block caches below keep memory only while there is one.
+// Live contexts, in all and per device: the block caches below keep memory only
+// while there is one (device blocks: on their device).
 std::atomic<int> g_contexts{0};
-
-// Returns the device blocks that are kept for later calls; true if there were any.
-bool drop_kept_device_blocks();
+constexpr int kDeviceSlots = 64;
+std::atomic<int> g_device_contexts[kDeviceSlots];
+std::atomic<int>& contexts_on(int device) { return g_device_contexts[device % kDeviceSlots]; }
 
 struct DevBuf {
     void* p = nullptr;
@@ -109,11 +110,7 @@ struct DevBuf {
         bytes = 0;
         n = (n + 255) & ~(size_t)255;
         if (injected_failure(0)) return hipErrorOutOfMemory;
-        hipError_t e = hipMalloc(&p, n);
-        if (e == hipErrorOutOfMemory && drop_kept_device_blocks()) {
-            (void)hipGetLastError();
-            e = hipMalloc(&p, n);
-        }
+        const hipError_t e = device_malloc(&p, n);
         if (e == hipSuccess) bytes = n;
         else p = nullptr;
         return e;
@@ -149,10 +146,12 @@ struct PinBuf {
 };
 
 // Device blocks that outlive a call (an adjoint's Jacobian patches): freed ones
-// are kept for the next adjoint on the same device, at most 1 GiB in all, and
-// handed back with the last context or when an allocation fails.  Every call
-// that uses a block waits for the device before it returns, so a freed one may
-// go to another stream or thread at once.
+// are kept for the next adjoint on the same device, at most 1 GiB in all.  They
+// are handed back with the device's last context, when an allocation of the
+// library fails, and when kIdleCalls locate calls have come and gone without
+// an adjoint taking one: a program that has stopped differentiating has its
+// memory back.  Every call that uses a block waits for the device before it
+// returns, so a freed one may go to another stream or thread at once.
 class DeviceBlockCache {
   public:
     struct Block {
@@ -165,6 +164,7 @@ class DeviceBlockCache {
         n = (std::max<size_t>(n, 256) + 255) & ~(size_t)255;
         {
             std::lock_guard<std::mutex> lk(mu());
+            idle() = 0;
             auto& v = blocks();
             size_t best = v.size();
             for (size_t i = 0; i < v.size(); ++i)
@@ -189,7 +189,7 @@ class DeviceBlockCache {
         std::vector<void*> drop;
         {
             std::lock_guard<std::mutex> lk(mu());
-            if (b.bytes > kMax || g_contexts.load() <= 0) {
+            if (b.bytes > kMax || contexts_on(b.device).load() <= 0) {
                 drop.push_back(b.p);
             } else {
                 auto& v = blocks();
@@ -205,12 +205,23 @@ class DeviceBlockCache {
         for (void* p : drop) (void)hipFree(p);
         b = Block{};
     }
-    static bool drain() {
-        std::vector<Block> drop;
+    // a locate call that takes no block
+    static void idle_call() {
         {
             std::lock_guard<std::mutex> lk(mu());
-            drop.swap(blocks());
-            total() = 0;
+            if (blocks().empty() || ++idle() < kIdleCalls) return;
+        }
+        drain();
+    }
+    // Frees what is kept (on one device, or -1: on all); true if there was any.
+    static bool drain(int device = -1) {
+        std::vector<Block> drop, stay;
+        {
+            std::lock_guard<std::mutex> lk(mu());
+            for (auto& b : blocks()) (device < 0 || b.device == device ? drop : stay).push_back(b);
+            for (auto& b : drop) total() -= b.bytes;
+            blocks().swap(stay);
+            idle() = 0;
         }
         for (auto& b : drop) (void)hipFree(b.p);
         return !drop.empty();
@@ -218,13 +229,13 @@ class DeviceBlockCache {
 
   private:
     static constexpr size_t kMax = (size_t)1 << 30;
+    static constexpr int kIdleCalls = 64;
     // never destroyed: adjoints may be freed during process teardown
     static std::mutex& mu() { static std::mutex* m = new std::mutex; return *m; }
     static std::vector<Block>& blocks() { static auto* v = new std::vector<Block>; return *v; }
     static size_t& total() { static size_t t = 0; return t; }
+    static int& idle() { static int n = 0; return n; }
 };
-
-bool drop_kept_device_blocks() { return DeviceBlockCache::drain(); }
 
 // ---- exact division check -------------------------------------------------
 
@@ -1111,6 +1122,8 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
         return GT_OK;
     }
 
+    if (!adj || !adj->jacobian) DeviceBlockCache::idle_call();
+
     // ---- batch plan -------------------------------------------------------
     const size_t max_batch = plain ? 1 : (batch_frames ? batch_frames : 4096);
     // host frames go up in pieces, so that one piece's kernels run beside the
@@ -1603,6 +1616,13 @@ gt_status run_locate(gt_context* ctx, const std::vector<FrameIn>& frames, int in
 
 namespace gt {
 gt_status set_last_error(gt_status s, const std::string& msg) { return fail(s, "%s", msg.c_str()); }
+
+hipError_t device_malloc(void** p, size_t n) {
+    const hipError_t e = hipMalloc(p, n);
+    if (e != hipErrorOutOfMemory || !DeviceBlockCache::drain()) return e;
+    (void)hipGetLastError();
+    return hipMalloc(p, n);
+}
 }  // namespace gt
 
 // ---- C ABI ----------------------------------------------------------------
@@ -1723,6 +1743,7 @@ gt_status gt_context_create(int device, gt_context** out) {
     gt_context* c = new gt_context();
     c->device = device;
     ++g_contexts;
+    ++contexts_on(device);
     bool ok = true;
     for (int i = 0; i < kStreams; ++i)
         ok = ok && hipStreamCreateWithFlags(&c->streams[i], hipStreamNonBlocking) == hipSuccess &&
@@ -1733,6 +1754,7 @@ gt_status gt_context_create(int device, gt_context** out) {
     if (!ok) {
         delete c;
         --g_contexts;
+        --contexts_on(device);
         return fail(GT_E_HIP, "stream/event creation failed");
     }
     c->stream = c->streams[0];
@@ -1761,10 +1783,8 @@ gt_status gt_context_destroy(gt_context* ctx) {
     for (DevBuf* b : bufs) b->release();
     ctx->up.release();
     ctx->down.release();
-    if (--g_contexts == 0) {
-        DeviceBlockCache::drain();
-        HostBlockCache::drain();
-    }
+    if (--contexts_on(ctx->device) == 0) DeviceBlockCache::drain(ctx->device);
+    if (--g_contexts == 0) HostBlockCache::drain();
     for (int i = 0; i < kStreams; ++i) ctx->ws[i].release();
     for (void* b : ctx->pinned)
         if (b) (void)hipHostFree(b);
@@ -2707,7 +2727,7 @@ gt_status gt_synth_u16(gt_context* ctx, uint16_t* d_frames, uint64_t n_frames, u
 gt_status gt_device_alloc(gt_context* ctx, uint64_t bytes, void** out) {
     if (!ctx || !out) return fail(GT_E_INVALID, "NULL argument");
     HIP_TRY(hipSetDevice(ctx->device));
-    HIP_TRY(hipMalloc(out, bytes ? bytes : 1));
+    HIP_TRY(device_malloc(out, bytes ? bytes : 1));
     return GT_OK;
 }
 

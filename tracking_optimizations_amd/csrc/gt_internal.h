@@ -150,6 +150,10 @@ struct AdjOut {
     float* jac;            // [rows_cap * 3 * S * S] Jacobian patches, or null
 };
 
+// hipMalloc; where that is out of memory, once more without the device blocks
+// that are kept for later calls (gt_api.hip).
+hipError_t device_malloc(void** p, size_t n);
+
 // Launchers (gt_kernels.hip, gt_bandpass.hip, gt_detect.hip).  All launch on
 // `s`; return hipSuccess or the first launch error.
 // The streaming bandpass handles every input type with 1 <= R <= 16 (all that

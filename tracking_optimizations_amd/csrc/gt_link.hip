@@ -132,7 +132,7 @@ struct Buf {
         if (p && n <= bytes) return hipSuccess;
         release();
         n = (n + 4095) & ~(size_t)4095;
-        const hipError_t e = PINNED ? hipHostMalloc(&p, n, hipHostMallocDefault) : hipMalloc(&p, n);
+        const hipError_t e = PINNED ? hipHostMalloc(&p, n, hipHostMallocDefault) : device_malloc(&p, n);
         if (e == hipSuccess) bytes = n;
         else p = nullptr;
         return e;

@@ -19,8 +19,8 @@
 //   sigma^2 = sum_r J[r]^2 * lambda[r],  lambda[r] = max(I[r], 0).
 //
 // The vector-Jacobian product used by the Python autograd wrapper adds the
-// patches of a frame's rows in row order, one workgroup per frame, so the
-// gradient is deterministic.
+// patches of a frame's rows in row order, one wave per tile of the frame, so
+// the gradient is deterministic.
 #include <algorithm>
 #include <type_traits>
 
@@ -374,12 +374,19 @@ __global__ __launch_bounds__(64) void k_adjoint_sep(Batch b, const Geom* __restr
 // The two norms multiply as reciprocals of two parts, so no output divides.
 //
 // Bound by issued instructions, about 400 per row at d = 9: 64 frames of
-// 512^2 (80 k rows) in 119 us, against 605 us for the form above with its
+// 512^2 (80 k rows) in 97 us, against 605 us for the form above with its
 // tables in LDS (5 LDS reads per 6 FMAs, six divisions per patch pixel).
+//
+// Waves per SIMD (adj_waves): the most whose registers hold all, or all but
+// four.  Four spilled ones cost less than a wave (64 frames of 512^2: RINT 2,
+// R 3 58.5 us at four waves, 61.1 at three without spills; RINT 3, R 4 63.9 at
+// three, 71.0 at two), 37 and 45 of them more (RINT 4 at three waves: R 4 117
+// against 97 us at two, R 5 104 against 83).
+constexpr int adj_waves(int rint) { return rint <= 2 ? 4 : rint <= 3 ? 3 : rint <= 5 ? 2 : 1; }
+
 template <int RINT, int R, typename T>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RINT <= 2 ? 4 : RINT <= 4 ? 3 : RINT <= 5 ? 2 : 1)))
-void k_adjoint_reg(Batch b, const Geom* __restrict__ g,
-                                                   AdjOut ao, uint32_t frame_pos0) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(adj_waves(RINT))))
+void k_adjoint_reg(Batch b, const Geom* __restrict__ g, AdjOut ao, uint32_t frame_pos0) {
     constexpr int D = 2 * RINT + 1, NT = 2 * R + 1, S = 2 * (RINT + R) + 1;
     constexpr int G = 64 / S;
     static_assert(S <= 64 && D <= NT, "a patch column per lane; prefix and suffix windows");

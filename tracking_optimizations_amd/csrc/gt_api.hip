@@ -809,8 +809,9 @@ FrameSizes sizes_of(uint32_t h, uint32_t w, int seg) {
 }
 
 // Whether the walk of a call over `tiles` detect tiles runs in its own kernel
-// although detect could do it.  A tile of a window of 18 or more holds at most
-// half a dozen candidates, and a wave of detect walks them alone: gathered
+// although detect could do it.  A tile of a window of 18 or more typically
+// holds a handful of candidates (2.5 at KD = 31 on spots; a plateau, whose
+// ties are kept, any number), and a wave of detect walks them alone: gathered
 // from 16 tiles they take 64 against 117 us of detect (the whole 121 -> 112 us
 // for 96 frames of 517 x 663 at KD = 19; 144 -> 106 us at KD = 25, 264 -> 155
 // us at KD = 31, 24 frames of 1024^2; 89 -> 111 us the other way at KD = 15).
@@ -2220,6 +2221,10 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
     HIP_TRY(hipSetDevice(ctx->device));
     Geom g;
     GT_TRY(make_geom(p, g));
+    // The walk runs inside detect where the window's own kernel does it, and in
+    // a kernel of its own elsewhere; run_locate's rule goes by the size of the
+    // call.  Inside detect a percentile takes a fourth record plane, which the
+    // scratch of wide windows was never counted with.
     g.walk_in_detect = ctx->fuse_walk && walk_in_own_detect(g) ? 1 : 0;
     const size_t es = elem_size(in_type);
     const bool generic = !bandpass_fast_path(in_type, w, g);
@@ -2346,7 +2351,7 @@ static gt_status locate_noalloc(gt_context* ctx, const void* frames, int in_type
         b.tile_frame = b.k1_frame + (uint64_t)nb * fs.k1_items;
         b.dblock_tile = b.tile_frame + (uint64_t)nb * fs.tiles;
         b.dblocks = (uint32_t)(nb * dblocks_pf);
-        b.dblock_side = 2;   // a table of every tile could exceed the host tables' bound
+        b.dblock_side = 2;   // a table of every tile would take more of the scratch
         b.nframes = nb;
         b.k1_items = nb * fs.k1_items;
         b.tiles = nb * fs.tiles;

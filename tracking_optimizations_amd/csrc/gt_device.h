@@ -9,10 +9,8 @@
 // address space.
 #if defined(__HIP_DEVICE_COMPILE__)
 #define GLOBAL __attribute__((address_space(1)))
-#define SHARED __attribute__((address_space(3)))
 #else
 #define GLOBAL
-#define SHARED
 #endif
 
 namespace gt {
@@ -41,18 +39,10 @@ __device__ __forceinline__ uint32_t pct_key(uint32_t bits) {
 template <typename T> struct IsFloat { static constexpr bool v = false; };
 template <> struct IsFloat<float> { static constexpr bool v = true; };
 
-template <typename T>
-__device__ __forceinline__ float ld_px(const T* p, size_t i) { return (float)p[i]; }
-
 __device__ __forceinline__ float raw_px(const void* in, int type, size_t i) {
     if (type == IN_U16) return (float)((const uint16_t*)in)[i];
     if (type == IN_U8) return (float)((const uint8_t*)in)[i];
     return ((const float*)in)[i];
-}
-
-__device__ __forceinline__ float wave_sum_f(float v) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
 }
 
 __device__ __forceinline__ uint32_t wave_sum_u(uint32_t v) {

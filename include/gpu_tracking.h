@@ -191,9 +191,11 @@ typedef struct gt_tuning {
 gt_status gt_context_autotune(gt_context* ctx, const gt_params* p, uint32_t h, uint32_t w,
                               uint32_t n_frames, gt_tuning* out);
 
-/* 1 (default): where the geometry allows it, the centroid walk runs inside
- * the detect kernel on the tile it has staged; 0: a separate refine kernel
- * walks every candidate.  Results are identical either way. */
+/* 1 (default): where the geometry allows it and it is the faster, the centroid
+ * walk runs inside the detect kernel on the tile it has staged (dilation
+ * windows of 18 and more over more than 1024 tiles of 48 x 64 pixels walk in
+ * a kernel of their own); 0: a separate kernel walks every candidate.  Results
+ * are identical either way. */
 gt_status gt_context_set_fused_walk(gt_context* ctx, int enable);
 
 /* Per-stage kernel timing (HIP events recorded around every launch on the

@@ -35,3 +35,25 @@ def test_columns_over_diameters(dtype, diameter):
     names, rnames = [n for n, _ in cols], [n for n, _ in rcols]
     for n in names:
         np.testing.assert_array_equal(raw[:, rnames.index(n)], rows[:, names.index(n)], err_msg=n)
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_signal_beside_a_pixel_that_is_not_finite(value):
+    """The host's circle of an even diameter reaches one pixel past the disk that
+    makes a row: a NaN in its first tap is the signal, one in another is
+    skipped, as the maximum in tap order does."""
+    f = np.zeros((1, 100, 120), np.float32)
+    for y, x in ((30, 40), (70, 40), (50, 90)):
+        yy, xx = np.mgrid[-4:5, -4:5]
+        f[0, y - 4:y + 5, x - 4:x + 5] += (300 * np.exp(-(yy ** 2 + xx ** 2) / 4.0)).astype(np.float32)
+    f[0, 30 - 9, 40] = value   # P is not finite in rows 17 to 25: the first tap
+    f[0, 70 + 9, 40] = value   # rows 75 to 83: the last
+    kw = dict(diameter=10, separation=7, smoothing_size=9, cpu_processed=True, characterize=True,
+              max_iterations=1, minmass=1000)
+    ref = _oracle_movie(f, kw)
+    at = {(30, 40): True, (70, 40): False, (50, 90): False}
+    for (y, x), nan in at.items():
+        k = np.nonzero(ref[1] == y * 120 + x)[0]
+        assert len(k) == 1 and np.isnan(ref[0][k[0], 6]) == nan
+    rows, cand, _, _ = locate(f, make_params(**kw), ctx=_lib.default_context(0))
+    _check(rows, cand, *ref, f"beside {value}")

@@ -142,6 +142,9 @@ __global__ __launch_bounds__(CH_WG) void k_char(Batch b, const Geom* __restrict_
                 const float t = __shfl_xor(sig, d, 64);
                 sig = t > sig ? t : sig;
             }
+            // in order from the first tap: a NaN there stays, later ones are skipped
+            const float lead = p[hoff[0]];
+            sig = lead != lead ? lead : sig;
             ss = ss * ss;
             cc = cc * cc;
             const float ecc = sqrtf(ss + cc);

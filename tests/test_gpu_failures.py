@@ -84,3 +84,29 @@ def test_disarmed_by_zero(frames, reference):
     assert np.array_equal(got[0], reference[0])
     with pytest.raises(_lib.GtError):
         _inject(2, 1)
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+def test_adjoint_allocation_failures(frames, kind):
+    """Each allocation of an adjoint in turn, on the device (workspaces, rows,
+    patches, the frames' row ranges) and for its host results: GT_E_OOM, and
+    the next call's rows, errors and patches are an untouched context's."""
+    from tracking_optimizations_amd.adjoint import _adjoint
+    p = make_params(**KW)
+    want = _adjoint(frames, p, True, ctx=_lib.Context(0))
+    want = [want.rows(), want.sigma(), want.origin(), want.jacobian()]
+    failed = 0
+    for after in range(1, 25):
+        ctx = _lib.Context(0)
+        _inject(kind, after)
+        try:
+            _adjoint(frames, p, True, ctx=ctx)
+        except _lib.GtError as e:
+            failed += 1
+            assert e.status == _lib.GT_E_OOM, (after, str(e))
+        finally:
+            _inject(kind, 0)
+        a = _adjoint(frames, p, True, ctx=ctx)
+        for x, y in zip(want, [a.rows(), a.sigma(), a.origin(), a.jacobian()]):
+            np.testing.assert_array_equal(x, y)
+    assert failed >= (5 if kind else 10)

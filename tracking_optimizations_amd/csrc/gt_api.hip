@@ -2535,8 +2535,9 @@ gt_status gt_locate_adjoint(gt_context* ctx, const void* frames, int dtype, uint
     gt_result* res = nullptr;
     GT_TRY(run_locate(ctx, v, in_type, p, flags & ~(uint32_t)(GT_RESULT_ON_DEVICE | GT_ADJ_JACOBIAN),
                       &res, &req));
-    gt_adjoint* a = new gt_adjoint();
-    a->fwd = res;
+    std::unique_ptr<gt_result> fwd(res);
+    std::unique_ptr<gt_adjoint> a(new gt_adjoint());
+    a->fwd = fwd.release();
     a->device = ctx->device;
     {
         Geom g;
@@ -2551,12 +2552,15 @@ gt_status gt_locate_adjoint(gt_context* ctx, const void* frames, int dtype, uint
     a->sigma.resize(n * 3);
     a->origin.resize(n * 2);
     a->rowpos.resize(n);
+    hipStream_t st = ctx->streams[0];
     auto cleanup = [&](hipError_t e) {
-        delete a;
-        return fail(GT_E_HIP, "adjoint readback: %s", hipGetErrorString(e));
+        // copies that were queued before the failing one still use the blocks
+        // that `a` and `req` are about to hand on
+        (void)hipStreamSynchronize(st);
+        return fail(e == hipErrorOutOfMemory ? GT_E_OOM : GT_E_HIP, "adjoint readback: %s",
+                    hipGetErrorString(e));
     };
     hipError_t e = hipSuccess;
-    hipStream_t st = ctx->streams[0];
     const void* d_origin = req.jacobian ? req.origin.p : ctx->adj_origin.p;
     if (n) {
         e = hipMemcpyAsync(a->sigma.data(), ctx->adj_sigma.p, n * 12, hipMemcpyDeviceToHost, st);
@@ -2576,7 +2580,7 @@ gt_status gt_locate_adjoint(gt_context* ctx, const void* frames, int dtype, uint
         if (e == hipSuccess) e = hipMemcpy(a->d_frame_rows.p, fr.data(), fr.size() * 8, hipMemcpyHostToDevice);
         if (e != hipSuccess) return cleanup(e);
     }
-    *out = a;
+    *out = a.release();
     return GT_OK;
     });
 }
